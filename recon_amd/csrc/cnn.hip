@@ -3,10 +3,11 @@
 // include/rt_cnn.h.
 //
 // Every convolution is an implicit GEMM over NHWC bfloat16 tensors. The
-// forward pass of the default network runs on v_mfma_f32_16x16x32_bf16
-// (k_conv_fwd_mfma); other layer shapes and the backward passes use
-// v_mfma_f32_16x16x16_bf16 tiles (64-lane wave, A: 16 rows x 4 k per lane
-// group, B: 4 k x 16 columns, D: 4 rows x 16 columns per lane group):
+// forward pass of the default network (k_conv_fwd_mfma and its LDS-staged
+// relatives) and the backward passes run on v_mfma_f32_16x16x32_bf16 (64-lane
+// wave, A: 16 rows x 8 k per lane group, B: 8 k x 16 columns, D: 4 rows x 16
+// columns per lane group); layers with 16 channels use
+// v_mfma_f32_16x16x16_bf16 tiles (4 k per lane group):
 //   forward      rows = output pixels (n, yo, xo), columns = Cout, k = (tap, Cin)
 //   input grad   rows = input pixels (n, yi, xi),  columns = Cin,  k = (tap, Cout)
 //   weight grad  rows = Cout, columns = (tap, Cin), k = output pixels, split
@@ -646,120 +647,372 @@ __global__ __launch_bounds__(256) void k_conv_bwd_data(ConvGeom g, const bf16* _
     }
 }
 
-// ---------------------------------------------------------------- weight gradient
-// ws[s][co][k] = sum over output pixels m of chunk s of dZ[m][co] * im2col(X)[m][k].
-// One wave per block: 32 output channels x 32 k.
-__global__ __launch_bounds__(64) void k_conv_bwd_w(ConvGeom g, const bf16* __restrict__ dZ, const bf16* __restrict__ X,
-                                                   float* __restrict__ ws, int chunk) {
-    const int lane = threadIdx.x;
-    const int r16 = lane & 15, kq = lane >> 4;
-    const int M = g.B * g.Ho * g.Wo, HW = g.Ho * g.Wo;
-    const int co0 = blockIdx.x * 32, kc0 = blockIdx.y * 32, s = blockIdx.z;
-    const int mbeg = s * chunk, mend = min(M, mbeg + chunk);
-    int tapj[2], cij[2];
-    bool kv[2];
+// The input gradient by parity class (blockIdx.z = 2 py + px): with stride 2 an
+// input pixel (yi, xi) receives only the taps of its parity, ky = 1 where yi
+// is even and ky in {0, 2} where it is odd (likewise kx), so each class is a
+// GEMM over its own pixels with 1, 2, 2 or 4 taps instead of nine taps masked
+// to a quarter of them. A workgroup tile of BM pixels x BN input channels, k =
+// (tap, Cout) in stages of KS staged through double-buffered LDS as in
+// k_conv_fwd_lds32; the tile leaves through LDS as 16-byte row chunks, masked
+// by the ReLU of the layer input (X > 0). 256 samples, five layers: 477 us in
+// the general kernel (nine masked taps, operands gathered from global memory
+// per MFMA), 78 us here; bound by the latency of the staged loads.
+template <int BM, int BN, int WGM, int KS>
+__global__ __launch_bounds__(256) void k_conv_bwd_data_lds(ConvGeom g, const bf16* __restrict__ dZ,
+                                                           const bf16* __restrict__ WT, const bf16* __restrict__ X,
+                                                           bf16* __restrict__ dX) {
+    constexpr int WGN = 4 / WGM, WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;
+    constexpr int LD = KS + 8;
+    constexpr int STAGE = (BM + BN) * LD;
+    constexpr int CR = KS / 8;
+    constexpr int AC = BM * CR, BC = BN * CR;
+    constexpr int AQ = (AC + 255) / 256, BQ = (BC + 255) / 256;
+    constexpr int TLD = BN + 8;
+    static_assert(BM * TLD <= 2 * STAGE, "epilogue tile fits in the stage buffers");
+    __shared__ __attribute__((aligned(16))) bf16 lds[2 * STAGE];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, r16 = lane & 15, kg = lane >> 4;
+    const int py = blockIdx.z >> 1, px = blockIdx.z & 1;
+    const int Hc = (g.Hi + 1 - py) >> 1, Wc = (g.Wi + 1 - px) >> 1, HWc = Hc * Wc;  // the class's pixels
+    const int M = g.B * HWc;
+    const int bm0 = blockIdx.x * BM, bn0 = blockIdx.y * BN;
+    if (bm0 >= M) return;
+    // the class's pixel m as (n, yi, xi)
+    auto pixel = [&](int m, int& n, int& yi, int& xi) {
+        n = m / HWc;
+        const int r = m - n * HWc, yc = r / Wc;
+        yi = 2 * yc + py;
+        xi = 2 * (r - yc * Wc) + px;
+    };
+    int arow[AQ], apart[AQ], ayi[AQ], axi[AQ];
+    size_t anb[AQ];
+    bool av[AQ], ae[AQ];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        int k = kc0 + j * 16 + r16;
-        tapj[j] = k >> g.ci_shift;
-        cij[j] = k & (g.Ci - 1);
-        kv[j] = k < g.K;
+    for (int q = 0; q < AQ; q++) {
+        const int e = t + 256 * q;
+        ae[q] = e < AC;
+        arow[q] = (e / CR) % BM;
+        apart[q] = e % CR;
+        const int m = bm0 + arow[q];
+        av[q] = ae[q] && m < M;
+        int n;
+        pixel(av[q] ? m : 0, n, ayi[q], axi[q]);
+        anb[q] = (size_t)n * g.Ho * g.Wo;
     }
+    int brow[BQ], bpart[BQ];
+    bool be[BQ];
+    const bf16* bp[BQ];
+#pragma unroll
+    for (int q = 0; q < BQ; q++) {
+        const int e = t + 256 * q;
+        be[q] = e < BC;
+        brow[q] = (e / CR) % BN;
+        bpart[q] = e % CR;
+        bp[q] = WT + (size_t)(bn0 + brow[q]) * 9 * g.Co + 8 * bpart[q];
+    }
+    uint4 ra[AQ], rb[BQ];
+    auto gload = [&](int s) {
+        const int k = KS * s;
+        const int j = k >> g.co_shift, co0 = k & (g.Co - 1);  // tap j of the class
+        const int jx = px ? (j & 1) : 0, jy = py ? (px ? j >> 1 : j) : 0;
+        const int ky = py ? 2 * jy : 1, kx = px ? 2 * jx : 1;
+#pragma unroll
+        for (int q = 0; q < AQ; q++) {
+            const int yo = (ayi[q] + 1 - ky) >> 1, xo = (axi[q] + 1 - kx) >> 1;  // exact: even by the class's taps
+            const bool ok = av[q] && yo >= 0 && xo >= 0 && yo < g.Ho && xo < g.Wo;
+            ra[q] = ok ? *(const uint4*)(dZ + (anb[q] + (size_t)yo * g.Wo + xo) * g.Co + co0 + 8 * apart[q])
+                       : make_uint4(0u, 0u, 0u, 0u);
+        }
+        const size_t bo = (size_t)(3 * ky + kx) * g.Co + co0;
+#pragma unroll
+        for (int q = 0; q < BQ; q++) rb[q] = be[q] ? *(const uint4*)(bp[q] + bo) : make_uint4(0u, 0u, 0u, 0u);
+    };
+    auto sstore = [&](int buf) {
+        bf16* A = lds + buf * STAGE;
+        bf16* Bs = A + BM * LD;
+#pragma unroll
+        for (int q = 0; q < AQ; q++)
+            if (ae[q]) *(uint4*)(A + arow[q] * LD + 8 * apart[q]) = ra[q];
+#pragma unroll
+        for (int q = 0; q < BQ; q++)
+            if (be[q]) *(uint4*)(Bs + brow[q] * LD + 8 * bpart[q]) = rb[q];
+    };
+    const int wm0 = (w % WGM) * WM, wn0 = (w / WGM) * WN;
+    f4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    const int steps = (1 + py) * (1 + px) * g.Co / KS;
+    gload(0);
+    sstore(0);
+    __syncthreads();
+    for (int s = 0; s < steps; s++) {
+        const int cur = s & 1;
+        if (s + 1 < steps) gload(s + 1);
+        const bf16* A = lds + cur * STAGE;
+        const bf16* Bs = A + BM * LD;
+#pragma unroll
+        for (int kk = 0; kk < KS; kk += 32) {
+            bf8 a[TM], b[TN];
+#pragma unroll
+            for (int i = 0; i < TM; i++) a[i] = *(const bf8*)(A + (wm0 + 16 * i + r16) * LD + kk + 8 * kg);
+#pragma unroll
+            for (int j = 0; j < TN; j++) b[j] = *(const bf8*)(Bs + (wn0 + 16 * j + r16) * LD + kk + 8 * kg);
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] = mfma32(a[i], b[j], acc[i][j]);
+        }
+        if (s + 1 < steps) sstore(cur ^ 1);
+        __syncthreads();
+    }
+    bf16* T = lds;
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                T[(wm0 + 16 * i + 4 * kg + e) * TLD + wn0 + 16 * j + r16] = f2bf(acc[i][j][e]);
+    __syncthreads();
+    constexpr int CPR = BN / 8;
+#pragma unroll
+    for (int e0 = 0; e0 < BM * CPR; e0 += 256) {
+        const int e = e0 + t;
+        if (e < BM * CPR) {
+            const int rr = e / CPR, c = e - rr * CPR;
+            const int m = bm0 + rr;
+            if (m < M) {
+                int n, yi, xi;
+                pixel(m, n, yi, xi);
+                const size_t o = (((size_t)n * g.Hi + yi) * g.Wi + xi) * g.Ci + bn0 + 8 * c;
+                const uint4 xv = *(const uint4*)(X + o);
+                uint4 v = *(const uint4*)(T + rr * TLD + 8 * c);
+                auto mask = [](unsigned x, unsigned u) {
+                    return (bf_pos((bf16)(x & 0xffffu)) ? u & 0xffffu : 0u) | (bf_pos((bf16)(x >> 16)) ? u & 0xffff0000u : 0u);
+                };
+                v = make_uint4(mask(xv.x, v.x), mask(xv.y, v.y), mask(xv.z, v.z), mask(xv.w, v.w));
+                *(uint4*)(dX + o) = v;
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------- weight gradient
+// ws[s][co][k] = sum over output pixels m of chunk s of dZ[m][co] * im2col(X)[m][k],
+// and, from the first column tile, ws_b[s][co] = the chunk's sum of dZ[m][co]
+// (the bias gradient). Workgroup tile: 64 output channels x 64 k, 128 pixels a
+// stage. The reduction runs over m, the slow index of both operands, so each
+// thread loads an 8 x 8 block (8 pixels x 8 channels, one 16-byte run per
+// pixel), transposes it in registers and stores eight 16-byte runs of m to
+// LDS, from which the MFMA operands are read whole; the next stage's loads
+// are issued before this stage's MFMAs. 256 samples, six layers: 324 us with
+// one wave per 32 x 32 tile and 2-byte gathers, plus 360 us of column sums;
+// 101 us here for both.
+constexpr int BW_M = 128, BW_LD = BW_M + 8;  // pixels a stage; LDS row pitch (bf16)
+__global__ __launch_bounds__(256) void k_conv_bwd_w(ConvGeom g, const bf16* __restrict__ dZ, const bf16* __restrict__ X,
+                                                    float* __restrict__ ws, float* __restrict__ ws_b, int chunk) {
+    __shared__ __attribute__((aligned(16))) bf16 lds[2 * 64 * BW_LD];  // A: [co][m], B: [k][m]
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, r16 = lane & 15, kg = lane >> 4;
+    const int M = g.B * g.Ho * g.Wo, HW = g.Ho * g.Wo;
+    const int co0 = blockIdx.x * 64, kc0 = blockIdx.y * 64, s = blockIdx.z;
+    const int mbeg = s * chunk, mend = min(M, mbeg + chunk);
+    // threads 0-127 stage dZ, 128-255 the im2col columns: pixel block mb, channel (or k) block cb
+    const int half = t >> 7, mb = t & 15, cb = (t >> 4) & 7;
+    const int col = (half ? kc0 : co0) + 8 * cb;
+    const bool cv = col < (half ? g.K : g.Co);  // K is a multiple of 4, Co of 16
+    const int tap0 = col >> g.ci_shift, tap1 = (col + 4) >> g.ci_shift;
+    const int ky0 = tap0 / 3, kx0 = tap0 - 3 * ky0, ky1 = tap1 / 3, kx1 = tap1 - 3 * ky1;
+    const int ci = col & (g.Ci - 1);
+    const bool cv1 = col + 4 < g.K;
+    uint4 r[8];
+    float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const bool bias = blockIdx.y == 0 && !half;
+    auto gload = [&](int m0) {
+        const int mf = m0 + 8 * mb;
+        int n = 0, yo = 0, xo = 0;
+        if (half) {
+            const int mm = min(mf, M - 1);
+            n = mm / HW;
+            const int q = mm - n * HW;
+            yo = q / g.Wo;
+            xo = q - yo * g.Wo;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const bool mok = cv && mf + e < mend;
+            r[e] = make_uint4(0u, 0u, 0u, 0u);
+            if (!half) {
+                if (mok) r[e] = *(const uint4*)(dZ + (size_t)(mf + e) * g.Co + col);
+            } else {
+                const bf16* Xn = X + (size_t)n * g.Hi * g.Wi * g.Ci;
+                const int yi = 2 * yo - 1 + ky0, xi = 2 * xo - 1 + kx0;
+                const bool ok = mok && yi >= 0 && yi < g.Hi && xi >= 0 && xi < g.Wi;
+                if (g.Ci == 4) {  // two taps of 4 channels
+                    const int yj = 2 * yo - 1 + ky1, xj = 2 * xo - 1 + kx1;
+                    const bool okj = mok && cv1 && yj >= 0 && yj < g.Hi && xj >= 0 && xj < g.Wi;
+                    const uint2 u = ok ? *(const uint2*)(Xn + ((size_t)yi * g.Wi + xi) * 4) : make_uint2(0u, 0u);
+                    const uint2 v = okj ? *(const uint2*)(Xn + ((size_t)yj * g.Wi + xj) * 4) : make_uint2(0u, 0u);
+                    r[e] = make_uint4(u.x, u.y, v.x, v.y);
+                } else if (ok) {
+                    r[e] = *(const uint4*)(Xn + ((size_t)yi * g.Wi + xi) * g.Ci + ci);
+                }
+                if (++xo == g.Wo) {
+                    xo = 0;
+                    if (++yo == g.Ho) { yo = 0; n++; }
+                }
+            }
+        }
+    };
+    auto sstore = [&]() {
+        bf16* base = lds + half * 64 * BW_LD + (8 * cb) * BW_LD + 8 * mb;
+        const unsigned* rw = reinterpret_cast<const unsigned*>(r);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {  // channels 2j, 2j + 1: the low and high halves of dword j of each pixel
+            unsigned lo[4], hi[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                lo[i] = __builtin_amdgcn_perm(rw[4 * (2 * i + 1) + j], rw[4 * (2 * i) + j], 0x05040100u);
+                hi[i] = __builtin_amdgcn_perm(rw[4 * (2 * i + 1) + j], rw[4 * (2 * i) + j], 0x07060302u);
+            }
+            *(uint4*)(base + (2 * j) * BW_LD) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+            *(uint4*)(base + (2 * j + 1) * BW_LD) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        }
+        if (bias) {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    bsum[2 * j] += __uint_as_float(rw[4 * e + j] << 16);
+                    bsum[2 * j + 1] += __uint_as_float(rw[4 * e + j] & 0xffff0000u);
+                }
+        }
+    };
+    const int wa0 = (w & 1) * 32, wb0 = (w >> 1) * 32;
     f4 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-    for (int m0 = mbeg; m0 < mend; m0 += 16) {
-        s4 a[2], b[2];
+    const bf16* A = lds;
+    const bf16* Bs = lds + 64 * BW_LD;
+    gload(mbeg);
+    for (int m0 = mbeg; m0 < mend; m0 += BW_M) {
+        sstore();
+        __syncthreads();
+        if (m0 + BW_M < mend) gload(m0 + BW_M);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            int m = m0 + kq * 4 + e;
-            bool mok = m < mend;
-            int mm = mok ? m : mbeg;
-            int n = mm / HW, r = mm - (mm / HW) * HW;
-            int yo = r / g.Wo, xo = r - (r / g.Wo) * g.Wo;
+        for (int kk = 0; kk < BW_M; kk += 32) {
+            bf8 a[2], b[2];
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                int co = co0 + i * 16 + r16;
-                a[i][e] = (mok && co < g.Co) ? (short)dZ[(size_t)mm * g.Co + co] : (short)0;
-            }
+            for (int i = 0; i < 2; i++) a[i] = *(const bf8*)(A + (wa0 + 16 * i + r16) * BW_LD + kk + 8 * kg);
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                int tap = tapj[j];
-                int ky = tap / 3, kx = tap - 3 * (tap / 3);
-                int yi = 2 * yo - 1 + ky, xi = 2 * xo - 1 + kx;
-                bool ok = mok && kv[j] && yi >= 0 && yi < g.Hi && xi >= 0 && xi < g.Wi;
-                b[j][e] = ok ? (short)X[(((size_t)n * g.Hi + yi) * g.Wi + xi) * g.Ci + cij[j]] : (short)0;
-            }
+            for (int j = 0; j < 2; j++) b[j] = *(const bf8*)(Bs + (wb0 + 16 * j + r16) * BW_LD + kk + 8 * kg);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[i][j] = mfma32(a[i], b[j], acc[i][j]);
         }
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) acc[i][j] = mfma(a[i], b[j], acc[i][j]);
+        __syncthreads();
     }
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            int k = kc0 + j * 16 + r16;
+            const int k = kc0 + wb0 + 16 * j + r16;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                int co = co0 + i * 16 + kq * 4 + e;
+                const int co = co0 + wa0 + 16 * i + kg * 4 + e;
                 if (co < g.Co && k < g.Kp) ws[((size_t)s * g.Co + co) * g.Kp + k] = acc[i][j][e];
             }
         }
+    if (blockIdx.y == 0) {  // the 16 pixel blocks' channel sums, in order
+        float* part = reinterpret_cast<float*>(lds);  // [16][64]; every wave is past its last operand read
+        if (!half) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) part[mb * 64 + 8 * cb + e] = bsum[e];
+        }
+        __syncthreads();
+        if (t < 64 && co0 + t < g.Co) {
+            float v = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 16; q++) v += part[q * 64 + t];
+            ws_b[(size_t)s * g.Co + co0 + t] = v;
+        }
+    }
 }
 
-// grad_w[co][k] = sum_s ws[s][co][k] (k < K), in order of s
-__global__ void k_reduce_w(const float* __restrict__ ws, int S, int Co, int Kp, int K, float* __restrict__ gw) {
-    int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= Co * K) return;
-    int co = idx / K, k = idx - (idx / K) * K;
-    float s = 0.0f;
-    for (int q = 0; q < S; q++) s += ws[((size_t)q * Co + co) * Kp + k];
-    gw[idx] = s;
-}
-
-// per-chunk column sums of dZ (bias gradient), then their ordered sum
-__global__ void k_colsum(const bf16* __restrict__ dZ, int M, int C, int chunk, float* __restrict__ ws) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    int s = blockIdx.y;
-    if (c >= C) return;
-    int mbeg = s * chunk, mend = min(M, mbeg + chunk);
-    float acc = 0.0f;
-    for (int m = mbeg; m < mend; m++) acc += bf2f(dZ[(size_t)m * C + c]);
-    ws[(size_t)s * C + c] = acc;
-}
-__global__ void k_reduce_rows(const float* __restrict__ ws, int S, int width, float* __restrict__ out) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= width) return;
-    float s = 0.0f;
-    for (int q = 0; q < S; q++) s += ws[(size_t)q * width + k];
-    out[k] = s;
+// Column sums of the backward pass's partial results, all in one launch: sum i
+// adds the rows of an S x width matrix (width a multiple of 2) into out; a
+// weight gradient's columns past K of each Kp-column group are padding. A
+// workgroup of 1024 threads takes 2 * 64 * (16 / slices) columns; wave `slice`
+// of a column group adds rows slice, slice + slices, ..., the slices then meet
+// in order (deterministic). One thread per column over all rows took 690 us
+// over the 14 sums of a 256-sample step; this launch takes 26 us.
+struct RowSum {
+    const float* src;
+    float* out;
+    int S, width, K, Kp, slices, block0;
+};
+constexpr int ROW_SUMS = 14;
+struct RowSums {
+    RowSum s[ROW_SUMS];
+    int n;
+};
+__global__ __launch_bounds__(1024) void k_row_sums(RowSums a) {
+    __shared__ float2 part[16][64];
+    int i = 0;
+    while (i + 1 < a.n && (int)blockIdx.x >= a.s[i + 1].block0) i++;
+    const RowSum& r = a.s[i];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int slices = r.slices, groups = 16 / slices, grp = w / slices, slice = w - grp * slices;
+    const int c = 2 * (64 * (((int)blockIdx.x - r.block0) * groups + grp) + lane);
+    float2 v = make_float2(0.0f, 0.0f);
+    if (c < r.width) {
+        const float* p = r.src + c;
+#pragma unroll 8
+        for (int q = slice; q < r.S; q += slices) {
+            const float2 u = *(const float2*)(p + (size_t)q * r.width);
+            v.x += u.x;
+            v.y += u.y;
+        }
+    }
+    part[w][lane] = v;
+    __syncthreads();
+    if (slice == 0 && c < r.width) {
+        for (int q = 1; q < slices; q++) {
+            const float2 u = part[w + q][lane];
+            v.x += u.x;
+            v.y += u.y;
+        }
+        const int row = r.Kp ? c / r.Kp : 0, k = c - row * r.Kp;  // Kp is even: both columns in one row
+        if (!r.Kp || k < r.K) r.out[r.Kp ? (size_t)row * r.K + k : (size_t)c] = v.x;
+        if (!r.Kp || k + 1 < r.K) r.out[r.Kp ? (size_t)row * r.K + k + 1 : (size_t)c + 1] = v.y;
+    }
 }
 
 // ---------------------------------------------------------------- head
 // One block per sample: mean pool, dense 6 outputs; with targets also the loss,
 // the dense-layer gradient contributions and dZ of the last convolution.
-// 1 / max(1, sum of the sample weights), in order
-__global__ void k_weight_norm(const float* __restrict__ wn, int n, float* __restrict__ inv_norm) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    float s = 0.0f;
-    for (int i = 0; i < n; i++) s += wn[i];
-    *inv_norm = 1.0f / fmaxf(1.0f, s);
-}
-
 __global__ __launch_bounds__(256) void k_head(int P6, int C6, const bf16* __restrict__ A6, const float* __restrict__ Wfc,
                                               const float* __restrict__ bfc, const float* __restrict__ y,
-                                              const float* __restrict__ wn, const float* __restrict__ inv_norm_p,
-                                              float* __restrict__ out,
+                                              const float* __restrict__ wn, int nw, float* __restrict__ out,
                                               bf16* __restrict__ dZ6, float* __restrict__ ws_fc, float* __restrict__ ws_loss) {
     extern __shared__ float sh[];  // h[C6], dh[C6]
     __shared__ float red[4][6];
     __shared__ float o6[6], d6[6];
     const int n = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const float inv_norm = y ? *inv_norm_p : 0.0f;
+    // 1 / max(1, sum of the nw sample weights): every block forms the same sum
+    float inv_norm = 0.0f;
+    if (y) {
+        float s = 0.0f;
+        for (int i = t; i < nw; i += 256) s += wn[i];
+        for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+        if (lane == 0) red[wv][0] = s;
+        __syncthreads();
+        inv_norm = 1.0f / fmaxf(1.0f, (red[0][0] + red[1][0]) + (red[2][0] + red[3][0]));
+        __syncthreads();
+    }
     float* h = sh;
     for (int c = t; c < C6; c += 256) {
         float s = 0.0f;
@@ -785,7 +1038,8 @@ __global__ __launch_bounds__(256) void k_head(int P6, int C6, const bf16* __rest
     if (t == 0) {
         float l = 0.0f;
         for (int j = 0; j < 6; j++) { float e = o6[j] - y[n * 6 + j]; l += e * e; }
-        ws_loss[n] = wn[n] * l * inv_norm;
+        ws_loss[2 * n] = wn[n] * l * inv_norm;  // rows of 2 columns, for the column sums
+        ws_loss[2 * n + 1] = 0.0f;
     }
     const int width = 6 * C6 + 6;
     float* dh = sh + C6;
@@ -950,7 +1204,7 @@ struct rt_cnn {
     bf16 *dz_a = nullptr, *dz_b = nullptr;
     bf16* xin = nullptr;        // inputs built by rt_batch_propose
     float *ws = nullptr, *ws_b = nullptr, *ws_fc = nullptr, *ws_loss = nullptr, *out = nullptr, *loss = nullptr;
-    size_t ws_floats = 0, ws_b_floats = 0;
+    size_t ws_off[6], wsb_off[6];  // of each layer in ws and ws_b
     FrameSrc* src_dev = nullptr;
     int* flags_dev = nullptr;
     float* trel_tmp = nullptr;
@@ -985,15 +1239,18 @@ static size_t act_elems(const rt_cnn* net, int l, int B) {
     return (size_t)B * net->H[l] * net->W[l] * net->cfg.channels[l];
 }
 
-// weight-gradient split: chunks of output pixels (multiple of 16) so that the
-// grid holds about 2048 waves
+// Weight-gradient split of layer l: chunks of output pixels (multiples of the
+// kernel's stage) so that the grid holds about two workgroups per CU; at most
+// wsplit_max parts for any batch up to B.
+static int wsplit_max(const rt_cnn* net, int l, int B) {
+    const int M = B * net->H[l + 1] * net->W[l + 1];
+    const int tiles = ((net->cfg.channels[l + 1] + 63) / 64) * ((net->Kp[l] + 63) / 64);
+    return std::max(1, std::min(512 / tiles, (M + BW_M - 1) / BW_M));
+}
 static void wsplit(const rt_cnn* net, int l, int B, int* S, int* chunk) {
-    int M = B * net->H[l + 1] * net->W[l + 1];
-    int tiles = ((net->cfg.channels[l + 1] + 31) / 32) * (net->Kp[l] / 32);
-    int s = std::max(1, std::min(2048 / std::max(tiles, 1), (M + 15) / 16));
-    int c = ((M + s - 1) / s + 15) / 16 * 16;
-    *chunk = c;
-    *S = (M + c - 1) / c;
+    const int M = B * net->H[l + 1] * net->W[l + 1], s = wsplit_max(net, l, B);
+    *chunk = ((M + s - 1) / s + BW_M - 1) / BW_M * BW_M;
+    *S = (M + *chunk - 1) / *chunk;
 }
 
 extern "C" int rt_cnn_create(int device, const rt_cnn_config* c, int max_batch, rt_cnn** out) {
@@ -1026,17 +1283,12 @@ extern "C" int rt_cnn_create(int device, const rt_cnn_config* c, int max_batch, 
     net->nparams = o;
     // workspace sizes
     size_t wsf = 0, wsb = 0, maxact = 0;
-    for (int l = 0; l < 6; l++) {
-        // wsplit never uses more than 2048 / tiles splits, whatever the batch
-        int tiles = ((cfg.channels[l + 1] + 31) / 32) * (net->Kp[l] / 32);
-        int S = std::max(1, 2048 / std::max(tiles, 1));
-        wsf = std::max(wsf, (size_t)S * cfg.channels[l + 1] * net->Kp[l]);
-        int M = max_batch * net->H[l + 1] * net->W[l + 1];
-        int Sb = std::min(1024, (M + 255) / 256);
-        wsb = std::max(wsb, (size_t)Sb * cfg.channels[l + 1]);
+    for (int l = 0; l < 6; l++) {  // every layer's parts at once: one launch sums them all
+        const size_t S = wsplit_max(net, l, max_batch);
+        net->ws_off[l] = wsf; wsf += S * cfg.channels[l + 1] * net->Kp[l];
+        net->wsb_off[l] = wsb; wsb += S * cfg.channels[l + 1];
     }
     for (int l = 1; l < 7; l++) maxact = std::max(maxact, act_elems(net, l, max_batch));
-    net->ws_floats = wsf; net->ws_b_floats = wsb;
     bool ok = hipStreamCreateWithFlags(&net->stream, hipStreamNonBlocking) == hipSuccess;
     auto al = [&](void** p, size_t bytes) {
         if (!ok) return;
@@ -1055,7 +1307,7 @@ extern "C" int rt_cnn_create(int device, const rt_cnn_config* c, int max_batch, 
     al((void**)&net->xin, 2 * act_elems(net, 0, max_batch));
     al((void**)&net->ws, 4 * wsf); al((void**)&net->ws_b, 4 * wsb);
     al((void**)&net->ws_fc, 4 * (size_t)max_batch * (6 * cfg.channels[6] + 6));
-    al((void**)&net->ws_loss, 4 * (size_t)max_batch);
+    al((void**)&net->ws_loss, 8 * (size_t)max_batch);
     al((void**)&net->out, 4 * 6 * (size_t)max_batch);
     al((void**)&net->loss, 256);
     al((void**)&net->src_dev, sizeof(FrameSrc) * (size_t)max_batch);
@@ -1200,40 +1452,71 @@ static int forward(rt_cnn* net, int n, const bf16* x, hipStream_t s, bool keep =
     return hipGetLastError() == hipSuccess ? RT_OK : set_error(RT_ERR_HIP, "rt_cnn forward launch");
 }
 
+// The input gradient of one layer. The parity-class kernel takes Cout and Cin
+// that are multiples of 32 (a stage of k then lies in one tap, a tile's
+// columns in the tensor); 16-channel layers run the general kernel. The tile
+// is the largest that still gives 512 workgroups, since a workgroup's stages
+// wait on their loads one after the other.
+static void backward_data(const ConvGeom& g, const bf16* dZ, const bf16* WT, const bf16* X, bf16* dX, hipStream_t s) {
+    if (g.Co % 32 || g.Ci % 32) {
+        const int Mi = g.B * g.Hi * g.Wi;
+        k_conv_bwd_data<<<dim3((Mi + 63) / 64, (g.Ci + 63) / 64), 256, 0, s>>>(g, dZ, WT, X, dX);
+        return;
+    }
+    const int M = g.B * ((g.Hi + 1) / 2) * ((g.Wi + 1) / 2);  // the largest class
+    const int bn = g.Ci % 64 ? 32 : 64;
+    auto grid = [&](int bm) { return dim3((M + bm - 1) / bm, g.Ci / bn, 4); };
+    auto blocks = [&](int bm) { return (long)grid(bm).x * grid(bm).y * 4; };
+    if (bn == 32) {
+        k_conv_bwd_data_lds<128, 32, 4, 32><<<grid(128), 256, 0, s>>>(g, dZ, WT, X, dX);
+    } else if (blocks(128) >= 512) {
+        k_conv_bwd_data_lds<128, 64, 4, 32><<<grid(128), 256, 0, s>>>(g, dZ, WT, X, dX);
+    } else if (g.Co % 64) {
+        k_conv_bwd_data_lds<64, 64, 2, 32><<<grid(64), 256, 0, s>>>(g, dZ, WT, X, dX);
+    } else if (blocks(64) >= 512) {
+        k_conv_bwd_data_lds<64, 64, 2, 64><<<grid(64), 256, 0, s>>>(g, dZ, WT, X, dX);
+    } else {
+        k_conv_bwd_data_lds<32, 64, 2, 64><<<grid(32), 256, 0, s>>>(g, dZ, WT, X, dX);
+    }
+}
+
 // forward + backward into net->grads; loss into net->loss[0] (device)
 static int loss_grad(rt_cnn* net, int n, const bf16* x, const float* y, const float* wn, hipStream_t s) {
     int rc = forward(net, n, x, s, true);
     if (rc) return rc;
-    k_weight_norm<<<1, 64, 0, s>>>(wn, n, net->loss + 1);
     const int C6 = net->cfg.channels[6], P6 = net->H[6] * net->W[6];
     bf16* dz = net->dz_a;
     bf16* dz_other = net->dz_b;
-    k_head<<<n, 256, 2 * C6 * 4, s>>>(P6, C6, net->act[6], net->params + net->fc_w, net->params + net->fc_b, y, wn,
-                                      net->loss + 1, net->out, dz, net->ws_fc, net->ws_loss);
-    int width = 6 * C6 + 6;
-    k_reduce_rows<<<(width + 255) / 256, 256, 0, s>>>(net->ws_fc, n, width, net->grads + net->fc_w);
-    k_reduce_rows<<<1, 256, 0, s>>>(net->ws_loss, n, 1, net->loss);
+    k_head<<<n, 256, 2 * C6 * 4, s>>>(P6, C6, net->act[6], net->params + net->fc_w, net->params + net->fc_b, y, wn, n,
+                                      net->out, dz, net->ws_fc, net->ws_loss);
+    RowSums sums;
+    sums.n = 0;
+    int blocks = 0;
+    auto add = [&](const float* src, float* out, int S, int width, int K, int Kp) {
+        int slices = 1;
+        while (slices < 16 && slices < S) slices *= 2;
+        sums.s[sums.n++] = RowSum{src, out, S, width, K, Kp, slices, blocks};
+        const int cols = 2 * 64 * (16 / slices);
+        blocks += (width + cols - 1) / cols;
+    };
     for (int l = 5; l >= 0; l--) {
         ConvGeom g = geom(net, l, n);
-        int M = n * g.Ho * g.Wo;
         int S, chunk;
         wsplit(net, l, n, &S, &chunk);
-        dim3 gw((g.Co + 31) / 32, g.Kp / 32, S);
-        k_conv_bwd_w<<<gw, 64, 0, s>>>(g, dz, net->act[l], net->ws, chunk);
-        int nw = g.Co * g.K;
-        k_reduce_w<<<(nw + 255) / 256, 256, 0, s>>>(net->ws, S, g.Co, g.Kp, g.K, net->grads + net->w_off[l]);
-        int Sb = std::min(1024, (M + 255) / 256);
-        int cb = (M + Sb - 1) / Sb;
-        Sb = (M + cb - 1) / cb;
-        k_colsum<<<dim3((g.Co + 255) / 256, Sb), 256, 0, s>>>(dz, M, g.Co, cb, net->ws_b);
-        k_reduce_rows<<<(g.Co + 255) / 256, 256, 0, s>>>(net->ws_b, Sb, g.Co, net->grads + net->b_off[l]);
+        float* ws = net->ws + net->ws_off[l];
+        float* ws_b = net->ws_b + net->wsb_off[l];
+        dim3 gw((g.Co + 63) / 64, (g.Kp + 63) / 64, S);
+        k_conv_bwd_w<<<gw, 256, 0, s>>>(g, dz, net->act[l], ws, ws_b, chunk);
+        add(ws, net->grads + net->w_off[l], S, g.Co * g.Kp, g.K, g.Kp);
+        add(ws_b, net->grads + net->b_off[l], S, g.Co, 0, 0);
         if (l > 0) {
-            int Mi = n * g.Hi * g.Wi;
-            dim3 gd((Mi + 63) / 64, (g.Ci + 63) / 64);
-            k_conv_bwd_data<<<gd, 256, 0, s>>>(g, dz, net->WT[l], net->act[l], dz_other);
+            backward_data(g, dz, net->WT[l], net->act[l], dz_other, s);
             std::swap(dz, dz_other);
         }
     }
+    add(net->ws_fc, net->grads + net->fc_w, n, 6 * C6 + 6, 0, 0);
+    add(net->ws_loss, net->loss, n, 2, 0, 0);
+    k_row_sums<<<blocks, 1024, 0, s>>>(sums);
     return hipGetLastError() == hipSuccess ? RT_OK : set_error(RT_ERR_HIP, "rt_cnn backward launch");
 }
 
@@ -1250,7 +1533,7 @@ extern "C" int rt_cnn_forward(rt_cnn* net, int n, const uint16_t* x_dev, float* 
     if ((rc = forward(net, n, x_dev, net->stream))) return rc;
     const int C6 = net->cfg.channels[6], P6 = net->H[6] * net->W[6];
     k_head<<<n, 256, 2 * C6 * 4, net->stream>>>(P6, C6, net->act[6], net->params + net->fc_w, net->params + net->fc_b,
-                                                nullptr, nullptr, nullptr, out_dev, nullptr, nullptr, nullptr);
+                                                nullptr, nullptr, 0, out_dev, nullptr, nullptr, nullptr);
     if (hipGetLastError() != hipSuccess) return set_error(RT_ERR_HIP, "rt_cnn head launch");
     return RT_OK;
 }
@@ -1351,7 +1634,7 @@ int cnn_propose(rt_cnn* net, int n, const FrameSrc* src, float* trel_dev, hipStr
     if ((rc = forward(net, n, x, s))) return rc;
     const int C6 = net->cfg.channels[6], P6 = net->H[6] * net->W[6];
     k_head<<<n, 256, 2 * C6 * 4, s>>>(P6, C6, net->act[6], net->params + net->fc_w, net->params + net->fc_b, nullptr,
-                                      nullptr, nullptr, net->out, nullptr, nullptr, nullptr);
+                                      nullptr, 0, net->out, nullptr, nullptr, nullptr);
     k_outputs_to_trel<<<(n + 255) / 256, 256, 0, s>>>(net->out, n, net->cfg.rot_scale_deg * (float)(M_PI / 180.0),
                                                       net->cfg.trans_scale_mm, trel_dev);
     return hipGetLastError() == hipSuccess ? RT_OK : set_error(RT_ERR_HIP, "rt_batch_propose launch");

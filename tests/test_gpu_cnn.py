@@ -94,6 +94,35 @@ def test_gradients_match_oracle(kw, B):
         assert err < 2e-2, (name, err)
 
 
+def _grad_errors(cfg, net, B, seed):
+    p, xr, xb, y, wn = case(cfg, B, seed)
+    net.set_params(p)
+    xd, yd, wd = DeviceBuffer.from_array(xb), DeviceBuffer.from_array(y), DeviceBuffer.from_array(wn)
+    loss, out, g = net.loss_grad(B, xd.ptr, yd.ptr, wd.ptr)
+    rl, rout, rg = oracle_fb(cfg, p, xr, y, wn)
+    assert abs(loss - rl) <= 2e-3 * max(1.0, abs(rl))
+    layers, fc_w, fc_b, total = layout(cfg)
+    spans = [(f"W{l}", w, b) for l, (w, b, co, ci) in enumerate(layers)] + \
+            [(f"b{l}", b, b + co) for l, (w, b, co, ci) in enumerate(layers)] + [("Wfc", fc_w, fc_b), ("bfc", fc_b, total)]
+    return {name: np.linalg.norm(g[a:b] - rg[a:b]) / max(np.linalg.norm(rg[a:b]), 1e-12) for name, a, b in spans}
+
+
+# Odd maps (parity classes of unequal size, one row or column, tiles and pixel
+# chunks that end inside), one sample, layers of 16 channels beside ones of 32
+# and more, several pixel chunks per layer, and the widest pixel tile.
+@pytest.mark.parametrize("kw,B,most", [
+    (dict(channels=[4, 32, 64, 128, 32, 64, 32], in_width=21, in_height=13), 1, 1),
+    (dict(channels=[4, 32, 64, 128, 32, 64, 32], in_width=21, in_height=13), 7, 40),
+    (dict(channels=[4, 16, 32, 64, 16, 128, 64], in_width=35, in_height=50), 9, 9),
+    ({}, 37, 64),
+    (dict(channels=[4, 64, 64, 16, 16, 16, 16]), 55, 55)])
+def test_gradients_at_tile_edges(kw, B, most):
+    print(f"case cnn gradient tiles {kw} B={B}", flush=True)
+    cfg = default_config(**kw)
+    err = _grad_errors(cfg, PoseNet(most, config=cfg), B, 5)
+    assert max(err.values()) < 2e-2, err
+
+
 def test_adam_step_matches_closed_form():
     print("case cnn adam", flush=True)
     cfg = default_config(**SMALL)
