@@ -171,6 +171,110 @@ __device__ __forceinline__ void reduce27(const double* acc, double* part, int gr
         part[(size_t)k * stride + group] = sum;
     }
 }
+// The end of an iteration: the photometric partials (gp groups of part) and the
+// geometric ones (gi groups of part2) combined in FP64, then the FP64 solve and
+// the pose update on one wave (solve_update_wave) from an LDS copy of the
+// system. It opens the next kernel that needs the pose and runs in every
+// workgroup of it alike (workgroup 0 also stores the pose): a launch of its own
+// (k_solve) costs a kernel boundary and another round trip to memory per
+// iteration. Measured with the separate launch and without: a 320x240
+// photometric pair of 8192 points 277 and 270 us, a 640x480 geometric pair 507
+// and 457 us. Bound by latency: kernel start, the partials' round trip, the
+// serial FP64 solve (1.4 us), the taps' round trip, the kernel's end.
+// Wave w sums terms w, w + NW, ... of the 54; lane l adds groups l, l + 64, ...
+// in order (all its loads issued first), then the lanes' sums meet in a fixed
+// exchange tree: the same order for every workgroup size. No update from an
+// empty geometric selection (nptr non-null with *nptr = 0).
+constexpr int COMBINE_LOADS = (PART_STRIDE + 63) / 64;  // groups per lane
+struct SolveIn {
+    const double* part;
+    const double* part2;
+    int gp, gi;
+    const int* nptr;
+    const float* tin;   // the pose before the update
+    float* tout;        // where workgroup 0 stores the updated pose
+    SolveCfg cfg;
+    int N1;
+    int pending;        // 0: no update, the pose is tin
+};
+struct SolveLds {
+    double ws[SOLVE_WS];
+    double sys[56];
+    float T[16];
+};
+template <int NT>
+__device__ __forceinline__ void combine_terms(const SolveIn& in, double* lsys, double* sys) {
+    constexpr int NW = NT / 64, TERMS = (54 + NW - 1) / NW;
+    const int wave = threadIdx.x >> 6, lane = lane_id();
+    double v[TERMS][COMBINE_LOADS];
+#pragma unroll
+    for (int j = 0; j < TERMS; j++) {
+        const int k = wave + NW * j;
+        const bool geo = k >= 27;
+        const int groups = k >= 54 ? 0 : (geo ? in.gi : in.gp);
+        const double* src = (geo ? in.part2 : in.part) + (size_t)(geo ? k - 27 : k) * PART_STRIDE;
+#pragma unroll
+        for (int i = 0; i < COMBINE_LOADS; i++) {
+            const int g = lane + 64 * i;
+            v[j][i] = g < groups ? src[g] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < TERMS; j++) {
+        const int k = wave + NW * j;
+        const int groups = k >= 54 ? 0 : (k >= 27 ? in.gi : in.gp);
+        if (groups == 0) continue;  // the wave's term k: the same for its lanes
+        double acc = 0.0;
+#pragma unroll
+        for (int i = 0; i < COMBINE_LOADS; i++) acc += v[j][i];
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
+        if (lane == 0) {
+            lsys[k] = acc;
+            if (sys) sys[k] = acc;
+        }
+    }
+}
+// The pose of the iteration that starts here, in q.T: ends with a barrier.
+template <int NT>
+__device__ __forceinline__ void solve_pending(const SolveIn& in, SolveLds& q) {
+    const int t = threadIdx.x;
+    if (t < 16) q.T[t] = in.tin[t];
+    if (in.pending) {
+        const int n2 = in.nptr ? *in.nptr : 1;
+        combine_terms<NT>(in, q.sys, nullptr);
+        __syncthreads();
+        if (t < 64 && n2 > 0) solve_update_wave(q.sys, q.T, in.cfg, in.N1, n2, q.ws);
+        __syncthreads();
+        if (blockIdx.x == 0 && t < 16) in.tout[t] = q.T[t];
+    } else {
+        __syncthreads();
+    }
+}
+// The frame's last update (solve), or the combined system alone for
+// inspection: the system to sys, the MAD histogram kept for inspection and
+// cleared (madhist non-null).
+constexpr int SOLVE_THREADS = 512;  // 8 waves, 2 per SIMD: room for the FP64 solve
+__global__ __launch_bounds__(SOLVE_THREADS) void k_solve(SolveIn in, unsigned* madhist, unsigned* madcopy, double* sys,
+                                                         int solve) {
+    __shared__ SolveLds q;
+    const int t = threadIdx.x;
+    if (t < 16) q.T[t] = in.tin[t];
+    const int n2 = in.nptr ? *in.nptr : 1;
+    unsigned mh = 0u;
+    if (madhist && t < 256) mh = madhist[t];
+    combine_terms<SOLVE_THREADS>(in, q.sys, sys);
+    if (madhist && t < 256) {
+        madcopy[t] = mh;
+        madhist[t] = 0u;
+    }
+    if (!solve) return;
+    __syncthreads();
+    if (t < 64 && n2 > 0) solve_update_wave(q.sys, q.T, in.cfg, in.N1, n2, q.ws);
+    __syncthreads();
+    if (t < 16) in.tout[t] = q.T[t];
+}
+
 // ------------------------------------------------------------------ A10 + A11
 // interpolateResidualKernel2 (warp.cu:269-332) with the level mapping of
 // interpolateResidual2 (:1160-1218); the MAD histogram of discretizeResidual
@@ -179,24 +283,32 @@ template <int NT>
 __device__ __forceinline__ void photo_res_body(const float4* __restrict__ pts, const float4* __restrict__ jac, int N,
                                                int layer, const float* __restrict__ img, int wl, int hl,
                                                const float* __restrict__ zcur, int W, int H,
-                                               const float* __restrict__ c, const float* __restrict__ trel, int bins,
+                                               const float* __restrict__ c, const SolveIn& in, int bins,
                                                float2* __restrict__ res, unsigned* __restrict__ madhist, int grp,
                                                int ngrp) {
     __shared__ unsigned h[256];
+    __shared__ SolveLds q;
     if (threadIdx.x < 256) h[threadIdx.x] = 0u;
+    const JacView jv = jac_view(const_cast<float4*>(jac), N);
+    // the thread's first point is loaded before the solve, which does not need it
+    int i = grp * NT + threadIdx.x;
+    float4 p4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float iref = 0.0f;
+    if (i < N) { p4 = pts[i]; iref = jv.iref[i]; }
+    solve_pending<NT>(in, q);
     float T[16];
 #pragma unroll
-    for (int k = 0; k < 16; k++) T[k] = trel[k];
-    __syncthreads();
+    for (int k = 0; k < 16; k++) T[k] = q.T[k];
     float a = 1.0f / (float)(1 << layer);
     float b = 0.5f * (a - 1.0f);
-    JacView jv = jac_view(const_cast<float4*>(jac), N);
-    for (int i = grp * NT + threadIdx.x; i < N; i += ngrp * NT) {
+    while (i < N) {
         float ir, zW;
-        photo_point(pts[i], jv.iref[i], T, a, b, F32Src{img}, wl, hl, F32Src{zcur}, W, H, c, ir, zW);
+        photo_point(p4, iref, T, a, b, F32Src{img}, wl, hl, F32Src{zcur}, W, H, c, ir, zW);
         res[i] = make_float2(ir, zW);
         int bn = (int)((float)(bins - 1) * fabsf(ir));
         if (bn >= 0 && bn < bins) atomicAdd(&h[bn], 1u);
+        i += ngrp * NT;
+        if (i < N) { p4 = pts[i]; iref = jv.iref[i]; }
     }
     __syncthreads();
     if (threadIdx.x < bins) {
@@ -207,10 +319,9 @@ __device__ __forceinline__ void photo_res_body(const float4* __restrict__ pts, c
 __global__ __launch_bounds__(256) void k_photo_res(const float4* __restrict__ pts, const float4* __restrict__ jac,
                                                    int N, int layer, const float* __restrict__ img, int wl, int hl,
                                                    const float* __restrict__ zcur, int W, int H,
-                                                   const float* __restrict__ c, const float* __restrict__ trel,
-                                                   int bins, float2* __restrict__ res, unsigned* __restrict__ madhist) {
-    photo_res_body<256>(pts, jac, N, layer, img, wl, hl, zcur, W, H, c, trel, bins, res, madhist, blockIdx.x,
-                        gridDim.x);
+                                                   const float* __restrict__ c, SolveIn in, int bins,
+                                                   float2* __restrict__ res, unsigned* __restrict__ madhist) {
+    photo_res_body<256>(pts, jac, N, layer, img, wl, hl, zcur, W, H, c, in, bins, res, madhist, blockIdx.x, gridDim.x);
 }
 
 // The MAD histogram's median bin (generateWeights64Kernel, histogram64.cu:79-94):
@@ -258,24 +369,28 @@ __device__ __forceinline__ void fold_partials(const double* __restrict__ raw, in
 template <int NT>
 __device__ __forceinline__ void photo_sys_body(const float2* __restrict__ res, const float4* __restrict__ jac, int N,
                                                int bins, int robust, const unsigned* __restrict__ madhist,
-                                               float* __restrict__ wts, double* part, int grp, int ngrp) {
+                                               unsigned* __restrict__ madnext, float* __restrict__ wts, double* part,
+                                               int grp, int ngrp) {
     __shared__ int med;
     const int t = threadIdx.x;
+    // the thread's first point is loaded beside the median
+    JacView jv = jac_view(const_cast<float4*>(jac), N);
+    int i = grp * NT + t;
+    float2 rz = make_float2(0.0f, 0.0f), jb = make_float2(0.0f, 0.0f);
+    float4 ja = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (i < N) { rz = res[i]; ja = jv.a[i]; jb = jv.b[i]; }
     if (t < 64) med_bin(madhist, bins, N, &med);
+    if (grp == 0 && t < 256) madnext[t] = 0u;  // the next iteration's histogram, last read an iteration ago
     __syncthreads();
     float s = mad_scale(med, bins);
     double acc[27];
 #pragma unroll
     for (int k = 0; k < 27; k++) acc[k] = 0.0;
-    JacView jv = jac_view(const_cast<float4*>(jac), N);
-    for (int i = grp * NT + t; i < N; i += ngrp * NT) {
-        float2 rz = res[i];
+    while (i < N) {
         float r = rz.x;
         float w = robust_weight(r, rz.y, s, robust);
         float wr = r * w;
         wts[i] = w;
-        float4 ja = jv.a[i];
-        float2 jb = jv.b[i];
         float jw[6] = {ja.x * w, ja.y * w, ja.z * w, ja.w * w, jb.x * w, jb.y * w};
         int k = 0;
 #pragma unroll
@@ -284,6 +399,8 @@ __device__ __forceinline__ void photo_sys_body(const float2* __restrict__ res, c
             for (int c0 = r0; c0 < 6; c0++) acc[k++] += (double)(jw[r0] * jw[c0]);
 #pragma unroll
         for (int r0 = 0; r0 < 6; r0++) acc[21 + r0] += (double)(jw[r0] * wr);
+        i += ngrp * NT;
+        if (i < N) { rz = res[i]; ja = jv.a[i]; jb = jv.b[i]; }
     }
     reduce27<NT>(acc, part, grp);
 }
@@ -292,70 +409,40 @@ __device__ __forceinline__ void photo_sys_body(const float2* __restrict__ res, c
 template <int NT>
 __global__ __launch_bounds__(NT) void k_photo_sys(const float2* __restrict__ res, const float4* __restrict__ jac,
                                                   int N, int bins, int robust, const unsigned* __restrict__ madhist,
-                                                  float* __restrict__ wts, double* part, int gs,
+                                                  unsigned* __restrict__ madnext, float* __restrict__ wts,
+                                                  double* part, int gs,
                                                   const double* __restrict__ raw, int nraw, double* fold, int nf) {
     if ((threadIdx.x >> 6) == 1) fold_partials(raw, nraw, fold, nf, blockIdx.x, threadIdx.x - 64);
-    if ((int)blockIdx.x < gs) photo_sys_body<NT>(res, jac, N, bins, robust, madhist, wts, part, blockIdx.x, gs);
+    if ((int)blockIdx.x < gs) photo_sys_body<NT>(res, jac, N, bins, robust, madhist, madnext, wts, part, blockIdx.x, gs);
 }
 
-// The end of an iteration, one workgroup of 512 threads: the photometric
-// partials (gp groups) into sys[0..27) and the geometric ones (gi groups) into
-// sys[27..54) in FP64, the MAD histogram kept for inspection and cleared for
-// the next iteration (madhist non-null), then, when solve is set, the FP64
-// solve and the pose update on one wave (solve_update_wave) from an LDS copy
-// of the system. A separate launch instead of the last workgroup of the system
-// pass: electing that workgroup needs a device-scope fence in every workgroup,
-// which writes back the L2.
-// Wave w sums terms w, w + 8, ..., w + 48 of the 54; lane l adds groups
-// l, l + 64, ... in order (all its loads issued first), then the lanes' sums
-// meet in a fixed exchange tree: the same order for every call. No update
-// from an empty geometric selection (nptr non-null with *nptr = 0).
-constexpr int SOLVE_THREADS = 512;  // 8 waves, 2 per SIMD: room for the FP64 solve
-constexpr int SOLVE_TERMS = 7;     // terms per wave (8 x 7 >= 54)
-constexpr int COMBINE_LOADS = (PART_STRIDE + 63) / 64;  // groups per lane
-__global__ __launch_bounds__(SOLVE_THREADS) void k_solve(const double* __restrict__ part, int gp,
-                                                         const double* __restrict__ part2, int gi, unsigned* madhist,
-                                                         const int* __restrict__ nptr, double* sys, float* trel,
-                                                         SolveCfg cfg, int solve, int N1) {
-    __shared__ double ws[SOLVE_WS];
-    __shared__ double lsys[56];
-    const int t = threadIdx.x, wave = t >> 6, lane = lane_id();
-    const int n2 = nptr ? *nptr : 1;
-    double v[SOLVE_TERMS][COMBINE_LOADS];
-#pragma unroll
-    for (int j = 0; j < SOLVE_TERMS; j++) {
-        const int k = wave + 8 * j;
-        const bool geo = k >= 27;
-        const int groups = k >= 54 ? 0 : (geo ? gi : gp);
-        const double* src = (geo ? part2 : part) + (size_t)(geo ? k - 27 : k) * PART_STRIDE;
-#pragma unroll
-        for (int i = 0; i < COMBINE_LOADS; i++) {
-            const int g = lane + 64 * i;
-            v[j][i] = g < groups ? src[g] : 0.0;
-        }
+// The sums of (w r)^2 and w^2 over the selected points of the last iteration,
+// one FP64 partial pair per workgroup (part[2 g], part[2 g + 1]): the host adds
+// RMS_GROUPS pairs instead of copying 12 bytes per point (61,440 points: 150 us
+// for the copy and the host's loop, 18 us with the launch here).
+__global__ __launch_bounds__(256) void k_residual_rms(const float2* __restrict__ res, const float* __restrict__ wts, int N,
+                                                      double* __restrict__ part) {
+    __shared__ double2 ws[4];
+    double a = 0.0, b = 0.0;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256) {
+        const double w = wts[i], wr = w * res[i].x;
+        a += wr * wr;
+        b += w * w;
     }
-    unsigned mh = 0u;
-    if (madhist && t < 256) mh = madhist[t];
 #pragma unroll
-    for (int j = 0; j < SOLVE_TERMS; j++) {
-        const int k = wave + 8 * j;
-        double acc = 0.0;
-#pragma unroll
-        for (int i = 0; i < COMBINE_LOADS; i++) acc += v[j][i];
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
-        const int groups = k >= 54 ? 0 : (k >= 27 ? gi : gp);
-        if (lane == 0 && k < 54) {
-            lsys[k] = acc;
-            if (groups > 0) sys[k] = acc;
-        }
+    for (int o = 32; o >= 1; o >>= 1) {
+        a += __shfl_xor(a, o, 64);
+        b += __shfl_xor(b, o, 64);
     }
-    if (madhist && t < 256) {
-        madhist[256 + t] = mh;
-        madhist[t] = 0u;
-    }
+    if (lane_id() == 0) ws[threadIdx.x >> 6] = make_double2(a, b);
     __syncthreads();
-    if (solve && wave == 0 && n2 > 0) solve_update_wave(lsys, trel, cfg, N1, n2, ws);
+    if (threadIdx.x == 0) {
+        part[2 * blockIdx.x] = (ws[0].x + ws[1].x) + (ws[2].x + ws[3].x);
+        part[2 * blockIdx.x + 1] = (ws[0].y + ws[1].y) + (ws[2].y + ws[3].y);
+    }
+}
+void launch_residual_rms(const Dev& d, hipStream_t s) {
+    k_residual_rms<<<RMS_GROUPS, 256, 0, s>>>(d.res, d.wts, d.N, d.rms);
 }
 
 int photo_groups(int N) {
@@ -370,29 +457,57 @@ static int sys_groups(int n) {
 // The photometric system pass: 256-thread workgroups while SYS_GROUPS of them
 // cover the points (one point per thread), else SYS_THREADS. Also folds nraw
 // raw geometric partials into nf groups. Returns its number of groups.
-static int launch_photo_sys(const Dev& d, int layer, const SolveCfg& c, const double* raw, int nraw, double* fold,
-                            int nf, hipStream_t s) {
+static int launch_photo_sys(const Dev& d, int layer, const SolveCfg& c, int it, const double* raw, int nraw,
+                            double* fold, int nf, hipStream_t s) {
+    unsigned* hist = d.madhist + (it & 1 ? 512 : 0);
+    unsigned* next = d.madhist + (it & 1 ? 0 : 512);
     const int g256 = (d.N + 255) / 256;
     if (g256 <= SYS_GROUPS) {
         const int gs = g256 < 1 ? 1 : g256;
-        k_photo_sys<256><<<gs > nf ? gs : nf, 256, 0, s>>>(d.res, d.jac[layer], d.N, c.mad_bins, c.robust, d.madhist,
+        k_photo_sys<256><<<gs > nf ? gs : nf, 256, 0, s>>>(d.res, d.jac[layer], d.N, c.mad_bins, c.robust, hist, next,
                                                            d.wts, d.part, gs, raw, nraw, fold, nf);
         return gs;
     }
     const int gs = sys_groups(d.N);
     k_photo_sys<SYS_THREADS><<<gs > nf ? gs : nf, SYS_THREADS, 0, s>>>(d.res, d.jac[layer], d.N, c.mad_bins, c.robust,
-                                                                       d.madhist, d.wts, d.part, gs, raw, nraw, fold,
+                                                                       hist, next, d.wts, d.part, gs, raw, nraw, fold,
                                                                        nf);
     return gs;
 }
 
-void launch_photo_iteration(const Dev& d, int layer, const SolveCfg& c, int finish, hipStream_t s) {
+// The solve that the next kernel starts with: consumes the pending one.
+static SolveIn take_pending(const Dev& d, const SolveCfg& c, EstState& e) {
+    SolveIn in;
+    in.part = d.part; in.part2 = e.part2; in.gp = e.gp; in.gi = e.gi; in.nptr = e.nptr;
+    in.tin = e.T; in.tout = e.T; in.cfg = c; in.N1 = d.N; in.pending = e.pending;
+    if (e.pending) {
+        in.tout = e.T == d.tbuf[0] ? d.tbuf[1] : d.tbuf[0];
+        e.T = in.tout;
+        e.pending = false;
+    }
+    return in;
+}
+static void set_pending(EstState& e, int gp, int gi, const double* part2, const int* nptr) {
+    e.pending = true;
+    e.gp = gp; e.gi = gi; e.part2 = part2; e.nptr = nptr;
+    e.it++;
+}
+void launch_finish(const Dev& d, const SolveCfg& c, EstState& e, int finish, hipStream_t s) {
+    if (!e.pending) return;
+    SolveIn in = take_pending(d, c, e);
+    in.tout = d.trel;
+    e.T = d.trel;
+    unsigned* hist = in.gp > 0 ? d.madhist + ((e.it - 1) & 1 ? 512 : 0) : nullptr;
+    k_solve<<<1, SOLVE_THREADS, 0, s>>>(in, hist, d.madhist + 256, d.sys, finish == FINISH_SOLVE ? 1 : 0);
+}
+
+void launch_photo_iteration(const Dev& d, int layer, const SolveCfg& c, EstState& e, hipStream_t s) {
     int G = photo_groups(d.N);
     k_photo_res<<<G, 256, 0, s>>>(d.pts, d.jac[layer], d.N, layer, d.cur.gray[layer], d.W >> layer, d.H >> layer,
-                                  d.cur.z, d.W, d.H, d.calib, d.trel, c.mad_bins, d.res, d.madhist);
-    const int Gs = launch_photo_sys(d, layer, c, nullptr, 0, nullptr, 0, s);
-    k_solve<<<1, SOLVE_THREADS, 0, s>>>(d.part, Gs, nullptr, 0, d.madhist, nullptr, d.sys, d.trel, c,
-                                        finish == FINISH_SOLVE ? 1 : 0, d.N);
+                                  d.cur.z, d.W, d.H, d.calib, take_pending(d, c, e), c.mad_bins, d.res,
+                                  d.madhist + (e.it & 1 ? 512 : 0));
+    const int Gs = launch_photo_sys(d, layer, c, e.it, nullptr, 0, nullptr, 0, s);
+    set_pending(e, Gs, 0, nullptr, nullptr);
 }
 
 // ------------------------------------------------------------------ A18 + A19
@@ -523,14 +638,15 @@ void launch_cur_cloud(const Dev& d, hipStream_t s) {
 // icpResidualKernel2 (rgb2gray.cu:223-260) over 1024-pixel row-major chunks;
 // the valid flags are kept as wave ballots for the ordered compaction.
 __global__ __launch_bounds__(1024) void k_icp_mask(const float4* __restrict__ rp, const float4* __restrict__ rn, int w,
-                                                   int h, int layer, const float* __restrict__ trel,
-                                                   const float* __restrict__ c, const float4* __restrict__ cp,
-                                                   float* __restrict__ rfull, uint64_t* __restrict__ bits,
-                                                   int* __restrict__ cnt) {
+                                                   int h, int layer, SolveIn in, const float* __restrict__ c,
+                                                   const float4* __restrict__ cp, float* __restrict__ rfull,
+                                                   uint64_t* __restrict__ bits, int* __restrict__ cnt) {
     __shared__ int wc[16];
+    __shared__ SolveLds q;
+    solve_pending<1024>(in, q);
     float T[16];
 #pragma unroll
-    for (int k = 0; k < 16; k++) T[k] = trel[k];
+    for (int k = 0; k < 16; k++) T[k] = q.T[k];
     int o = blockIdx.x * 1024 + threadIdx.x;
     bool valid = false;
     if (o < w * h) {
@@ -660,32 +776,32 @@ struct IcpSysArgs {
     int w, h, layer;
     const float* c;
     const float4* cp;
-    const float* trel;
     double* part;
     int stride;  // of part
     float scale_in;
 };
 template <int NT>
-__device__ __forceinline__ void icp_sys_body(const IcpSysArgs& g, int grp, int ngrp) {
+__device__ __forceinline__ void icp_sys_body(const IcpSysArgs& g, const SolveIn& in, int grp, int ngrp) {
+    __shared__ SolveLds q;
     const float4* __restrict__ rp = g.rp;
     const float4* __restrict__ rn = g.rn;
     const int* __restrict__ sel = g.sel;
     const float* __restrict__ r2 = g.r2;
     const float* __restrict__ c = g.c;
     const float4* __restrict__ cp = g.cp;
-    const float* __restrict__ trel = g.trel;
     const float* __restrict__ var = g.var;
     const int w = g.w, h = g.h, layer = g.layer;
     const float scale_in = g.scale_in;
     const int* nptr = g.nptr;
     int n = *nptr;
+    float v3 = var[2];
+    solve_pending<NT>(in, q);
     float T[16];
 #pragma unroll
-    for (int k = 0; k < 16; k++) T[k] = trel[k];
+    for (int k = 0; k < 16; k++) T[k] = q.T[k];
     double acc[27];
 #pragma unroll
     for (int k = 0; k < 27; k++) acc[k] = 0.0;
-    float v3 = var[2];
     float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
     for (int i = grp * NT + threadIdx.x; i < n; i += ngrp * NT) {
         float res, J[6];
@@ -700,8 +816,8 @@ __device__ __forceinline__ void icp_sys_body(const IcpSysArgs& g, int grp, int n
     }
     reduce27<NT>(acc, g.part, grp, g.stride);
 }
-__global__ __launch_bounds__(SYS_THREADS) void k_icp_sys(IcpSysArgs g) {
-    icp_sys_body<SYS_THREADS>(g, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(SYS_THREADS) void k_icp_sys(IcpSysArgs g, SolveIn in) {
+    icp_sys_body<SYS_THREADS>(g, in, blockIdx.x, gridDim.x);
 }
 // A bi-objective iteration's photometric residuals (first gp workgroups) and
 // its geometric system (the rest) in one launch: the geometric system does not
@@ -713,20 +829,20 @@ __global__ __launch_bounds__(SYS_THREADS) void k_bi_res(const float4* __restrict
                                                         const float* __restrict__ zcur, int W, int H,
                                                         const float* __restrict__ c, int bins,
                                                         float2* __restrict__ res, unsigned* __restrict__ madhist,
-                                                        int gp, IcpSysArgs g) {
+                                                        int gp, IcpSysArgs g, SolveIn in) {
     if ((int)blockIdx.x < gp)
-        photo_res_body<SYS_THREADS>(pts, jac, N, layer, img, wl, hl, zcur, W, H, c, g.trel, bins, res, madhist,
-                                    blockIdx.x, gp);
+        photo_res_body<SYS_THREADS>(pts, jac, N, layer, img, wl, hl, zcur, W, H, c, in, bins, res, madhist, blockIdx.x,
+                                    gp);
     else
-        icp_sys_body<SYS_THREADS>(g, blockIdx.x - gp, gridDim.x - gp);
+        icp_sys_body<SYS_THREADS>(g, in, blockIdx.x - gp, gridDim.x - gp);
 }
 
-void launch_icp_select(const Dev& d, int layer, hipStream_t s) {
+void launch_icp_select(const Dev& d, int layer, const SolveCfg& c, EstState& e, hipStream_t s) {
     int w = d.W >> layer, h = d.H >> layer, npix = w * h;
     int G = (npix + 1023) / 1024;
     uint64_t* words = d.icp_bits;
-    k_icp_mask<<<G, 1024, 0, s>>>(d.rpos[layer], d.rnrm[layer], w, h, layer, d.trel, d.calib, d.cpos[layer], d.rfull,
-                                  words, d.icp_cnt);
+    k_icp_mask<<<G, 1024, 0, s>>>(d.rpos[layer], d.rnrm[layer], w, h, layer, take_pending(d, c, e), d.calib,
+                                  d.cpos[layer], d.rfull, words, d.icp_cnt);
     k_icp_compact<<<G, 1024, 0, s>>>(d.rfull, words, d.icp_cnt, G, d.icp_sel[layer], d.icp_r2[layer],
                                      d.icp_n + layer);
     const int stride = (d.W * d.H + 1023) / 1024;
@@ -737,32 +853,34 @@ void launch_icp_select(const Dev& d, int layer, hipStream_t s) {
 
 static IcpSysArgs icp_sys_args(const Dev& d, int layer, const SolveCfg& c, double* part, int stride) {
     return IcpSysArgs{d.rpos[layer], d.rnrm[layer], d.icp_sel[layer], d.icp_r2[layer], d.icp_n + layer,
-                      d.icp_var + layer * 4, d.W >> layer, d.H >> layer, layer, d.calib, d.cpos[layer], d.trel,
-                      part, stride, c.scale_in};
+                      d.icp_var + layer * 4, d.W >> layer, d.H >> layer, layer, d.calib, d.cpos[layer], part, stride,
+                      c.scale_in};
 }
 
-void launch_icp_system(const Dev& d, int layer, const SolveCfg& c, int finish, hipStream_t s) {
+void launch_icp_system(const Dev& d, int layer, const SolveCfg& c, EstState& e, hipStream_t s) {
+    // Two partial buffers in turn: a workgroup that has finished writes this
+    // iteration's sums while another still combines the last one's.
     const int Gi = sys_groups((d.W >> layer) * (d.H >> layer));
-    k_icp_sys<<<Gi, SYS_THREADS, 0, s>>>(icp_sys_args(d, layer, c, d.part2, PART_STRIDE));
-    k_solve<<<1, SOLVE_THREADS, 0, s>>>(nullptr, 0, d.part2, Gi, nullptr, d.icp_n + layer, d.sys, d.trel, c,
-                                        finish == FINISH_SOLVE ? 1 : 0, d.N);
+    double* part = e.it & 1 ? d.part : d.part2;
+    const SolveIn in = take_pending(d, c, e);
+    k_icp_sys<<<Gi, SYS_THREADS, 0, s>>>(icp_sys_args(d, layer, c, part, PART_STRIDE), in);
+    set_pending(e, 0, Gi, part, d.icp_n + layer);
 }
 
 // The geometric system runs beside the photometric residuals on up to
 // RAW_STRIDE workgroups (every CU busy); the photometric system pass folds its
 // partials to at most SYS_GROUPS for the combine.
-void launch_biobjective_iteration(const Dev& d, int layer, const SolveCfg& c, int finish, bool select, hipStream_t s) {
+void launch_biobjective_iteration(const Dev& d, int layer, const SolveCfg& c, EstState& e, hipStream_t s) {
     const int Gr = d.N > 0 ? (d.N + SYS_THREADS - 1) / SYS_THREADS : 1;  // residuals, one point per thread
     int Gi = ((d.W >> layer) * (d.H >> layer) + SYS_THREADS - 1) / SYS_THREADS;
     Gi = Gi < 1 ? 1 : (Gi > RAW_STRIDE ? RAW_STRIDE : Gi);
     const int nf = Gi < SYS_GROUPS ? Gi : SYS_GROUPS;
-    if (select) launch_icp_select(d, layer, s);
     k_bi_res<<<Gr + Gi, SYS_THREADS, 0, s>>>(d.pts, d.jac[layer], d.N, layer, d.cur.gray[layer], d.W >> layer,
-                                             d.H >> layer, d.cur.z, d.W, d.H, d.calib, c.mad_bins, d.res, d.madhist,
-                                             Gr, icp_sys_args(d, layer, c, d.part3, RAW_STRIDE));
-    const int Gs = launch_photo_sys(d, layer, c, d.part3, Gi, d.part2, nf, s);
-    k_solve<<<1, SOLVE_THREADS, 0, s>>>(d.part, Gs, d.part2, nf, d.madhist, d.icp_n + layer, d.sys, d.trel, c,
-                                        finish == FINISH_SOLVE ? 1 : 0, d.N);
+                                             d.H >> layer, d.cur.z, d.W, d.H, d.calib, c.mad_bins, d.res,
+                                             d.madhist + (e.it & 1 ? 512 : 0), Gr,
+                                             icp_sys_args(d, layer, c, d.part3, RAW_STRIDE), take_pending(d, c, e));
+    const int Gs = launch_photo_sys(d, layer, c, e.it, d.part3, Gi, d.part2, nf, s);
+    set_pending(e, Gs, nf, d.part2, d.icp_n + layer);
 }
 
 // ------------------------------------------------------------------ A25

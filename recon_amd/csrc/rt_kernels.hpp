@@ -44,10 +44,12 @@ struct Dev {
     // photometric iteration
     float2* res;                // N: r, zWeight
     float* wts;                 // N: robust weight of the last iteration
-    unsigned* madhist;          // 512: accumulating histogram | copy of the last one
+    unsigned* madhist;          // 768: histogram of even iterations | copy of the last one | of odd iterations
     double* part;               // photometric system partials (27 x PART_STRIDE)
+    double* rms;                // 2 x RMS_GROUPS: partial sums of the residual RMS
     double* sys;                // 54: photometric 27 | geometric 27
     float* trel;                // 16
+    float* tbuf[2];             // 16 each: the pose of the iterations inside a frame, in turn
     // geometric
     float4* rpos[4];            // ref cloud (x,y,z,mask)
     float4* rnrm[4];            // ref normals
@@ -100,13 +102,33 @@ constexpr int PART_STRIDE = SYS_GROUPS;
 // Geometric system beside the photometric residuals: up to RAW_STRIDE
 // workgroups, partials at part3[k * RAW_STRIDE + group].
 constexpr int RAW_STRIDE = 256;
-void launch_photo_iteration(const Dev& d, int layer, const SolveCfg& c, int finish, hipStream_t s);
-void launch_icp_select(const Dev& d, int layer, hipStream_t s);
-// finish is FINISH_COMBINE or FINISH_SOLVE.
-void launch_icp_system(const Dev& d, int layer, const SolveCfg& c, int finish, hipStream_t s);
-// One bi-objective iteration: photometric residuals, the ICP selection of the
-// level (select), both systems in one launch, the combine (and solve).
-void launch_biobjective_iteration(const Dev& d, int layer, const SolveCfg& c, int finish, bool select, hipStream_t s);
+
+// The Gauss-Newton loop of a frame as it is launched. An iteration ends with
+// its system's partial sums in memory; the combine, the solve and the pose
+// update (gp photometric and gi geometric groups, pending) run at the start of
+// the kernel that needs the pose next, in every workgroup alike, and only the
+// frame's last ones are a launch of their own (launch_finish). The pose goes
+// from trel through the two buffers tbuf in turn, so that no workgroup writes
+// what another may still read.
+struct EstState {
+    float* T;         // the pose the pending solve starts from (or the current one)
+    int it = 0;       // iterations launched
+    bool pending = false;
+    int gp = 0, gi = 0;
+    const double* part2 = nullptr;  // the geometric sums
+    const int* nptr = nullptr;
+};
+void launch_photo_iteration(const Dev& d, int layer, const SolveCfg& c, EstState& e, hipStream_t s);
+void launch_icp_select(const Dev& d, int layer, const SolveCfg& c, EstState& e, hipStream_t s);
+void launch_icp_system(const Dev& d, int layer, const SolveCfg& c, EstState& e, hipStream_t s);
+// One bi-objective iteration: photometric residuals beside the geometric
+// system, then the photometric system.
+void launch_biobjective_iteration(const Dev& d, int layer, const SolveCfg& c, EstState& e, hipStream_t s);
+// The pending sums combined into sys (FINISH_COMBINE: inspection), or combined,
+// solved and the pose stored in trel (FINISH_SOLVE).
+void launch_finish(const Dev& d, const SolveCfg& c, EstState& e, int finish, hipStream_t s);
+constexpr int RMS_GROUPS = 64;
+void launch_residual_rms(const Dev& d, hipStream_t s);
 void launch_fuse(const Dev& d, hipStream_t s);
 void launch_error_image_photo(const Dev& d, hipStream_t s);
 void launch_error_image_icp(const Dev& d, hipStream_t s);

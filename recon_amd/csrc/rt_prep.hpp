@@ -500,21 +500,40 @@ __device__ bool solve_update(const double* sys, float* trel, const SolveCfg& cfg
     return ok;
 }
 
+// a / b rounded to nearest, given y = RN(1/b): div_rn in FP64. Equal to the
+// IEEE quotient while nothing over- or underflows (|a| >= 2^-969 or a = 0, b
+// and the quotient far inside the exponent range): the values here come from
+// sums of FP32 products. Three instructions instead of eleven, and y leaves
+// the dependent chain or serves several quotients.
+__device__ __forceinline__ double div_rn64(double a, double b, double y) {
+    const double q = a * y;
+    const double r = __builtin_fma(-b, q, a);
+    return __builtin_fma(r, y, q);
+}
 // expm_update with every matrix in registers instead of a workspace: the same
 // operations in the same order (se3_exp, normalize_mat4_safe, the product
-// T * Ti, normalize_mat4_safe). Run by every lane of a wave on the same x,
+// T * Ti, normalize_mat4_safe) without the ones whose result is exact by the
+// matrices' structure: products with the zero diagonal of W, sums with a zero
+// or a one of I or of Ti's last row, and squares and products that occur
+// twice. The quotients by one length share its reciprocal (div_rn64). 470
+// FP64 instructions instead of 790. Run by every lane of a wave on the same x,
 // so that no lane waits on the others; lane `writer` stores the pose.
 __device__ __forceinline__ void normalize_mat4_safe_regs(double* T) {
     double u[3] = {T[0], T[4], T[8]}, v[3] = {T[1], T[5], T[9]}, w[3] = {T[2], T[6], T[10]};
     double lenU = (double)sqrtf((float)(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]));
     double lenW = (double)sqrtf((float)(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]));
-    if (lenW > 1e-8f) { w[0] /= lenW; w[1] /= lenW; w[2] /= lenW; }
-    else { w[0] = 0; w[1] = 0; w[2] = 1; }
+    const double iU = 1.0 / lenU, iW = 1.0 / lenW;
+    if (lenW > 1e-8f) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) w[k] = div_rn64(w[k], lenW, iW);
+    } else { w[0] = 0; w[1] = 0; w[2] = 1; }
     u[0] = v[1] * w[2] - v[2] * w[1];
     u[1] = -(v[0] * w[2] - v[2] * w[0]);
     u[2] = v[0] * w[1] - v[1] * w[0];
-    if (lenU > 1e-8f) { u[0] /= lenU; u[1] /= lenU; u[2] /= lenU; }
-    else { u[0] = 1; u[1] = 0; u[2] = 0; }
+    if (lenU > 1e-8f) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) u[k] = div_rn64(u[k], lenU, iU);
+    } else { u[0] = 1; u[1] = 0; u[2] = 0; }
     v[0] = w[1] * u[2] - w[2] * u[1];
     v[1] = -(w[0] * u[2] - w[2] * u[0]);
     v[2] = w[0] * u[1] - w[1] * u[0];
@@ -522,62 +541,69 @@ __device__ __forceinline__ void normalize_mat4_safe_regs(double* T) {
     T[1] = v[0]; T[5] = v[1]; T[9] = v[2];
     T[2] = w[0]; T[6] = w[1]; T[10] = w[2];
 }
-__device__ __forceinline__ void expm_update_regs(const double* x, float* TF, double scale, bool writer) {
-    double Ti[16];
+// TI: the pose before the update, TO: where it is stored (may be the same)
+__device__ __forceinline__ void expm_update_regs(const double* x, const float* TI, float* TO, double scale, bool writer) {
+    double Ti[12];  // rows 0-2 of the increment; row 3 is 0 0 0 1
     double mx = 0;
 #pragma unroll
     for (int i = 0; i < 6; i++) mx = fmax(mx, fabs(x[i]));
     if (mx != 0) {
         // se3_exp
         const double wx = x[0], wy = x[1], wz = x[2];
-        const double th2 = wx * wx + wy * wy + wz * wz, th = sqrt(th2);
+        const double xx = wx * wx, yy = wy * wy, zz = wz * wz, xy = wx * wy, xz = wx * wz, yz = wy * wz;
+        const double th2 = xx + yy + zz, th = sqrt(th2);
         double a, b, cc;
         if (th < 1e-4) {
-            a = 1.0 - th2 / 6.0 + th2 * th2 / 120.0;
-            b = 0.5 - th2 / 24.0 + th2 * th2 / 720.0;
-            cc = 1.0 / 6.0 - th2 / 120.0 + th2 * th2 / 5040.0;
+            const double th4 = th2 * th2;
+            a = 1.0 - div_rn64(th2, 6.0, 1.0 / 6.0) + div_rn64(th4, 120.0, 1.0 / 120.0);
+            b = 0.5 - div_rn64(th2, 24.0, 1.0 / 24.0) + div_rn64(th4, 720.0, 1.0 / 720.0);
+            cc = 1.0 / 6.0 - div_rn64(th2, 120.0, 1.0 / 120.0) + div_rn64(th4, 5040.0, 1.0 / 5040.0);
         } else {
             const double sn = sin(th), co = cos(th);
             a = sn / th; b = (1.0 - co) / th2; cc = (th - sn) / (th2 * th);
         }
-        const double Wm[9] = {0, -wz, wy, wz, 0, -wx, -wy, wx, 0};
-        double W2[9];
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int j = 0; j < 3; j++) {
-                double s2 = 0;
-#pragma unroll
-                for (int k = 0; k < 3; k++) s2 += Wm[i * 3 + k] * Wm[k * 3 + j];
-                W2[i * 3 + j] = s2;
-            }
-        double V[9];
-#pragma unroll
-        for (int i = 0; i < 9; i++) {
-            const double I = (i % 4 == 0) ? 1.0 : 0.0;
-            Ti[(i / 3) * 4 + (i % 3)] = I + a * Wm[i] + b * W2[i];
-            V[i] = I + b * Wm[i] + cc * W2[i];
-        }
-#pragma unroll
-        for (int i = 0; i < 3; i++) Ti[i * 4 + 3] = V[i * 3 + 0] * x[3] + V[i * 3 + 1] * x[4] + V[i * 3 + 2] * x[5];
-        Ti[12] = 0; Ti[13] = 0; Ti[14] = 0; Ti[15] = 1;
+        // W = [0 -wz wy; wz 0 -wx; -wy wx 0], W2 = W W
+        const double d0 = -(zz + yy), d1 = -(zz + xx), d2 = -(yy + xx);
+        const double ax = a * wx, ay = a * wy, az = a * wz;
+        const double bxy = b * xy, bxz = b * xz, byz = b * yz;
+        Ti[0] = 1.0 + b * d0; Ti[1] = bxy - az;     Ti[2] = ay + bxz;
+        Ti[4] = az + bxy;     Ti[5] = 1.0 + b * d1; Ti[6] = byz - ax;
+        Ti[8] = bxz - ay;     Ti[9] = ax + byz;     Ti[10] = 1.0 + b * d2;
+        const double bx = b * wx, by = b * wy, bz = b * wz;
+        const double cxy = cc * xy, cxz = cc * xz, cyz = cc * yz;
+        Ti[3] = (1.0 + cc * d0) * x[3] + (cxy - bz) * x[4] + (by + cxz) * x[5];
+        Ti[7] = (bz + cxy) * x[3] + (1.0 + cc * d1) * x[4] + (cyz - bx) * x[5];
+        Ti[11] = (cxz - by) * x[3] + (bx + cyz) * x[4] + (1.0 + cc * d2) * x[5];
         normalize_mat4_safe_regs(Ti);
         Ti[3] *= scale; Ti[7] *= scale; Ti[11] *= scale;
     } else {
 #pragma unroll
-        for (int i = 0; i < 16; i++) Ti[i] = (i % 5 == 0) ? 1.0 : 0.0;
+        for (int i = 0; i < 12; i++) Ti[i] = (i % 5 == 0) ? 1.0 : 0.0;
     }
-    double R[16];
+    double R[12];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const double t0 = TF[i * 4 + 0], t1 = TF[i * 4 + 1], t2 = TF[i * 4 + 2], t3 = TF[i * 4 + 3];
+    for (int i = 0; i < 3; i++) {
+        const double t0 = TI[i * 4 + 0], t1 = TI[i * 4 + 1], t2 = TI[i * 4 + 2], t3 = TI[i * 4 + 3];
 #pragma unroll
-        for (int j = 0; j < 4; j++) R[i * 4 + j] = t0 * Ti[0 * 4 + j] + t1 * Ti[1 * 4 + j] + t2 * Ti[2 * 4 + j] + t3 * Ti[3 * 4 + j];
+        for (int j = 0; j < 4; j++) {
+            R[i * 4 + j] = t0 * Ti[0 * 4 + j] + t1 * Ti[1 * 4 + j] + t2 * Ti[2 * 4 + j];
+            if (j == 3) R[i * 4 + j] += t3;
+        }
+    }
+    // the last row of a pose is 0 0 0 1 and stays so; another one is multiplied out
+    float b3[4] = {TI[12], TI[13], TI[14], TI[15]};
+    if (b3[0] != 0.0f || b3[1] != 0.0f || b3[2] != 0.0f || b3[3] != 1.0f) {
+        const double t0 = b3[0], t1 = b3[1], t2 = b3[2], t3 = b3[3];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            b3[j] = (float)(t0 * Ti[j] + t1 * Ti[4 + j] + t2 * Ti[8 + j] + t3 * (j == 3 ? 1.0 : 0.0));
     }
     normalize_mat4_safe_regs(R);
     if (writer) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) TF[i] = (float)R[i];
+        for (int i = 0; i < 12; i++) TO[i] = (float)R[i];
+#pragma unroll
+        for (int i = 0; i < 4; i++) TO[12 + i] = b3[i];
     }
 }
 
@@ -588,44 +614,55 @@ __device__ __forceinline__ double lane_bcast(double v, int src) {
     return __hiloint2double(hi, lo);
 }
 // solve_update with the Cholesky solver, run by the 64 lanes of one wave: lane
-// r < 6 holds row r of A and of L in registers, the factorisation computes a
-// column's entries of all rows at once, and the substitutions exchange values
-// by lane reads instead of a workspace. The system is assembled as in
+// r < 6 holds row r of A and of L in registers, lane 6 the right-hand side as
+// a seventh row, so that the factorisation's columns, formed for all rows at
+// once, leave the forward substitution's y in that row (the same operations:
+// y_j = (b_j - sum y_k L[j][k]) / L[j][j]). The back substitution exchanges
+// values by lane reads and divides by reciprocals that were formed for the
+// whole diagonal at once (div_rn64). The system is assembled as in
 // solve_update (photometric terms, geometric terms, or their linear fuse with
 // the same operations), and every entry is computed by the same operations in
 // the same order as in solve_cholesky, so the result is the same bit for bit;
 // the exponential update runs in every lane's registers and lane 0 stores the
-// pose. The CG solver runs solve_update on lane 0. The return value is
-// meaningful in lane 0.
-__device__ bool solve_update_wave(const double* sys, float* trel, const SolveCfg& cfg, int N1, int N2, double* w) {
+// pose from TI to TO (the same array unless TO is given). The CG solver runs
+// solve_update on lane 0. The return value is meaningful in lane 0. Bound by
+// its serial chain of FP64 operations: 1,158 of them with a separate forward
+// substitution and every structural zero multiplied out, 710 now.
+__device__ bool solve_update_wave(const double* sys, float* TI, const SolveCfg& cfg, int N1, int N2, double* w,
+                                  float* TO = nullptr) {
     const int lane = lane_id();
+    if (!TO) TO = TI;
     if (cfg.solver != 0) {
         bool ok = true;
-        if (lane == 0) ok = solve_update(sys, trel, cfg, N1, N2, w);
+        if (lane == 0) {
+            float T[16];
+            for (int i = 0; i < 16; i++) T[i] = TI[i];
+            ok = solve_update(sys, T, cfg, N1, N2, w);
+            for (int i = 0; i < 16; i++) TO[i] = T[i];
+        }
         return ok;
     }
-    const int r = lane < 6 ? lane : 5;
-    // row r of A and b_r from the 27 packed terms (unpack27's order)
+    const int r = lane < 6 ? lane : 6;
+    // row r of A, or b, from the 27 packed terms (unpack27's order)
     const double* s0 = cfg.mode == 0 ? sys + 27 : sys;
-    double Ar[6];
+    int at[6];
 #pragma unroll
     for (int c = 0; c < 6; c++) {
         const int lo = r < c ? r : c, hi = r < c ? c : r;
-        Ar[c] = s0[lo * 6 - lo * (lo - 1) / 2 + (hi - lo)];
+        at[c] = r == 6 ? 21 + c : lo * 6 - lo * (lo - 1) / 2 + (hi - lo);
     }
-    double br = s0[21 + r];
+    double Ar[6];
+#pragma unroll
+    for (int c = 0; c < 6; c++) Ar[c] = s0[at[c]];
     if (cfg.mode == 2) {
         // linearFuse (warp.cu:1498-1509) as in solve_update
         const double s1 = (1.0 - (double)cfg.lambda) / (double)N1, s2 = (double)cfg.lambda / (double)N2;
         const double* sg = sys + 27;
 #pragma unroll
-        for (int c = 0; c < 6; c++) {
-            const int lo = r < c ? r : c, hi = r < c ? c : r;
-            Ar[c] = s1 * Ar[c] + s2 * sg[lo * 6 - lo * (lo - 1) / 2 + (hi - lo)];
-        }
-        br = s1 * br + s2 * sg[21 + r];
+        for (int c = 0; c < 6; c++) Ar[c] = s1 * Ar[c] + s2 * sg[at[c]];
     }
     double Lr[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    double diag = 1.0;  // L[r][r]
     bool ok = true;
 #pragma unroll
     for (int j = 0; j < 6; j++) {
@@ -638,27 +675,20 @@ __device__ bool solve_update_wave(const double* sys, float* trel, const SolveCfg
         const double dg = sqrt(sj);
         const double q = u / dg;
         Lr[j] = r == j ? dg : (r > j ? q : Lr[j]);
+        diag = r == j ? dg : diag;
     }
     double x[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     if (ok) {
-        double yv = 0.0;
-#pragma unroll
-        for (int i = 0; i < 6; i++) {
-            double t = br;
-#pragma unroll
-            for (int k = 0; k < i; k++) t -= Lr[k] * lane_bcast(yv, k);
-            const double yi = t / Lr[i];
-            yv = r == i ? yi : yv;
-        }
+        const double inv = 1.0 / diag;
 #pragma unroll
         for (int i = 5; i >= 0; i--) {
-            double t = lane_bcast(yv, i);
+            double t = lane_bcast(Lr[i], 6);
 #pragma unroll
             for (int k = i + 1; k < 6; k++) t -= lane_bcast(Lr[i], k) * x[k];
-            x[i] = t / lane_bcast(Lr[i], i);
+            x[i] = div_rn64(t, lane_bcast(diag, i), lane_bcast(inv, i));
         }
     }
-    expm_update_regs(x, trel, (double)cfg.scale_out, lane == 0);
+    expm_update_regs(x, TI, TO, (double)cfg.scale_out, lane == 0);
     return ok;
 }
 

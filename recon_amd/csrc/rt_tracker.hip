@@ -47,7 +47,8 @@ struct rt_tracker {
     uint8_t* g8[2] = {nullptr, nullptr};
     uint16_t* d16[2] = {nullptr, nullptr};
     float* rgbd = nullptr;
-    float* trel_host = nullptr;   // pinned
+    float* trel_host = nullptr;   // pinned: the pose, then the partial sums of the residual RMS
+    double* rms_host = nullptr;   // in trel_host's allocation
     double* seq_poses = nullptr;  // device, grows on demand
     int seq_cap = 0;
     // PhotoTracker / ShapeTracker state
@@ -167,8 +168,9 @@ extern "C" int rt_create(int device, int W, int H, const float* calib, const rt_
     A(d.ref.z, npx); A(d.cur.z, npx); A(d.kf_w, npx);
     A(d.gmag, npx); A(d.ghist, 256); A(d.seg, 2600); A(d.sel, p.n_select); A(d.pts, p.n_select);
     for (int l = 0; l < L; l++) A(d.jac[l], (jac_bytes(p.n_select) + 15) / 16);
-    A(d.res, p.n_select); A(d.wts, p.n_select); A(d.madhist, 512);
-    A(d.part, 27 * PART_STRIDE); A(d.part2, 27 * PART_STRIDE); A(d.part3, 27 * RAW_STRIDE); A(d.sys, 64); A(d.trel, 16);
+    A(d.res, p.n_select); A(d.wts, p.n_select); A(d.madhist, 768);
+    A(d.part, 27 * PART_STRIDE); A(d.part2, 27 * PART_STRIDE); A(d.part3, 27 * RAW_STRIDE); A(d.sys, 64); A(d.rms, 2 * RMS_GROUPS); A(d.trel, 16);
+    A(d.tbuf[0], 16); A(d.tbuf[1], 16);
     for (int l = 0; l < L; l++) {
         size_t nl = (size_t)(W >> l) * (H >> l);
         A(d.rpos[l], nl); A(d.rnrm[l], nl); A(d.cpos[l], nl); A(d.icp_sel[l], nl); A(d.icp_r2[l], nl);
@@ -183,10 +185,11 @@ extern "C" int rt_create(int device, int W, int H, const float* calib, const rt_
     for (int k = 0; k < 2; k++) { A(t->g8[k], npx); A(t->d16[k], npx); }
     A(t->rgbd, 4 * npx);
 #undef A
-    if (!ok || hipHostMalloc((void**)&t->trel_host, 64 * sizeof(float), 0) != hipSuccess) {
+    if (!ok || hipHostMalloc((void**)&t->trel_host, 64 * sizeof(float) + 2 * RMS_GROUPS * sizeof(double), 0) != hipSuccess) {
         free_all(t); delete t;
         return set_error(RT_ERR_NOMEM, "rt_create: allocation failed");
     }
+    t->rms_host = (double*)(t->trel_host + 64);
     if (hipMemcpy(cal, calib, RT_CALIB_SIZE * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) {
         free_all(t); delete t;
         return set_error(RT_ERR_HIP, "rt_create: calibration upload failed");
@@ -470,19 +473,18 @@ static int preprocess(rt_tracker* t, bool seq) {
 // gpuEstimateIncrement (phototracker.cpp:666-689)
 static void estimate_launches(rt_tracker* t, const SolveCfg& c) {
     int m = t->mode;
+    EstState e;
+    e.T = t->d.trel;
     for (int layer = t->L - 1; layer >= 0; layer--) {
         int n = t->prm.iters[t->L - 1 - layer];
         for (int j = 0; j < n; j++) {
-            if (m == RT_PHOTOMETRIC) {
-                launch_photo_iteration(t->d, layer, c, FINISH_SOLVE, t->stream);
-            } else if (m == RT_GEOMETRIC) {
-                if (j == 0) launch_icp_select(t->d, layer, t->stream);
-                launch_icp_system(t->d, layer, c, FINISH_SOLVE, t->stream);
-            } else {
-                launch_biobjective_iteration(t->d, layer, c, FINISH_SOLVE, j == 0, t->stream);
-            }
+            if (m != RT_PHOTOMETRIC && j == 0) launch_icp_select(t->d, layer, c, e, t->stream);
+            if (m == RT_PHOTOMETRIC) launch_photo_iteration(t->d, layer, c, e, t->stream);
+            else if (m == RT_GEOMETRIC) launch_icp_system(t->d, layer, c, e, t->stream);
+            else launch_biobjective_iteration(t->d, layer, c, e, t->stream);
         }
     }
+    launch_finish(t->d, c, e, FINISH_SOLVE, t->stream);
 }
 
 // gpuEstimateIncrement (phototracker.cpp:666-689): every level's iterations.
@@ -557,15 +559,14 @@ extern "C" int rt_get_residual_rms(rt_tracker* t, float* rms) {
     if (!t || !rms) return set_error(RT_ERR_ARG, "null argument");
     if (t->mode == RT_GEOMETRIC) return set_error(RT_ERR_STATE, "no photometric residuals in geometric mode");
     HIP_TRY(hipSetDevice(t->device));
-    std::vector<float> rz(2 * (size_t)t->N), w(t->N);
-    HIP_TRY(hipMemcpyAsync(rz.data(), t->d.res, rz.size() * 4, hipMemcpyDeviceToHost, t->stream));
-    HIP_TRY(hipMemcpyAsync(w.data(), t->d.wts, w.size() * 4, hipMemcpyDeviceToHost, t->stream));
+    launch_residual_rms(t->d, t->stream);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(t->rms_host, t->d.rms, 2 * RMS_GROUPS * sizeof(double), hipMemcpyDeviceToHost, t->stream));
     HIP_TRY(hipStreamSynchronize(t->stream));
     double a = 0.0, b = 0.0;
-    for (int i = 0; i < t->N; i++) {
-        double wr = (double)w[i] * rz[2 * (size_t)i];
-        a += wr * wr;
-        b += (double)w[i] * w[i];
+    for (int g = 0; g < RMS_GROUPS; g++) {
+        a += t->rms_host[2 * g];
+        b += t->rms_host[2 * g + 1];
     }
     *rms = b > 0.0 ? (float)sqrt(a / b) : 0.0f;
     return RT_OK;
@@ -859,14 +860,13 @@ extern "C" int rt_debug_linearize(rt_tracker* t, int level, int it) {
     HIP_TRY(hipSetDevice(t->device));
     SolveCfg c = solve_cfg(t);
     int m = t->mode;
-    if (m == RT_PHOTOMETRIC) {
-        launch_photo_iteration(t->d, level, c, FINISH_COMBINE, t->stream);
-    } else if (m == RT_GEOMETRIC) {
-        if (it == 0) launch_icp_select(t->d, level, t->stream);
-        launch_icp_system(t->d, level, c, FINISH_COMBINE, t->stream);
-    } else {
-        launch_biobjective_iteration(t->d, level, c, FINISH_COMBINE, it == 0, t->stream);
-    }
+    EstState e;
+    e.T = t->d.trel;
+    if (m != RT_PHOTOMETRIC && it == 0) launch_icp_select(t->d, level, c, e, t->stream);
+    if (m == RT_PHOTOMETRIC) launch_photo_iteration(t->d, level, c, e, t->stream);
+    else if (m == RT_GEOMETRIC) launch_icp_system(t->d, level, c, e, t->stream);
+    else launch_biobjective_iteration(t->d, level, c, e, t->stream);
+    launch_finish(t->d, c, e, FINISH_COMBINE, t->stream);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(t->stream));
     return RT_OK;

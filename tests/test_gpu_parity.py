@@ -215,6 +215,37 @@ def test_track_matches_oracle(mode, solver):
     assert np.allclose(tr.get_global_pose(), np.linalg.inv(Tdev), atol=1e-3)
 
 
+# Schedules at their edges: a single iteration (no update inside the frame),
+# levels without iterations, a frame without any (the pose stays), and point
+# counts below, at and above the system pass's 64 workgroups of 256.
+@pytest.mark.parametrize("mode", [PHOTOMETRIC, GEOMETRIC, BIOBJECTIVE])
+@pytest.mark.parametrize("iters,N", [((1, 0, 0, 0), 256), ((0, 0, 3, 0), 16384), ((2, 0, 1, 0), 16640),
+                                     ((0, 0, 0, 0), 4096), ((0, 1, 0, 0), 4352)])
+def test_track_schedules_match_oracle(mode, iters, N):
+    import oracle
+    print(f"case track schedule mode {mode} iters {iters} N {N}", flush=True)
+    W, H, L = 320, 240, 3
+    g0, d0, g1, d1, Tgt = _pair(W, H, 17)
+    cal = synth.calib_block_np(W, H)
+    init = synth.sample_motion(5, 0.5, 8.0) @ Tgt
+    tr = PhotoTracker(W, H, cal, mode=mode, levels=L, n_select=N, iters=iters, lam=0.5)
+    for frame in range(2):  # the second frame starts from what the first left behind
+        tr.set_reference_points(g0, d0, mode=mode, lam=0.5, force=True)
+        tr.set_current_image(g1, d1)
+        tr.track_from(np.linalg.inv(init))
+        Tdev = tr.trel().astype(np.float64)
+        o = oracle.Tracker(W, H, cal, mode=mode, levels=L, iters=iters, nselect=N, lam=0.5, dtype=np.float32)
+        o.set_reference(g0, d0); o.set_current(g1, d1); o.prepare(); o.set_trel(init); o.track()
+        rot, tmm = synth.pose_error(Tdev, o.poses()[0])
+        print(f"  frame {frame}: {rot:.2e} deg {tmm:.2e} mm", flush=True)
+        assert np.radians(rot) < 1e-5 and tmm < 1e-2
+        if mode != GEOMETRIC and any(iters):
+            rz = tr.debug_read("RESIDUAL", 0, np.float32, 2 * N).reshape(N, 2)[:, 0].astype(np.float64)
+            w = tr.list_selected()[2].astype(np.float64)
+            want = np.sqrt(np.sum((w * rz) ** 2) / np.sum(w * w))
+            assert abs(tr.residual_rms() - want) <= 1e-6 * want
+
+
 @pytest.mark.parametrize("W,H,L,N,seed", CASES[:2])
 def test_inspection_images_bitexact(W, H, L, N, seed):
     """updateErrorImage / getDebugImage1C / getRefImage1C against
