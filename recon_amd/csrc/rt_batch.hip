@@ -596,166 +596,58 @@ __global__ __launch_bounds__(256) void kb_ref_points(const PairDesc* __restrict_
 // level 0 from the 16-bit depths (ShapeTracker::setReferencePoints /
 // generatePyramids, shapetracker.cpp:195-211,254-258), then the masked 2x2
 // pyramids level by level. The per-pixel bodies are the single-pair kernels'
-// (ref_cloud_pixel, cur_cloud_pixel, cloud_down_pixel), reading the depth
+// (ref_cloud_pixel, cur_cloud_pixel, cloud_tile_levels), reading the depth
 // through the same exact conversion, so the clouds are the same bit for bit.
 __global__ __launch_bounds__(256) void kb_clouds(const PairDesc* __restrict__ P) {
+    __shared__ float4 lp[CLOUD_TILE], ln[CLOUD_TILE], lc[CLOUD_TILE];
     const PairDesc& d = P[blockIdx.z];
-    const int x = blockIdx.x * 16 + (threadIdx.x & 15), y = blockIdx.y * 16 + (threadIdx.x >> 4);
-    if (x >= d.W || y >= d.H) return;
-    ref_cloud_pixel(U16DepthSrc{d.d16[0]}, d.W, d.H, x, y, d.calib, d.rpos[0], d.rnrm[0]);
-    cur_cloud_pixel(U16DepthSrc{d.d16[1]}, d.W, x + y * d.W, d.calib, d.cpos[0]);
-}
-__global__ __launch_bounds__(256) void kb_clouds_down(const PairDesc* __restrict__ P, int level) {
-    const PairDesc& d = P[blockIdx.y];
-    if (level >= d.L) return;
-    const int Wd = d.W >> level, Hd = d.H >> level;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= Wd * Hd) return;
-    cloud_down_pixel(d.rpos[level - 1], d.rnrm[level - 1], Wd, i, d.rpos[level], d.rnrm[level]);
-    cloud_down_pixel(d.cpos[level - 1], nullptr, Wd, i, d.cpos[level], nullptr);
+    const int t = threadIdx.x;
+    if ((int)blockIdx.x * 16 >= d.W || (int)blockIdx.y * 16 >= d.H) return;
+    const int x = blockIdx.x * 16 + (t & 15), y = blockIdx.y * 16 + (t >> 4);
+    lp[t] = lc[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (x < d.W && y < d.H) {
+        const size_t o = (size_t)x + (size_t)y * d.W;
+        float4 pos, nrm;
+        ref_cloud_pixel(U16DepthSrc{d.d16[0]}, d.W, d.H, x, y, d.calib, d.ifx, d.ify, pos, nrm);
+        const float4 cur = cur_cloud_pixel(U16DepthSrc{d.d16[1]}[o], x, y, d.calib, d.ifx, d.ify);
+        stg(d.rpos[0], o, pos);
+        stg(d.rnrm[0], o, nrm);
+        stg(d.cpos[0], o, cur);
+        lp[t] = pos; ln[t] = nrm; lc[t] = cur;
+    }
+    cloud_tile_levels<true>(lp, ln, blockIdx.x, blockIdx.y, d.W, d.H, d.L, d.rpos, d.rnrm);
+    cloud_tile_levels<false>(lc, nullptr, blockIdx.x, blockIdx.y, d.W, d.H, d.L, d.cpos, nullptr);
 }
 
 __global__ void kb_reset_queue(int* q) {
     if (threadIdx.x == 0) q[0] = 0;
 }
 
-// ------------------------------------------------------------------ geometric terms in one workgroup
-// ICP selection of one level (icpResidualKernel2 + selectValidIndex +
-// packIndex, rgb2gray.cu:223-260,827-850): ordered compaction of the valid
-// keyframe pixels into d.isel / d.ir2 (squared residual), BS pixels a step:
-// a ballot per wave, the waves' counts in LDS. Ascending pixel order, as the
-// single-pair compaction. Returns the count (the same in every thread).
-template <int BS>
-__device__ int icp_select_wg(const PairDesc& d, int layer, const float* T, const float* c) {
-    constexpr int NW = BS / 64;
-    __shared__ int wc[NW];
-    const int t = threadIdx.x, wave = t >> 6, lane = lane_id();
-    const int w = d.W >> layer, h = d.H >> layer, npix = w * h;
-    const float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
-    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    RT_GLOBAL int* isel = gmem(d.isel);
-    RT_GLOBAL float* ir2 = gmem(d.ir2);
-    int base = 0;
-    for (int o0 = 0; o0 < npix; o0 += BS) {
-        const int o = o0 + t;
-        float r = 0.0f;
-        const bool valid = o < npix && icp_mask_pixel(d.rpos[layer], d.rnrm[layer], d.cpos[layer], w, h, o, T, c, a, b, r);
-        const uint64_t bl = __ballot(valid);
-        if (lane == 0) wc[wave] = __popcll(bl);
-        __syncthreads();
-        int off = 0, tot = 0;
+// Median bin of a MAD histogram by one wave, lane l the bins 4l .. 4l + 3: the
+// first bin whose running count exceeds N / 2 (histogram64.cu:48-61).
+__device__ __forceinline__ void median_bin(const unsigned* hist, int N, int* med) {
+    const int lane = lane_id();
+    unsigned c4[4];
+    unsigned run = 0;
 #pragma unroll
-        for (int q = 0; q < NW; q++) {
-            const int cq = wc[q];
-            off += q < wave ? cq : 0;
-            tot += cq;
-        }
-        if (valid) {
-            const int k = base + off + __popcll(bl & lt);
-            isel[k] = o;
-            ir2[k] = r * r;
-        }
-        base += tot;
-        __syncthreads();
+    for (int q = 0; q < 4; q++) { c4[q] = hist[lane * 4 + q]; run += c4[q]; }
+    unsigned incl = run;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        unsigned v = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += v;
     }
-    return base;
-}
-// generateStudentTWeights (rgb2gray.cu:470-568, 854-877) in one workgroup: the
-// three variance rounds with the single-pair kernels' arithmetic and trees
-// (the product truncated to int per point, a 1024-wide FP32 tree per block of
-// 1024 points, the block sums truncated to int and reduced by the same tree,
-// clamped to at least n), so the sums are the same bit for bit. var: three
-// values in LDS, unchanged when n = 0 (no solve follows then).
-template <int BS>
-__device__ void student_t_wg(const float* __restrict__ r2, int n, float* var) {
-    __shared__ float p[1024];
-    __shared__ float bsum[512];  // n <= W*H <= 512 * 1024 (checked at preparation)
-    const int t = threadIdx.x;
-    if (n <= 0) return;
-    const int nb = (n + 1023) / 1024;
-    auto tree = [&]() {
-        for (int s2 = 512; s2 >= 1; s2 >>= 1) {
-            for (int e = t; e < s2; e += BS) p[e] += p[e + s2];
-            __syncthreads();
-        }
-    };
-    for (int round = 1; round <= 3; round++) {
-        const float prev = round > 1 ? var[round - 2] : 0.0f;
-        for (int bk = 0; bk < nb; bk++) {
-            for (int e = t; e < 1024; e += BS) {
-                const int i = bk * 1024 + e;
-                int sum = 0;
-                if (i < n) {
-                    const float x = r2[i];
-                    const float w = round == 1 ? 6 / (5 + x / 100.0f) : 6 / (5 + x / (prev / (float)n));
-                    sum += x * w;
-                }
-                p[e] = (float)sum;
-            }
-            __syncthreads();
-            tree();
-            if (t == 0) bsum[bk] = p[0];
-            __syncthreads();
-        }
-        if (nb == 1) {
-            if (t == 0) var[round - 1] = bsum[0];
-        } else {
-            for (int e = t; e < 1024; e += BS) {
-                int ss = 0;
-                for (int q = e; q < nb; q += 1024) ss += bsum[q];
-                p[e] = (float)ss;
-            }
-            __syncthreads();
-            tree();
-            if (t == 0) {
-                float v = p[0];
-                const float mn = (float)n;
-                if (v < mn) v = mn;
-                var[round - 1] = v;
-            }
-        }
-        __syncthreads();
+    unsigned acc = incl - run;
+    int found = 1 << 30;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        acc += c4[q];
+        if (found == (1 << 30) && (int)acc > N / 2) found = lane * 4 + q;
     }
-}
-// The geometric system of one iteration (icpResidualIndexKernel2,
-// rgb2gray.cu:323-390, and the 27 dot products): per thread in FP32 over its
-// points, per wave by halving exchanges, across waves in FP64 into sysg[27].
-template <int BS>
-__device__ void icp_system_wg(const PairDesc& d, int layer, int n, float v3, const float* T, const float* c,
-                              double (*wsum)[29], double* sysg) {
-    constexpr int NW = BS / 64;
-    const int t = threadIdx.x, wave = t >> 6, lane = lane_id();
-    const int w = d.W >> layer, h = d.H >> layer;
-    const float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
-    const RT_GLOBAL int* isel = gmem(d.isel);
-    const RT_GLOBAL float* ir2 = gmem(d.ir2);
-    float acc[27];
+    int m = found;
 #pragma unroll
-    for (int k = 0; k < 27; k++) acc[k] = 0.0f;
-    for (int i = t; i < n; i += BS) {
-        float res, J[6];
-        icp_point_terms(d.rpos[layer], d.rnrm[layer], d.cpos[layer], w, h, isel[i], ir2[i], v3, n, T, c, a, b, 1e-3f,
-                        res, J);
-        int q = 0;
-#pragma unroll
-        for (int r0 = 0; r0 < 6; r0++)
-#pragma unroll
-            for (int c0 = r0; c0 < 6; c0++) acc[q++] += J[r0] * J[c0];
-#pragma unroll
-        for (int r0 = 0; r0 < 6; r0++) acc[21 + r0] += J[r0] * res;
-    }
-    float v32[32];
-#pragma unroll
-    for (int k = 0; k < 32; k++) v32[k] = k < 27 ? acc[k] : 0.0f;
-    const float tot = wave_sum32(v32);
-    if ((lane & 1) == 0 && (lane >> 1) < 27) wsum[wave][lane >> 1] = (double)tot;
-    __syncthreads();
-    if (t < 27) {
-        double v = 0.0;
-        for (int w2 = 0; w2 < NW; w2++) v += wsum[w2][t];
-        sysg[t] = v;
-    }
-    __syncthreads();
+    for (int o = 32; o >= 1; o >>= 1) m = min(m, __shfl_xor(m, o, 64));
+    if (lane == 0) *med = m == (1 << 30) ? 0 : m;
 }
 
 // ------------------------------------------------------------------ persistent tracking
@@ -764,7 +656,6 @@ struct TrackCfg {
     int robust;
     int mad_bins;
     float scale_out;
-    float lambda;  // bi-objective weight of the geometric system (linearFuse)
     int pc_cap;  // point-cache capacity (points; PC variants)
     int rz_len;  // length of the RZ residual array (the batch's largest point count)
 };
@@ -786,24 +677,16 @@ constexpr int PC_MAX = 8192;
 // would overlap one pair's serial phases with the other's point passes, were
 // measured slower than one 1024-thread workgroup at 640x480: the kernel is
 // bound by memory traffic, not by those phases.
-// MODE: the tracking mode (RT_GEOMETRIC 0, RT_PHOTOMETRIC 1, RT_BIOBJECTIVE 2).
-// The geometric modes add, per level, the ICP selection and Student-t weights
-// at the level's first iteration and the geometric system every iteration
-// (ShapeTracker::updateLinearSystem, shapetracker.cpp:357-382), fused with the
-// photometric one by linearFuse in the bi-objective mode (:392-394).
-template <int BS, int PPT, int RZ, int WPE = 1, int PC = 0, int MODE = 1>
+template <int BS, int PPT, int RZ, int WPE = 1, int PC = 0>
 __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__ P, const int* __restrict__ order,
                                                     int npairs, int* queue, TrackCfg cfg) {
     constexpr int NW = BS / 64;
-    // system terms: photometric 27 | geometric 27 (geometric modes) | the two
-    // sums of the photometric residual RMS
-    constexpr int NSYS = MODE == 1 ? 29 : 56, RMS0 = MODE == 1 ? 27 : 54;
+    constexpr int NSYS = 29;  // 27 system terms | the two sums of the residual RMS
     __shared__ float cal[96];
     __shared__ float T[16];
     __shared__ unsigned hist[256];
     __shared__ double wsum[NW][29];
     __shared__ double sys[NSYS];
-    __shared__ float s_var[3];
     __shared__ double ws[SOLVE_WS];
     __shared__ int s_pair, s_med;
     __shared__ int s_ok;
@@ -844,14 +727,12 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
             const JacView jv = jac_view(d.jac[layer], N);
             const int wl = W >> layer, hl = H >> layer;
             const float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
-            int nicp = 0;  // ICP points of the level (geometric modes)
             for (int it = 0; it < nit; it++) {
                 for (int k = t; k < 256; k += BS) hist[k] = 0u;
                 float Tl[16];
 #pragma unroll
                 for (int k = 0; k < 16; k++) Tl[k] = uni(T[k]);
                 __syncthreads();
-              if constexpr (MODE != 0) {
                 // residual pass: r and zWeight stay in registers (RZ 0) or go to LDS (RZ 1)
                 float r[RZ ? 1 : PPT], zw[RZ ? 1 : PPT];
                 auto residual = [&](int i, float& rr, float& zz) {
@@ -902,30 +783,7 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
                 }
                 xyz_cached = true;
                 __syncthreads();
-                // median bin: first bin whose running count exceeds N/2 (histogram64.cu:48-61)
-                if (wave == 0) {
-                    unsigned c4[4];
-                    unsigned run = 0;
-#pragma unroll
-                    for (int q = 0; q < 4; q++) { c4[q] = hist[lane * 4 + q]; run += c4[q]; }
-                    unsigned incl = run;
-#pragma unroll
-                    for (int o = 1; o < 64; o <<= 1) {
-                        unsigned v = __shfl_up(incl, o, 64);
-                        if (lane >= o) incl += v;
-                    }
-                    unsigned acc = incl - run;
-                    int found = 1 << 30;
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        acc += c4[q];
-                        if (found == (1 << 30) && (int)acc > N / 2) found = lane * 4 + q;
-                    }
-                    int m = found;
-#pragma unroll
-                    for (int o = 32; o >= 1; o >>= 1) m = min(m, __shfl_xor(m, o, 64));
-                    if (lane == 0) s_med = m == (1 << 30) ? 0 : m;
-                }
+                if (wave == 0) median_bin(hist, N, &s_med);
                 __syncthreads();
                 const float s = mad_scale(s_med, cfg.mad_bins);
                 float acc[29];
@@ -975,34 +833,18 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
                 if (t < 29) {
                     double v = 0.0;
                     for (int w2 = 0; w2 < NW; w2++) v += wsum[w2][t];
-                    sys[t < 27 ? t : RMS0 + t - 27] = v;
+                    sys[t] = v;
                 }
                 __syncthreads();
-              }
-                if constexpr (MODE != 1) {
-                    // the level's ICP points and Student-t weights at its first
-                    // iteration (under the pose the iteration starts from)
-                    if (it == 0) {
-                        nicp = icp_select_wg<BS>(d, layer, Tl, cl);
-                        student_t_wg<BS>(d.ir2, nicp, s_var);
-                        if (t == 0) {
-                            d.icnt[layer] = nicp;
-                            for (int k = 0; k < 3; k++) d.ivar[layer * 3 + k] = nicp > 0 ? s_var[k] : 0.0f;
-                        }
-                    }
-                    icp_system_wg<BS>(d, layer, nicp, s_var[2], Tl, cl, wsum, sys + 27);
-                }
                 if (wave == 0) {
                     SolveCfg sc;
-                    sc.solver = cfg.solver; sc.mode = MODE; sc.lambda = cfg.lambda; sc.scale_out = cfg.scale_out;
+                    sc.solver = cfg.solver; sc.mode = RT_PHOTOMETRIC; sc.lambda = 0.0f; sc.scale_out = cfg.scale_out;
                     sc.robust = cfg.robust; sc.mad_bins = cfg.mad_bins; sc.scale_in = 1e-3f;
-                    // no update from an empty geometric selection (as the single-pair path)
-                    if (MODE == 1 || nicp > 0) {
-                        const bool ok = solve_update_wave(sys, T, sc, N, nicp, ws);
-                        if (t == 0 && !ok) s_ok = 0;
+                    const bool ok = solve_update_wave(sys, T, sc, N, 0, ws);
+                    if (t == 0) {
+                        if (!ok) s_ok = 0;
+                        rms_last = sys[28] > 0.0 ? (float)sqrt(sys[27] / sys[28]) : 0.0f;
                     }
-                    if (t == 0 && MODE != 0)
-                        rms_last = sys[RMS0 + 1] > 0.0 ? (float)sqrt(sys[RMS0] / sys[RMS0 + 1]) : 0.0f;
                 }
                 __syncthreads();
             }
@@ -1012,8 +854,390 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
     }
 }
 
+// ------------------------------------------------------------------ lockstep tracking
+// The Gauss-Newton loop of every pair at once, one launch per pass instead of
+// one workgroup per pair: all pairs advance one iteration per step, and a
+// pair's points are spread over many workgroups. It tracks the geometric and
+// bi-objective batches (a level has up to W x H points, 75 to 300 per lane of
+// one workgroup: 64 pairs of 320x240 took 4.05 ms on 64 of the 256 CUs) and the
+// small photometric batches, which would leave most CUs idle.
+//
+// The sums are those of a 1024-thread workgroup of kb_track, bit for bit:
+// virtual lane (wave v of 16, lane l) adds its points 64 v + l + 1024 j in
+// order of j in FP32, the 64 lanes of a wave meet in the exchange order
+// 32, 16, ..., 1, and the 16 waves add in order in FP64. A workgroup of 8
+// waves is one virtual wave: in each round wave w forms the terms' factors of
+// the points j = 8 round + w (one per lane) and leaves them in LDS, and after
+// a barrier four of the waves add eight terms each over the round's eight j, so
+// that the points are formed by eight waves while each sum stays one chain.
+constexpr int LK_BLOCKS = 512;  // blocks of 1024 pixels: W x H <= 512 x 1024, checked at preparation
+struct LockBufs {
+    char* base;        // per pair: the arrays below
+    size_t stride, o_rz, o_bits, o_rfull;
+    __host__ __device__ float* wsum(int p, int geo) const { return (float*)(base + stride * p) + geo * 512; }  // [16][32]
+    __host__ __device__ unsigned* hist(int p, int par) const { return (unsigned*)(base + stride * p + 4096) + 256 * par; }
+    __host__ __device__ int* cnt(int p) const { return (int*)(base + stride * p + 6144); }
+    __host__ __device__ float* bsum(int p, int round) const {
+        return (float*)(base + stride * p + 6144 + 4 * LK_BLOCKS) + LK_BLOCKS * round;
+    }
+    __host__ __device__ float2* rz(int p) const { return (float2*)(base + stride * p + o_rz); }
+    __host__ __device__ uint64_t* bits(int p) const { return (uint64_t*)(base + stride * p + o_bits); }
+    __host__ __device__ float* rfull(int p) const { return (float*)(base + stride * p + o_rfull); }
+};
+constexpr size_t LK_FIXED = 6144 + 4 * LK_BLOCKS * 4;  // wsum, two histograms, counts, three rounds of block sums
+
+// The level and its iteration at a step of the pair's schedule; false past its end.
+__host__ __device__ __forceinline__ bool lock_level(int L, const int* iters, int step, int& layer, int& it) {
+    for (layer = L - 1; layer >= 0; layer--) {
+        const int n = iters[L - 1 - layer];
+        if (step < n) { it = step; return true; }
+        step -= n;
+    }
+    return false;
+}
+// The pose of the pair (trel_out holds it while it is tracked) and the depth
+// intrinsics as wave-uniform values.
+__device__ __forceinline__ void lock_pose(const PairDesc& d, float* T) {
+#pragma unroll
+    for (int k = 0; k < 16; k++) T[k] = uni(d.trel_out[k]);
+}
+
+__global__ __launch_bounds__(256) void kl_init(const PairDesc* __restrict__ P, LockBufs B) {
+    const int p = blockIdx.x, t = threadIdx.x;
+    const PairDesc& d = P[p];
+    B.hist(p, 0)[t] = 0u;
+    B.hist(p, 1)[t] = 0u;
+    if (t < 16) d.trel_out[t] = d.trel_in[t];
+    if (t == 0) { *d.rms = 0.0f; *d.status = 0; }
+}
+
+// ICP selection of the levels that begin at this step (icpResidualKernel2 +
+// selectValidIndex + packIndex, rgb2gray.cu:223-260,827-850): the mask and
+// residual of 1024 pixels a workgroup, then the ordered compaction.
+__global__ __launch_bounds__(1024) void kl_icp_mask(const PairDesc* __restrict__ P, LockBufs B, int step) {
+    __shared__ int wc[16];
+    const int p = blockIdx.y, g = blockIdx.x;
+    const PairDesc& d = P[p];
+    int layer, it;
+    if (!lock_level(d.L, d.iters, step, layer, it) || it != 0) return;
+    const int w = d.W >> layer, h = d.H >> layer, npix = w * h;
+    if (g * 1024 >= npix) return;
+    float T[16], cl[96];
+    lock_pose(d, T);
+#pragma unroll
+    for (int k = 0; k < 9; k++) cl[KL + k] = uni(d.calib[KL + k]);
+    const int o = g * 1024 + threadIdx.x, wave = threadIdx.x >> 6;
+    const float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
+    float r = 0.0f;
+    const bool valid = o < npix && icp_mask_pixel(d.rpos[layer], d.rnrm[layer], d.cpos[layer], w, h, o, T, cl, a, b, r);
+    if (valid) B.rfull(p)[o] = r;
+    const uint64_t bl = __ballot(valid);
+    if (lane_id() == 0) {
+        B.bits(p)[g * 16 + wave] = bl;
+        wc[wave] = __popcll(bl);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int s = 0;
+        for (int q = 0; q < 16; q++) s += wc[q];
+        B.cnt(p)[g] = s;
+    }
+}
+__global__ __launch_bounds__(1024) void kl_icp_compact(const PairDesc* __restrict__ P, LockBufs B, int step) {
+    __shared__ int red[16], wpre[16];
+    const int p = blockIdx.y, g = blockIdx.x, t = threadIdx.x, wave = t >> 6, lane = lane_id();
+    const PairDesc& d = P[p];
+    int layer, it;
+    if (!lock_level(d.L, d.iters, step, layer, it) || it != 0) return;
+    const int npix = (d.W >> layer) * (d.H >> layer);
+    if (g * 1024 >= npix) return;
+    int v = t < g ? B.cnt(p)[t] : 0;  // g < LK_BLOCKS
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (lane == 0) red[wave] = v;
+    const uint64_t word = B.bits(p)[g * 16 + wave];
+    if (lane == 0) wpre[wave] = __popcll(word);
+    __syncthreads();
+    int k0 = 0, tot = 0;
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        k0 += red[q] + (q < wave ? wpre[q] : 0);
+        tot += red[q] + wpre[q];
+    }
+    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    if ((word >> lane) & 1ull) {
+        const int k = k0 + __popcll(word & lt), o = g * 1024 + t;
+        const float r = B.rfull(p)[o];
+        gmem(d.isel)[k] = o;
+        gmem(d.ir2)[k] = r * r;
+    }
+    if ((g + 1) * 1024 >= npix && t == 0) {  // the last block holds the total
+        d.icnt[layer] = tot;
+        if (tot == 0)
+            for (int q = 0; q < 3; q++) d.ivar[layer * 3 + q] = 0.0f;
+    }
+}
+// Student-t round 1, 2 or 3 (generateStudentTWeights, rgb2gray.cu:470-568,
+// 854-877): one wave per block of 1024 points.
+__global__ __launch_bounds__(256) void kl_student(const PairDesc* __restrict__ P, LockBufs B, int step, int round) {
+    const int p = blockIdx.y, bk = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const PairDesc& d = P[p];
+    int layer, it;
+    if (!lock_level(d.L, d.iters, step, layer, it) || it != 0) return;
+    const int n = d.icnt[layer], nb = (n + 1023) / 1024;
+    if (bk >= nb) return;
+    float prev = 0.0f;
+    if (round > 1) {
+        prev = wave_student_total(B.bsum(p, round - 2), nb, n);
+        if (bk == 0 && lane_id() == 0) d.ivar[layer * 3 + round - 2] = prev;
+    }
+    const float s = wave_student_block(d.ir2, bk, n, round, prev);
+    if (lane_id() == 0) B.bsum(p, round - 1)[bk] = s;
+}
+
+// Term k of the system as the product of two of a point's factors: the 21
+// products J[r] J[c] (r <= c) of factors 0-5, the 6 J[r] times factor 6, then
+// 6 x 6 and 7 x 7 (the residual RMS).
+struct LockTerms { int a[32], b[32]; };
+constexpr LockTerms make_lock_terms() {
+    LockTerms t{};
+    int k = 0;
+    for (int r = 0; r < 6; r++)
+        for (int c = r; c < 6; c++) { t.a[k] = r; t.b[k++] = c; }
+    for (int r = 0; r < 6; r++) { t.a[k] = r; t.b[k++] = 6; }
+    for (int q = 6; k < 32; k++) { t.a[k] = t.b[k] = q; q = 7; }
+    return t;
+}
+// The factors of the 8 points of a round per virtual lane, f[j][half][lane]
+// (factors 0-3, 4-7: two 16-byte reads a point), and the sums of terms 8 G ..
+// 8 G + 7 by wave G: four of the eight waves add while the others go on to the
+// next round. Reading the factors of four terms in each of eight waves took
+// twice the instructions and LDS traffic (64 bi-objective pairs of 320x240: 106
+// us a launch, 95 here).
+typedef float4 LockRound[8][2][64];
+template <int G, int NT, bool FMA>
+__device__ __forceinline__ void lock_add(const LockRound& f, float* acc) {
+    constexpr LockTerms tm = make_lock_terms();
+    const int lane = lane_id();
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const float4 u = f[j][0][lane], v = f[j][1][lane];
+        const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+            if (8 * G + q < NT) {
+                const float p = x[tm.a[8 * G + q]], r = x[tm.b[8 * G + q]];
+                acc[q] = FMA ? __builtin_fmaf(p, r, acc[q]) : acc[q] + p * r;
+            }
+    }
+}
+template <int NT, bool FMA>
+__device__ __forceinline__ void lock_add(int wave, const LockRound& f, float* acc) {
+    switch (wave) {
+        case 0: lock_add<0, NT, FMA>(f, acc); break;
+        case 1: lock_add<1, NT, FMA>(f, acc); break;
+        case 2: lock_add<2, NT, FMA>(f, acc); break;
+        case 3: lock_add<3, NT, FMA>(f, acc); break;
+        default: break;
+    }
+}
+// The lanes' sums of the wave's terms into the pair's table.
+template <int NT>
+__device__ __forceinline__ void lock_store(int wave, float* acc, float* wsum) {
+    if (wave > 3) return;
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+        acc[q] = wave_sum(acc[q]);
+        if (lane_id() == 0 && 8 * wave + q < NT) wsum[8 * wave + q] = acc[q];
+    }
+}
+
+// One pass of an iteration. GEO workgroups (the first 16 of a pair): the
+// geometric system of virtual wave blockIdx.x (icpResidualIndexKernel2,
+// rgb2gray.cu:323-390, and the 27 dot products). RES workgroups (the rest):
+// residual and zWeight of 512 photometric points and their MAD histogram. The
+// two halves of a bi-objective iteration do not depend on each other. Bound by
+// memory traffic for full batches (80 B per geometric point), by latency for
+// small ones.
+//
+// XCD-aware as kb_ref_points: all workgroups of pair p run on XCD p % 8, so
+// that a row of the current cloud, which the points of two keyframe rows and
+// thus different virtual waves read, is fetched into one L2. 64 bi-objective
+// pairs of 320x240: 402 MB fetched a level-0 launch without, 280 MB with; 95 and
+// 66 us a launch (with 32-bit offsets for the gathers), 3.2 TB/s and half of
+// the vector issue rate at level 0.
+template <bool GEO, bool RES>
+__global__ __launch_bounds__(512, GEO ? 6 : 4) void kl_terms(const PairDesc* __restrict__ P, LockBufs B, int step,
+                                                             int mad_bins, int n_pairs, int chunks) {
+    const int xk = (int)blockIdx.x >> 3, p = ((int)blockIdx.x & 7) + 8 * (xk / chunks), chunk = xk % chunks;
+    if (p >= n_pairs) return;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = lane_id();
+    const PairDesc& d = P[p];
+    int layer, it;
+    if (!lock_level(d.L, d.iters, step, layer, it)) return;
+    const float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
+    float T[16];
+    lock_pose(d, T);
+    if constexpr (GEO) {
+        if (chunk < 16) {
+            __shared__ LockRound f[2];
+            const int vw = chunk;
+            const int w = d.W >> layer, h = d.H >> layer;
+            const int n = d.icnt[layer];
+            float v3 = 0.0f;
+            if (it == 0) {
+                if (n > 0) v3 = wave_student_total(B.bsum(p, 2), (n + 1023) / 1024, n);
+                if (vw == 0 && t == 0 && n > 0) d.ivar[layer * 3 + 2] = v3;
+            } else {
+                v3 = d.ivar[layer * 3 + 2];
+            }
+            float cl[96];
+#pragma unroll
+            for (int k = 0; k < 9; k++) cl[KL + k] = uni(d.calib[KL + k]);
+            float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+            const RT_GLOBAL int* isel = gmem(d.isel);
+            const RT_GLOBAL float* ir2 = gmem(d.ir2);
+            const IcpWeight iw = icp_weight(v3, n);
+            const float4* rp = d.rpos[layer];
+            const float4* rn = d.rnrm[layer];
+            const float4* cp = d.cpos[layer];
+            // the next round's point is loaded a round ahead
+            int i = 64 * vw + lane + 1024 * wave;
+            float x2 = 0.0f;
+            float4 p4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), n4 = p4;
+            if (i < n) {
+                const int o = isel[i];
+                x2 = ir2[i]; p4 = ldo(rp, o); n4 = ldo(rn, o);
+            }
+            for (int i0 = 64 * vw, buf = 0; i0 < n; i0 += 8192, buf ^= 1) {
+                float res = 0.0f, J[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                const bool in = i < n;
+                const float4 pc = p4, nc = n4;
+                const float xc = x2;
+                i += 8192;
+                if (i < n) {
+                    const int o = isel[i];
+                    x2 = ir2[i]; p4 = ldo(rp, o); n4 = ldo(rn, o);
+                }
+                if (in) icp_point_terms(pc, nc, cp, w, h, xc, iw, T, cl, a, b, 1e-3f, res, J);
+                f[buf][wave][0][lane] = make_float4(J[0], J[1], J[2], J[3]);
+                f[buf][wave][1][lane] = make_float4(J[4], J[5], res, 0.0f);
+                __syncthreads();  // one barrier a round: the other buffer was read before the previous one
+                lock_add<27, false>(wave, f[buf], acc);
+            }
+            lock_store<27>(wave, acc, B.wsum(p, 1) + 32 * vw);
+            return;
+        }
+    }
+    if constexpr (RES) {
+        __shared__ float lut[256];
+        __shared__ unsigned hist[256];
+        const int N = d.N, W = d.W, H = d.H;
+        const int c0 = (chunk - (GEO ? 16 : 0)) * 512;
+        if (c0 >= N) return;
+        if (layer == 0) load_lut(lut);
+        if (t < 256) hist[t] = 0u;
+        __syncthreads();
+        const int i = c0 + t;
+        if (i < N) {
+            const float* __restrict__ cl = d.calib;  // wave-uniform: scalar loads of what the path needs
+            const float4 p4 = ldg(d.pts, i);
+            const float ir = ldg(jac_view(d.jac[layer], N).iref, i);
+            const int wl = W >> layer, hl = H >> layer;
+            const U16BlockDepthSrc zs{gmem(d.zblk)};
+            float rr, zz;
+            if (layer == 0) {
+                const U8Src g{d.g8[1], lut};
+                if (d.simple) photo_point<true>(p4, ir, T, a, b, g, wl, hl, zs, W, H, cl, rr, zz);
+                else photo_point<false>(p4, ir, T, a, b, g, wl, hl, zs, W, H, cl, rr, zz);
+            } else {
+                const F32Src g{d.gray[1][layer]};
+                if (d.simple) photo_point<true>(p4, ir, T, a, b, g, wl, hl, zs, W, H, cl, rr, zz);
+                else photo_point<false>(p4, ir, T, a, b, g, wl, hl, zs, W, H, cl, rr, zz);
+            }
+            B.rz(p)[i] = make_float2(rr, zz);
+            const int bn = (int)((float)(mad_bins - 1) * fabsf(rr));
+            if (bn >= 0 && bn < mad_bins) atomicAdd(&hist[bn], 1u);
+        }
+        __syncthreads();
+        if (t < mad_bins && hist[t]) atomicAdd(&B.hist(p, step & 1)[t], hist[t]);
+    }
+}
+// The photometric system of virtual wave blockIdx.x: median of the MAD
+// histogram, robust weights, the 27 terms and the two sums of the residual RMS.
+__global__ __launch_bounds__(512) void kl_photo_sys(const PairDesc* __restrict__ P, LockBufs B, int step, int mad_bins,
+                                                    int robust) {
+    __shared__ LockRound f[2];
+    __shared__ int s_med;
+    const int p = blockIdx.y, vw = blockIdx.x, t = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = lane_id();
+    const PairDesc& d = P[p];
+    int layer, it;
+    if (!lock_level(d.L, d.iters, step, layer, it)) return;
+    const int N = d.N;
+    const JacView jv = jac_view(d.jac[layer], N);
+    const float2* rz = B.rz(p);
+    int i = 64 * vw + lane + 1024 * wave;
+    float2 v = make_float2(0.0f, 0.0f), jb = v;
+    float4 ja = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (i < N) { v = ldg(rz, i); ja = ldg(jv.a, i); jb = ldg(jv.b, i); }  // beside the median
+    if (wave == 0) median_bin(B.hist(p, step & 1), N, &s_med);
+    if (vw == 0 && t < 256) B.hist(p, (step + 1) & 1)[t] = 0u;  // last read a step ago
+    __syncthreads();
+    const float s = mad_scale(s_med, mad_bins);
+    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i0 = 64 * vw, buf = 0; i0 < N; i0 += 8192, buf ^= 1) {
+        float w = 0.0f, wr = 0.0f, jw[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        if (i < N) {
+            w = robust_weight(v.x, v.y, s, robust);
+            wr = v.x * w;
+            jw[0] = ja.x * w; jw[1] = ja.y * w; jw[2] = ja.z * w; jw[3] = ja.w * w; jw[4] = jb.x * w; jw[5] = jb.y * w;
+        }
+        i += 8192;
+        if (i < N) { v = ldg(rz, i); ja = ldg(jv.a, i); jb = ldg(jv.b, i); }
+        f[buf][wave][0][lane] = make_float4(jw[0], jw[1], jw[2], jw[3]);
+        f[buf][wave][1][lane] = make_float4(jw[4], jw[5], wr, w);
+        __syncthreads();
+        lock_add<29, true>(wave, f[buf], acc);
+    }
+    lock_store<29>(wave, acc, B.wsum(p, 0) + 32 * vw);
+}
+// The end of an iteration, one wave per pair: the 16 virtual waves' sums in
+// FP64 in order, the solve and the pose update; no update from an empty
+// geometric selection.
+__global__ __launch_bounds__(64) void kl_solve(const PairDesc* __restrict__ P, LockBufs B, int step, SolveCfg cfg) {
+    __shared__ double sys[56], ws[SOLVE_WS];
+    __shared__ float T[16];
+    const int p = blockIdx.x, t = threadIdx.x;
+    const PairDesc& d = P[p];
+    int layer, it;
+    if (!lock_level(d.L, d.iters, step, layer, it)) return;
+    const int n2 = cfg.mode == RT_PHOTOMETRIC ? 1 : d.icnt[layer];
+    // lane t: photometric terms 0-26, geometric ones 27-53, the RMS sums 54, 55
+    const bool geo = t >= 27 && t < 54;
+    if (t < 56 && (geo ? cfg.mode != RT_PHOTOMETRIC : cfg.mode != RT_GEOMETRIC)) {
+        const float* s = B.wsum(p, geo) + (geo ? t - 27 : (t < 27 ? t : t - 27));
+        float u[16];
+#pragma unroll
+        for (int q = 0; q < 16; q++) u[q] = s[32 * q];
+        double v = 0.0;
+#pragma unroll
+        for (int q = 0; q < 16; q++) v += (double)u[q];
+        sys[t] = v;
+    }
+    if (t < 16) T[t] = d.trel_out[t];
+    __syncthreads();
+    if (n2 > 0) {
+        const bool ok = solve_update_wave(sys, T, cfg, d.N, n2, ws);
+        if (t == 0 && !ok) *d.status = -1;
+    }
+    __syncthreads();
+    if (t < 16) d.trel_out[t] = T[t];
+    if (t == 0 && cfg.mode != RT_GEOMETRIC) *d.rms = sys[55] > 0.0 ? (float)sqrt(sys[54] / sys[55]) : 0.0f;
+}
+
 typedef void (*TrackFn)(const PairDesc*, const int*, int, int*, TrackCfg);
-struct Variant { int bs, ppt, rz, wpe; TrackFn fn; int pc = 0; int mode = RT_PHOTOMETRIC; };
+struct Variant { int bs, ppt, rz, wpe; TrackFn fn; int pc = 0; };
 static const Variant kVariants[] = {
     {256, 8, 0, 1, kb_track<256, 8, 0>},     {256, 16, 0, 1, kb_track<256, 16, 0>},
     {256, 32, 0, 1, kb_track<256, 32, 0>},   {512, 4, 0, 1, kb_track<512, 4, 0>},
@@ -1032,18 +1256,6 @@ static const Variant kVariants[] = {
     {512, 16, 0, 1, kb_track<512, 16, 0, 1, 1>, 8192},
     {1024, 2, 1, 1, kb_track<1024, 2, 1, 1, 1>, 5632},   {1024, 4, 1, 1, kb_track<1024, 4, 1, 1, 1>, 5632},
     {512, 4, 1, 1, kb_track<512, 4, 1, 1, 1>, 5632},     {1024, 2, 1, 1, kb_track<1024, 2, 1, 1, 1>, 5120},
-    // bi-objective: the photometric variants' shapes with the geometric terms
-    // (the selection's LDS leaves room for a smaller point cache)
-    {1024, 2, 1, 1, kb_track<1024, 2, 1, 1, 1, RT_BIOBJECTIVE>, 4608, RT_BIOBJECTIVE},
-    {1024, 4, 1, 1, kb_track<1024, 4, 1, 1, 1, RT_BIOBJECTIVE>, 4608, RT_BIOBJECTIVE},
-    {1024, 2, 1, 1, kb_track<1024, 2, 1, 1, 0, RT_BIOBJECTIVE>, 0, RT_BIOBJECTIVE},
-    {1024, 8, 0, 1, kb_track<1024, 8, 0, 1, 0, RT_BIOBJECTIVE>, 0, RT_BIOBJECTIVE},
-    {512, 4, 1, 1, kb_track<512, 4, 1, 1, 0, RT_BIOBJECTIVE>, 0, RT_BIOBJECTIVE},
-    {256, 4, 1, 1, kb_track<256, 4, 1, 1, 0, RT_BIOBJECTIVE>, 0, RT_BIOBJECTIVE},
-    // geometric only: no photometric points (ppt and rz unused)
-    {1024, 1, 0, 1, kb_track<1024, 1, 0, 1, 0, RT_GEOMETRIC>, 0, RT_GEOMETRIC},
-    {512, 1, 0, 1, kb_track<512, 1, 0, 1, 0, RT_GEOMETRIC>, 0, RT_GEOMETRIC},
-    {256, 1, 0, 1, kb_track<256, 1, 0, 1, 0, RT_GEOMETRIC>, 0, RT_GEOMETRIC},
 };
 
 }  // namespace rt
@@ -1095,9 +1307,23 @@ struct rt_batch {
     int variant = -1, grid = 0;
     hipGraphExec_t graph_pyr = nullptr, graph_bins = nullptr, graph_sel = nullptr, graph_track = nullptr;
     int graph_n = -1, graph_variant = -1, graph_grid = -1, graph_maxN = -1;  // the track graph's launch shape
+    // lockstep tracking: its arrays for the first lock_pairs pairs, and the
+    // graph of its launches with the shape they were captured for
+    LockBufs lock{};
+    int lock_pairs = 0;
+    hipGraphExec_t graph_lock = nullptr;
+    int lock_key[5] = {-1, -1, -1, -1, -1};  // pairs, largest width, height and point count, pyramid depths
 };
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// Photometric batches up to this many pairs track in lockstep; larger ones
+// keep enough CUs busy with a workgroup of kb_track each. Tracking alone at
+// 8192 points, lockstep and the best kb_track variant: 640x480, 1 pair 259 and
+// 300 us, 16 pairs 293 and 325, 32 pairs 335 and 331, 64 pairs 440 and 371;
+// 320x240, 1 pair 198 and 243 us, 16 pairs 214 and 257, 32 pairs 244 and 260,
+// 64 pairs 318 and 282.
+constexpr int LOCK_PHOTO_PAIRS = 24;
 
 // Device memory a batch's descriptors point into: per-pair arenas of
 // pair_bytes (sized for max_w x max_h and nsel points) and the per-pair tables.
@@ -1167,6 +1393,13 @@ extern "C" int rt_batch_create(int device, int max_pairs, int max_w, int max_h, 
               dal((void**)&b->queue, 256) && dal((void**)&b->calib_dev, 96 * 4 * (size_t)max_pairs) &&
               dal((void**)&b->trel_in, 64 * (size_t)max_pairs) && dal((void**)&b->trel_out, 64 * (size_t)max_pairs) &&
               dal((void**)&b->rms, 4 * (size_t)max_pairs) && dal((void**)&b->status, 4 * (size_t)max_pairs);
+    b->lock_pairs = b->prm.mode == RT_PHOTOMETRIC ? std::min(max_pairs, LOCK_PHOTO_PAIRS) : max_pairs;
+    const bool icp = b->prm.mode != RT_PHOTOMETRIC;
+    b->lock.o_rz = align256(LK_FIXED);
+    b->lock.o_bits = b->lock.o_rz + align256(8 * (size_t)b->prm.n_select);
+    b->lock.o_rfull = b->lock.o_bits + (icp ? 8 * 16 * (size_t)LK_BLOCKS : 0);
+    b->lock.stride = align256(b->lock.o_rfull + (icp ? 4 * (size_t)max_w * max_h : 0));
+    ok = ok && dal((void**)&b->lock.base, b->lock.stride * (size_t)b->lock_pairs);
     if (!ok) {
         rt_batch_destroy(b);
         return set_error(RT_ERR_NOMEM, "batch buffers");
@@ -1184,6 +1417,7 @@ extern "C" void rt_batch_destroy(rt_batch* b) {
     if (b->graph_bins) hipGraphExecDestroy(b->graph_bins);
     if (b->graph_sel) hipGraphExecDestroy(b->graph_sel);
     if (b->graph_track) hipGraphExecDestroy(b->graph_track);
+    if (b->graph_lock) hipGraphExecDestroy(b->graph_lock);
     for (void* p : b->allocs) hipFree(p);
     b->st_desc.release(); b->st_calib.release(); b->st_order.release(); b->st_trel.release(); b->st_res.release();
     if (b->inputs) hipEventDestroy(b->inputs);
@@ -1235,14 +1469,11 @@ static void launch_prep(const BatchView& v, hipStream_t s, int part = 0) {
     kb_ref_points<<<8 * ((n + 7) / 8) * chunks, 256, 0, s>>>(v.desc, n, chunks);
     if (v.mode != RT_PHOTOMETRIC) {
         kb_clouds<<<dim3((v.maxW + 15) / 16, (v.maxH + 15) / 16, n), 256, 0, s>>>(v.desc);
-        for (int l = 1; l < 4; l++)
-            kb_clouds_down<<<dim3(((v.maxW >> l) * (v.maxH >> l) + 255) / 256, n), 256, 0, s>>>(v.desc, l);
     }
 }
 
 static TrackCfg track_cfg(const BatchView& bv, const Variant& v) {
     TrackCfg c;
-    c.lambda = bv.lambda;
     c.pc_cap = v.pc;
     c.rz_len = bv.maxN;
     c.solver = bv.solver;
@@ -1254,7 +1485,7 @@ static TrackCfg track_cfg(const BatchView& bv, const Variant& v) {
 
 static size_t track_dyn_lds(const Variant& v, int maxN) {
     size_t n = 0;
-    if (v.rz && v.mode != RT_GEOMETRIC) n += sizeof(float2) * (size_t)maxN;
+    if (v.rz) n += sizeof(float2) * (size_t)maxN;
     if (v.pc) n += sizeof(float4) * (size_t)std::min(maxN, v.pc);
     return n;
 }
@@ -1313,10 +1544,7 @@ static int autotune(rt_batch* b) {
     int bv = -1, bg = 0;
     for (int v = 0; v < NUM_VARIANTS; v++) {
         const Variant& var = kVariants[v];
-        if (var.mode != b->prm.mode) continue;
-        if (var.mode == RT_GEOMETRIC) {
-            if (!lds_variant_ready(var, b->maxN)) continue;  // no photometric points to cover
-        } else if (var.rz) {
+        if (var.rz) {
             if (!lds_variant_ready(var, b->maxN)) continue;
         } else {
             if (var.bs * var.ppt < b->maxN) continue;
@@ -1354,21 +1582,74 @@ static int autotune(rt_batch* b) {
     return RT_OK;
 }
 
+// The lockstep launches of the prepared batch: depths has bit L set where a
+// pair has L pyramid levels.
+static void launch_lockstep(const rt_batch* b, int depths, hipStream_t s) {
+    const BatchView v = view_of(b);
+    const int n = v.n;
+    const int* iters = b->prm.iters;
+    SolveCfg cfg;
+    cfg.solver = v.solver; cfg.mode = v.mode; cfg.lambda = v.lambda; cfg.scale_out = 1e3f;
+    cfg.robust = v.robust; cfg.mad_bins = v.mad_bins; cfg.scale_in = 1e-3f;
+    int steps = 0;
+    for (int L = 1; L <= 4; L++) {
+        int c = 0;
+        for (int k = 0; k < L; k++) c += iters[k];
+        if (depths >> L & 1) steps = std::max(steps, c);
+    }
+    const int res = (v.maxN + 511) / 512;
+    kl_init<<<n, 256, 0, s>>>(v.desc, b->lock);
+    for (int step = 0; step < steps; step++) {
+        if (v.mode != RT_PHOTOMETRIC) {
+            int blocks = 0;  // 1024-pixel blocks of the largest level that begins here
+            for (int L = 1; L <= 4; L++) {
+                int layer, it;
+                if (!(depths >> L & 1) || !lock_level(L, iters, step, layer, it) || it != 0) continue;
+                blocks = std::max(blocks, ((v.maxW >> layer) * (v.maxH >> layer) + 1023) / 1024);
+            }
+            if (blocks) {
+                kl_icp_mask<<<dim3(blocks, n), 1024, 0, s>>>(v.desc, b->lock, step);
+                kl_icp_compact<<<dim3(blocks, n), 1024, 0, s>>>(v.desc, b->lock, step);
+                for (int r = 1; r <= 3; r++)
+                    kl_student<<<dim3((blocks + 3) / 4, n), 256, 0, s>>>(v.desc, b->lock, step, r);
+            }
+        }
+        const int chunks = (v.mode != RT_PHOTOMETRIC ? 16 : 0) + (v.mode != RT_GEOMETRIC ? res : 0);
+        const int grid = 8 * ((n + 7) / 8) * chunks;
+        if (v.mode == RT_GEOMETRIC)
+            kl_terms<true, false><<<grid, 512, 0, s>>>(v.desc, b->lock, step, v.mad_bins, n, chunks);
+        else if (v.mode == RT_PHOTOMETRIC)
+            kl_terms<false, true><<<grid, 512, 0, s>>>(v.desc, b->lock, step, v.mad_bins, n, chunks);
+        else kl_terms<true, true><<<grid, 512, 0, s>>>(v.desc, b->lock, step, v.mad_bins, n, chunks);
+        if (v.mode != RT_GEOMETRIC)
+            kl_photo_sys<<<dim3(16, n), 512, 0, s>>>(v.desc, b->lock, step, v.mad_bins, v.robust);
+        kl_solve<<<n, 64, 0, s>>>(v.desc, b->lock, step, cfg);
+    }
+}
+// The geometric modes always, photometric batches while they are small (a
+// variant forced through the environment keeps kb_track).
+static bool tracks_in_lockstep(const rt_batch* b) {
+    if (b->prm.mode != RT_PHOTOMETRIC) return true;
+    return b->n <= b->lock_pairs && !getenv("RT_BATCH_VARIANT");
+}
+
 // The kernel variant table, for tests that force each variant through
 // RT_BATCH_VARIANT: info = {workgroup size, points per thread (unroll depth
 // for rz), residuals in LDS, point-cache capacity, waves per SIMD, mode}.
 extern "C" int rt_batch_variant_info(int v, int info[6]) {
     if (!info || v < 0 || v >= NUM_VARIANTS) return set_error(RT_ERR_ARG, "rt_batch_variant_info: no such variant");
     const Variant& k = kVariants[v];
-    info[0] = k.bs; info[1] = k.ppt; info[2] = k.rz; info[3] = k.pc; info[4] = k.wpe; info[5] = k.mode;
+    info[0] = k.bs; info[1] = k.ppt; info[2] = k.rz; info[3] = k.pc; info[4] = k.wpe; info[5] = RT_PHOTOMETRIC;
     return RT_OK;
 }
 
-// prep: 0 the tracking launch, else the part of the preparation (launch_prep)
-static int capture(rt_batch* b, hipGraphExec_t* out, int prep) {
+// prep: 0 the tracking launch, -1 the lockstep launches of pairs with the given
+// depths, else the part of the preparation (launch_prep)
+static int capture(rt_batch* b, hipGraphExec_t* out, int prep, int depths = 0) {
     hipGraph_t g;
     if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return set_error(RT_ERR_HIP, "begin capture");
-    if (prep) launch_prep(view_of(b), b->stream, prep);
+    if (prep > 0) launch_prep(view_of(b), b->stream, prep);
+    else if (prep < 0) launch_lockstep(b, depths, b->stream);
     else launch_track(b, b->variant, b->grid, b->stream);
     if (hipStreamEndCapture(b->stream, &g) != hipSuccess) return set_error(RT_ERR_HIP, "end capture");
     if (*out) hipGraphExecDestroy(*out);
@@ -1404,7 +1685,19 @@ static int fetch_results(rt_batch* b, rt_pair_result* out) {
 }
 
 static int run_track(rt_batch* b, rt_pair_result* out) {
-    int rc = autotune(b);
+    int rc;
+    if (tracks_in_lockstep(b)) {
+        int depths = 0;
+        for (const PairDesc& d : b->desc) depths |= 1 << d.L;
+        const int key[5] = {b->n, b->maxW, b->maxH, b->maxN, depths};
+        if (!b->graph_lock || memcmp(key, b->lock_key, sizeof(key))) {
+            if ((rc = capture(b, &b->graph_lock, -1, depths))) return rc;
+            memcpy(b->lock_key, key, sizeof(key));
+        }
+        if (hipGraphLaunch(b->graph_lock, b->stream) != hipSuccess) return set_error(RT_ERR_HIP, "graph launch");
+        return out ? fetch_results(b, out) : RT_OK;
+    }
+    rc = autotune(b);
     if (rc) return rc;
     // the captured launch depends on the batch size, the variant, the grid and,
     // through its dynamic LDS, on the largest point count
@@ -1724,7 +2017,7 @@ int noalloc_variant(int maxN) {
     int fallback = -1;
     for (int v = 0; v < NUM_VARIANTS; v++) {
         const rt::Variant& k = rt::kVariants[v];
-        if (k.bs != 1024 || k.mode != RT_PHOTOMETRIC) continue;
+        if (k.bs != 1024) continue;
         if (k.rz && k.pc && k.ppt == 4 && lds_variant_ready(k, maxN)) return v;
         if (!k.rz && !k.pc && k.bs * k.ppt >= maxN && fallback < 0) fallback = v;
     }

@@ -116,6 +116,12 @@ __device__ __forceinline__ float2 ldg(const float2* p, size_t i) {
     return make_float2(v.x, v.y);
 }
 
+// element i of a float4 array of less than 2^28: a scalar base and a 32-bit offset
+__device__ __forceinline__ float4 ldo(const float4* p, unsigned i) {
+    const nfloat4 v = at_offset((const RT_GLOBAL nfloat4*)p, 16u * i);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
 // stores of element i through the global address space
 __device__ __forceinline__ void stg(float4* p, size_t i, float4 v) {
     ((RT_GLOBAL nfloat4*)p)[i] = nfloat4{v.x, v.y, v.z, v.w};

@@ -517,23 +517,39 @@ __global__ __launch_bounds__(256) void k_ref_cloud(const float* __restrict__ z, 
                                                    float4* __restrict__ pos, float4* __restrict__ nrm) {
     int x = blockIdx.x * 16 + (threadIdx.x & 15), y = blockIdx.y * 16 + (threadIdx.x >> 4);
     if (x >= W || y >= H) return;
-    ref_cloud_pixel(F32Src{z}, W, H, x, y, c, pos, nrm);
+    float4 p, n;
+    ref_cloud_pixel(F32Src{z}, W, H, x, y, c, 1.0f / c[KL], 1.0f / c[KL + 4], p, n);
+    pos[x + (size_t)y * W] = p;
+    nrm[x + (size_t)y * W] = n;
 }
 
-// genPointsCloud6Kernel (d2z.cu:436-469): every z < 0 is valid.
-__global__ __launch_bounds__(256) void k_cur_cloud(const float* __restrict__ z, int W, int H, const float* __restrict__ c,
-                                                   float4* __restrict__ pos) {
-    int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= W * H) return;
-    cur_cloud_pixel(F32Src{z}, W, i, c, pos);
+struct CloudPtrs {
+    float4* pos[4];
+    float4* nrm[4];
+};
+// downSampleCloud6Kernel (d2z.cu:557-588), every level in one launch: masked
+// 2x2 mean, normal renormalised, from level 0 in place.
+__global__ __launch_bounds__(256) void k_ref_cloud_levels(CloudPtrs r, int W, int H, int L) {
+    __shared__ float4 lp[CLOUD_TILE], ln[CLOUD_TILE];
+    const int t = threadIdx.x, x = blockIdx.x * 16 + (t & 15), y = blockIdx.y * 16 + (t >> 4);
+    const bool in = x < W && y < H;
+    lp[t] = in ? r.pos[0][x + (size_t)y * W] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    ln[t] = in ? r.nrm[0][x + (size_t)y * W] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    cloud_tile_levels<true>(lp, ln, blockIdx.x, blockIdx.y, W, H, L, r.pos, r.nrm);
 }
-
-// downSampleCloud6Kernel (d2z.cu:557-588): masked 2x2 mean, normal renormalised.
-__global__ __launch_bounds__(256) void k_cloud_down(const float4* __restrict__ sp, const float4* __restrict__ sn, int Wd,
-                                                    int Hd, float4* __restrict__ dp, float4* __restrict__ dn) {
-    int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= Wd * Hd) return;
-    cloud_down_pixel(sp, sn, Wd, i, dp, dn);
+// genPointsCloud6Kernel (d2z.cu:436-469), every z < 0 is valid, and its levels.
+__global__ __launch_bounds__(256) void k_cur_cloud(const float* __restrict__ z, int W, int H, int L,
+                                                   const float* __restrict__ c, CloudPtrs r) {
+    __shared__ float4 lp[CLOUD_TILE];
+    const int t = threadIdx.x, x = blockIdx.x * 16 + (t & 15), y = blockIdx.y * 16 + (t >> 4);
+    lp[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (x < W && y < H) {
+        const size_t o = x + (size_t)y * W;
+        const float4 p = cur_cloud_pixel(z[o], x, y, c, 1.0f / c[KL], 1.0f / c[KL + 4]);
+        r.pos[0][o] = p;
+        lp[t] = p;
+    }
+    cloud_tile_levels<false>(lp, nullptr, blockIdx.x, blockIdx.y, W, H, L, r.pos, nullptr);
 }
 
 void launch_ref_cloud(const Dev& d, hipStream_t s) {
@@ -618,20 +634,17 @@ void launch_ref_oriented(const Dev& d, const float* xyz, const float* nrm, hipSt
     const int n = d.W * d.H;
     k_ref_oriented<<<(n + 255) / 256, 256, 0, s>>>((const float4*)xyz, (const float4*)nrm, n, d.rpos[0], d.rnrm[0]);
 }
+static CloudPtrs cloud_ptrs(float4* const* pos, float4* const* nrm) {
+    CloudPtrs r;
+    for (int l = 0; l < 4; l++) { r.pos[l] = pos[l]; r.nrm[l] = nrm ? nrm[l] : nullptr; }
+    return r;
+}
 void launch_ref_cloud_pyramid(const Dev& d, hipStream_t s) {
-    for (int l = 1; l < d.L; l++) {
-        int n = (d.W >> l) * (d.H >> l);
-        k_cloud_down<<<(n + 255) / 256, 256, 0, s>>>(d.rpos[l - 1], d.rnrm[l - 1], d.W >> l, d.H >> l, d.rpos[l],
-                                                     d.rnrm[l]);
-    }
+    k_ref_cloud_levels<<<dim3((d.W + 15) / 16, (d.H + 15) / 16), 256, 0, s>>>(cloud_ptrs(d.rpos, d.rnrm), d.W, d.H, d.L);
 }
 void launch_cur_cloud(const Dev& d, hipStream_t s) {
-    int n = d.W * d.H;
-    k_cur_cloud<<<(n + 255) / 256, 256, 0, s>>>(d.cur.z, d.W, d.H, d.calib, d.cpos[0]);
-    for (int l = 1; l < d.L; l++) {
-        int m = (d.W >> l) * (d.H >> l);
-        k_cloud_down<<<(m + 255) / 256, 256, 0, s>>>(d.cpos[l - 1], nullptr, d.W >> l, d.H >> l, d.cpos[l], nullptr);
-    }
+    k_cur_cloud<<<dim3((d.W + 15) / 16, (d.H + 15) / 16), 256, 0, s>>>(d.cur.z, d.W, d.H, d.L, d.calib,
+                                                                       cloud_ptrs(d.cpos, nullptr));
 }
 
 // ------------------------------------------------------------------ A20 + A21
@@ -705,62 +718,25 @@ __global__ __launch_bounds__(1024) void k_icp_compact(const float* __restrict__ 
 
 // generateStudentTWeights (rgb2gray.cu:470-568, 854-877), round k in 1..3: the
 // weights of the previous round are recomputed from its variance, the products
-// are truncated to int per element (one element per thread) and summed by the
-// reference's 1024-wide tree into this round's block sums. The variance of the
-// previous round, the reference's last-block combination of its block sums
-// (int truncation per block sum, the same tree, clamped to at least n with
-// more than one block), is recomputed by every block from those sums, and
-// stored by block 0; k_student_finish combines the third round's.
-__device__ __forceinline__ void tree1024(float* p, int t) {
-    for (int s = 512; s >= 1; s >>= 1) {
-        if (t < s) p[t] += p[t + s];
-        __syncthreads();
-    }
-}
-__device__ __forceinline__ float student_total(const float* __restrict__ bsum, int nb, int n, float* p, int t) {
-    if (nb == 1) return bsum[0];
-    int ss = 0;
-    for (int q = t; q < nb; q += 1024) ss += bsum[q];
-    p[t] = (float)ss;
-    __syncthreads();
-    tree1024(p, t);
-    float v = p[0];
-    const float mn = (float)n;
-    if (v < mn) v = mn;
-    __syncthreads();
-    return v;
-}
-__global__ __launch_bounds__(1024) void k_student_round(const float* __restrict__ r2, const int* __restrict__ nptr,
-                                                        int round, float* var, float* bsum, int stride) {
-    __shared__ float p[1024];
+// are truncated to int per element and summed by the reference's 1024-wide
+// tree into this round's block sums, one wave per block of 1024. The variance
+// of the previous round, the reference's last-block combination of its block
+// sums (int truncation per block sum, the same tree, clamped to at least n with
+// more than one block), is recomputed by every wave from those sums, and stored
+// by the first; the level's first system pass combines the third round's.
+__global__ __launch_bounds__(256) void k_student_round(const float* __restrict__ r2, const int* __restrict__ nptr,
+                                                       int round, float* var, float* bsum, int stride) {
     const int n = *nptr;
-    const int t = threadIdx.x;
+    const int bk = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int nb = (n + 1023) / 1024;
+    if (bk >= nb) return;
     float prev = 0.0f;
-    if (round > 1 && nb >= 1) {
-        prev = student_total(bsum + (size_t)(round - 2) * stride, nb, n, p, t);
-        if (blockIdx.x == 0 && t == 0) var[round - 2] = prev;
+    if (round > 1) {
+        prev = wave_student_total(bsum + (size_t)(round - 2) * stride, nb, n);
+        if (bk == 0 && lane_id() == 0) var[round - 2] = prev;
     }
-    const int i = blockIdx.x * 1024 + t;
-    int sum = 0;
-    if (i < n) {
-        float x = r2[i];
-        float w = round == 1 ? 6 / (5 + x / 100.0f) : 6 / (5 + x / (prev / (float)n));
-        sum += x * w;
-    }
-    p[t] = (float)sum;
-    __syncthreads();
-    tree1024(p, t);
-    if (t == 0) bsum[(size_t)(round - 1) * stride + blockIdx.x] = p[0];
-}
-__global__ __launch_bounds__(1024) void k_student_finish(const int* __restrict__ nptr, float* var,
-                                                         const float* __restrict__ bsum, int stride) {
-    __shared__ float p[1024];
-    const int n = *nptr;
-    const int nb = (n + 1023) / 1024;
-    if (nb < 1) return;
-    const float v = student_total(bsum + 2 * (size_t)stride, nb, n, p, threadIdx.x);
-    if (threadIdx.x == 0) var[2] = v;
+    const float s = wave_student_block(r2, bk, n, round, prev);
+    if (lane_id() == 0) bsum[(size_t)(round - 1) * stride + bk] = s;
 }
 
 // icpResidualIndexKernel2 (rgb2gray.cu:323-390) with the final clamped
@@ -772,7 +748,9 @@ struct IcpSysArgs {
     const int* sel;
     const float* r2;
     const int* nptr;
-    const float* var;
+    float* var;         // the rounds' variance sums; the third is formed at the level's first pass
+    const float* bsum3; // block sums of the third round
+    int first;
     int w, h, layer;
     const float* c;
     const float4* cp;
@@ -789,12 +767,24 @@ __device__ __forceinline__ void icp_sys_body(const IcpSysArgs& g, const SolveIn&
     const float* __restrict__ r2 = g.r2;
     const float* __restrict__ c = g.c;
     const float4* __restrict__ cp = g.cp;
-    const float* __restrict__ var = g.var;
     const int w = g.w, h = g.h, layer = g.layer;
     const float scale_in = g.scale_in;
     const int* nptr = g.nptr;
     int n = *nptr;
-    float v3 = var[2];
+    // the thread's first point is loaded before the solve, which does not need it
+    int i = grp * NT + threadIdx.x;
+    int o = 0;
+    float x2 = 0.0f;
+    float4 p4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), n4 = p4;
+    if (i < n) { o = sel[i]; x2 = r2[i]; p4 = ldo(rp, o); n4 = ldo(rn, o); }
+    float v3 = 0.0f;
+    if (!g.first) {
+        v3 = g.var[2];
+    } else if (n > 0) {
+        v3 = wave_student_total(g.bsum3, (n + 1023) / 1024, n);
+        if (grp == 0 && threadIdx.x == 0) g.var[2] = v3;
+    }
+    const IcpWeight iw = icp_weight(v3, n);
     solve_pending<NT>(in, q);
     float T[16];
 #pragma unroll
@@ -803,9 +793,13 @@ __device__ __forceinline__ void icp_sys_body(const IcpSysArgs& g, const SolveIn&
 #pragma unroll
     for (int k = 0; k < 27; k++) acc[k] = 0.0;
     float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
-    for (int i = grp * NT + threadIdx.x; i < n; i += ngrp * NT) {
+    while (i < n) {
         float res, J[6];
-        icp_point_terms(rp, rn, cp, w, h, sel[i], r2[i], v3, n, T, c, a, b, scale_in, res, J);
+        const float4 pc = p4, nc = n4;
+        const float xc = x2;
+        i += ngrp * NT;
+        if (i < n) { o = sel[i]; x2 = r2[i]; p4 = ldo(rp, o); n4 = ldo(rn, o); }  // the next point, ahead
+        icp_point_terms(pc, nc, cp, w, h, xc, iw, T, c, a, b, scale_in, res, J);
         int k = 0;
 #pragma unroll
         for (int r0 = 0; r0 < 6; r0++)
@@ -847,13 +841,16 @@ void launch_icp_select(const Dev& d, int layer, const SolveCfg& c, EstState& e, 
                                      d.icp_n + layer);
     const int stride = (d.W * d.H + 1023) / 1024;
     for (int r = 1; r <= 3; r++)
-        k_student_round<<<G, 1024, 0, s>>>(d.icp_r2[layer], d.icp_n + layer, r, d.icp_var + layer * 4, d.bsum, stride);
-    k_student_finish<<<1, 1024, 0, s>>>(d.icp_n + layer, d.icp_var + layer * 4, d.bsum, stride);
+        k_student_round<<<(G + 3) / 4, 256, 0, s>>>(d.icp_r2[layer], d.icp_n + layer, r, d.icp_var + layer * 4, d.bsum,
+                                                    stride);
+    e.first = true;
 }
 
-static IcpSysArgs icp_sys_args(const Dev& d, int layer, const SolveCfg& c, double* part, int stride) {
+static IcpSysArgs icp_sys_args(const Dev& d, int layer, const SolveCfg& c, EstState& e, double* part, int stride) {
+    const int first = e.first;
+    e.first = false;
     return IcpSysArgs{d.rpos[layer], d.rnrm[layer], d.icp_sel[layer], d.icp_r2[layer], d.icp_n + layer,
-                      d.icp_var + layer * 4, d.W >> layer, d.H >> layer, layer, d.calib, d.cpos[layer], part, stride,
+                      d.icp_var + layer * 4, d.bsum + 2 * (size_t)((d.W * d.H + 1023) / 1024), first, d.W >> layer, d.H >> layer, layer, d.calib, d.cpos[layer], part, stride,
                       c.scale_in};
 }
 
@@ -863,7 +860,7 @@ void launch_icp_system(const Dev& d, int layer, const SolveCfg& c, EstState& e, 
     const int Gi = sys_groups((d.W >> layer) * (d.H >> layer));
     double* part = e.it & 1 ? d.part : d.part2;
     const SolveIn in = take_pending(d, c, e);
-    k_icp_sys<<<Gi, SYS_THREADS, 0, s>>>(icp_sys_args(d, layer, c, part, PART_STRIDE), in);
+    k_icp_sys<<<Gi, SYS_THREADS, 0, s>>>(icp_sys_args(d, layer, c, e, part, PART_STRIDE), in);
     set_pending(e, 0, Gi, part, d.icp_n + layer);
 }
 
@@ -878,7 +875,7 @@ void launch_biobjective_iteration(const Dev& d, int layer, const SolveCfg& c, Es
     k_bi_res<<<Gr + Gi, SYS_THREADS, 0, s>>>(d.pts, d.jac[layer], d.N, layer, d.cur.gray[layer], d.W >> layer,
                                              d.H >> layer, d.cur.z, d.W, d.H, d.calib, c.mad_bins, d.res,
                                              d.madhist + (e.it & 1 ? 512 : 0), Gr,
-                                             icp_sys_args(d, layer, c, d.part3, RAW_STRIDE), take_pending(d, c, e));
+                                             icp_sys_args(d, layer, c, e, d.part3, RAW_STRIDE), take_pending(d, c, e));
     const int Gs = launch_photo_sys(d, layer, c, e.it, d.part3, Gi, d.part2, nf, s);
     set_pending(e, Gs, nf, d.part2, d.icp_n + layer);
 }

@@ -114,6 +114,7 @@ struct EstState {
     float* T;         // the pose the pending solve starts from (or the current one)
     int it = 0;       // iterations launched
     bool pending = false;
+    bool first = false;  // the level's ICP points have just been selected
     int gp = 0, gi = 0;
     const double* part2 = nullptr;  // the geometric sums
     const int* nptr = nullptr;

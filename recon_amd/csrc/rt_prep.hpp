@@ -772,25 +772,37 @@ __device__ __forceinline__ float robust_weight(float r, float zw, float s, int r
 
 
 // ------------------------------------------------------------------ A18-A23 per pixel / point
+// backproject with the quotients by the focal lengths as div_rn (ifx, ify: RN
+// of their reciprocals): the same values, a zero coordinate's sign aside.
+__device__ __forceinline__ bool backproject_rn(float z, int xi, int yi, const float* c, float ifx, float ify, f3& p) {
+    if (z < -c[MIND] && z > -c[MAXD]) {
+        p.x = div_rn(((float)xi - c[KL + 2]) * z, c[KL], ifx);
+        p.y = div_rn(((float)yi - c[KL + 5]) * z, c[KL + 4], ify);
+        p.z = z;
+        return true;
+    }
+    p.x = 0.0f; p.y = 0.0f; p.z = 0.0f;
+    return false;
+}
 // convertZMapToXYZ6Kernel (rgb2gray.cu:595-624) + computeNormalsCudaKernel
 // (d2z.cu:503-537) for pixel (x, y): position (x, y, z, mask) and normal from
 // the depth source zs (z < 0 valid).
 template <class ZS>
 __device__ __forceinline__ void ref_cloud_pixel(const ZS& zs, int W, int H, int x, int y, const float* __restrict__ c,
-                                                float4* __restrict__ pos, float4* __restrict__ nrm) {
+                                                float ifx, float ify, float4& pos, float4& nrm) {
     size_t o = (size_t)x + (size_t)y * W;
     f3 p;
-    bool valid = backproject(zs[o], x, y, c, p);
+    bool valid = backproject_rn(zs[o], x, y, c, ifx, ify, p);
     float mask = valid ? 1.0f : 0.0f;
-    float4 n = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    nrm = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (x < 1 || y < 1 || x > W - 2 || y > H - 2) {
         mask = 0.0f;
     } else {
         f3 a, b2, cc, dd;
-        backproject(zs[o - 1], x - 1, y, c, a);
-        backproject(zs[o + 1], x + 1, y, c, b2);
-        backproject(zs[o - W], x, y - 1, c, cc);
-        backproject(zs[o + W], x, y + 1, c, dd);
+        backproject_rn(zs[o - 1], x - 1, y, c, ifx, ify, a);
+        backproject_rn(zs[o + 1], x + 1, y, c, ifx, ify, b2);
+        backproject_rn(zs[o - W], x, y - 1, c, ifx, ify, cc);
+        backproject_rn(zs[o + W], x, y + 1, c, ifx, ify, dd);
         if (a.z < 0.0f && b2.z < 0.0f && cc.z < 0.0f && dd.z < 0.0f) {
             f3 u{b2.x - a.x, b2.y - a.y, b2.z - a.z};
             f3 v{dd.x - cc.x, dd.y - cc.y, dd.z - cc.z};
@@ -799,57 +811,83 @@ __device__ __forceinline__ void ref_cloud_pixel(const ZS& zs, int W, int H, int 
             float nz = u.x * v.y - u.y * v.x;
             float len = nx * nx + ny * ny + nz * nz;
             len = 1.0f / sqrtf(len);
-            n = make_float4(nx * len, ny * len, nz * len, 0.0f);
+            nrm = make_float4(nx * len, ny * len, nz * len, 0.0f);
         } else {
             mask = 0.0f;
         }
     }
-    pos[o] = make_float4(p.x, p.y, p.z, mask);
-    nrm[o] = n;
+    pos = make_float4(p.x, p.y, p.z, mask);
 }
-// genPointsCloud6Kernel (d2z.cu:436-469) for pixel i: every z < 0 is valid.
-template <class ZS>
-__device__ __forceinline__ void cur_cloud_pixel(const ZS& zs, int W, int i, const float* __restrict__ c,
-                                                float4* __restrict__ pos) {
-    int x = i % W, y = i / W;
-    float zz = zs[(size_t)i];
-    if (zz < 0.0f) {
-        float fx = c[KL], fy = c[KL + 4], cx = c[KL + 2], cy = c[KL + 5];
-        pos[i] = make_float4(((float)x - cx) * zz / fx, ((float)y - cy) * zz / fy, zz, 1.0f);
-    } else {
-        pos[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
+// genPointsCloud6Kernel (d2z.cu:436-469) for pixel (x, y): every z < 0 is valid.
+__device__ __forceinline__ float4 cur_cloud_pixel(float z, int x, int y, const float* __restrict__ c, float ifx,
+                                                  float ify) {
+    if (!(z < 0.0f)) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    return make_float4(div_rn(((float)x - c[KL + 2]) * z, c[KL], ifx), div_rn(((float)y - c[KL + 5]) * z, c[KL + 4], ify),
+                       z, 1.0f);
 }
-// downSampleCloud6Kernel (d2z.cu:557-588) for destination pixel i of a
-// Wd x Hd level: masked 2x2 mean, normal renormalised (sn / dn may be null).
-__device__ __forceinline__ void cloud_down_pixel(const float4* __restrict__ sp, const float4* __restrict__ sn, int Wd,
-                                                 int i, float4* __restrict__ dp, float4* __restrict__ dn) {
-    int x = i % Wd, y = i / Wd;
-    int Ws = Wd * 2;
-    size_t h = (size_t)x * 2 + (size_t)y * 2 * Ws;
-    size_t hs[4] = {h, h + 1, h + Ws, h + Ws + 1};
+// downSampleCloud6Kernel (d2z.cu:557-588) for one pixel from its four taps:
+// masked mean position and, with normals, their masked mean renormalised.
+template <bool NRM>
+__device__ __forceinline__ void cloud_mean(const float4* p, const float4* q, float4& op, float4& on) {
     float d[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     float n = 0.0f;
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-        float4 p = sp[hs[t]];
-        if (p.w != 0.0f) {
+        if (p[t].w != 0.0f) {
             n++;
-            d[0] += p.x; d[1] += p.y; d[2] += p.z;
-            if (sn) { float4 q = sn[hs[t]]; d[3] += q.x; d[4] += q.y; d[5] += q.z; }
+            d[0] += p[t].x; d[1] += p[t].y; d[2] += p[t].z;
+            if (NRM) { d[3] += q[t].x; d[4] += q[t].y; d[5] += q[t].z; }
         }
     }
     if (n > 0.0f) {
-        for (int k = 0; k < 6; k++) d[k] /= n;
-        dp[i] = make_float4(d[0], d[1], d[2], 1.0f);
-        if (dn) {
+#pragma unroll
+        for (int k = 0; k < (NRM ? 6 : 3); k++) d[k] /= n;
+        op = make_float4(d[0], d[1], d[2], 1.0f);
+        if (NRM) {
             float len = d[3] * d[3] + d[4] * d[4] + d[5] * d[5];
             len = 1.0f / sqrtf(len);
-            dn[i] = make_float4(d[3] * len, d[4] * len, d[5] * len, 0.0f);
+            on = make_float4(d[3] * len, d[4] * len, d[5] * len, 0.0f);
         }
     } else {
-        dp[i] = make_float4(d[0], d[1], d[2], 0.0f);
-        if (dn) dn[i] = make_float4(d[3], d[4], d[5], 0.0f);
+        op = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (NRM) on = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+}
+// Levels 1 .. L-1 of a cloud from a workgroup's 16 x 16 tile of level 0 (256
+// threads, the tile's records in the first 256 entries of lp, ln): each level
+// is formed from the one before in LDS and stored, so a level is neither read
+// back nor a launch of its own. The sizes are multiples of 2^(L-1), so a pixel
+// of a level has its four taps inside the tile. (64 bi-objective pairs of
+// 320x240, both clouds: 183 us as a launch per level, 100 us as one.)
+constexpr int CLOUD_TILE = 256 + 64 + 16 + 4;
+template <bool NRM>
+__device__ __forceinline__ void cloud_tile_levels(float4* lp, float4* ln, int bx, int by, int W, int H, int L,
+                                                  float4* const* dp, float4* const* dn) {
+    const int t = threadIdx.x;
+    int src = 0, dst = 256;
+    for (int l = 1; l < L; l++) {
+        __syncthreads();
+        const int side = 16 >> l;
+        if (t < side * side) {
+            const int x = t & (side - 1), y = t / side, o = src + 2 * x + 4 * y * side;
+            const int at[4] = {o, o + 1, o + 2 * side, o + 2 * side + 1};
+            float4 p[4], q[4], op, on;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                p[k] = lp[at[k]];
+                if (NRM) q[k] = ln[at[k]];
+            }
+            cloud_mean<NRM>(p, q, op, on);
+            lp[dst + t] = op;
+            if (NRM) ln[dst + t] = on;
+            const int gx = bx * side + x, gy = by * side + y;
+            if (gx < (W >> l) && gy < (H >> l)) {
+                stg(dp[l], (size_t)gx + (size_t)gy * (W >> l), op);
+                if (NRM) stg(dn[l], (size_t)gx + (size_t)gy * (W >> l), on);
+            }
+        }
+        src = dst;
+        dst += side * side;
     }
 }
 // icpResidualKernel2 (rgb2gray.cu:223-260) for keyframe pixel o of a w x h
@@ -858,20 +896,22 @@ __device__ __forceinline__ void cloud_down_pixel(const float4* __restrict__ sp, 
 __device__ __forceinline__ bool icp_mask_pixel(const float4* __restrict__ rp, const float4* __restrict__ rn,
                                                const float4* __restrict__ cp, int w, int h, int o, const float* T,
                                                const float* c, float a, float b, float& r) {
-    float4 p = rp[o];
+    float4 p = ldo(rp, o), nn = ldo(rn, o);
     if (p.w == 0.0f) return false;
-    float4 nn = rn[o];
     f3 p3{p.x, p.y, p.z}, n3{nn.x, nn.y, nn.z};
     f3 q3 = mul4(T, p3);
     f3 cn = rot4(T, n3);
     const float* K = c + KL;
-    float qx = q3.x / q3.z, qy = q3.y / q3.z;
+    // the quotients as div_rn (a zero or non-finite z gives NaN where the
+    // division gives an infinity, which the bounds reject alike)
+    const float iz = 1.0f / q3.z;
+    float qx = div_rn(q3.x, q3.z, iz), qy = div_rn(q3.y, q3.z, iz);
     float px = a * (K[0] * qx + K[2]) + b;
     float py = a * (K[4] * qy + K[5]) + b;
     if (!(px >= 0.0f && px < (float)(w - 1) && py >= 0.0f && py < (float)(h - 1))) return false;
     int xdi = (int)px, ydi = (int)py;
     int o2 = xdi + ydi * w;
-    float4 c0 = cp[o2], c1 = cp[o2 + 1], c2 = cp[o2 + w], c3 = cp[o2 + w + 1];
+    float4 c0 = ldo(cp, o2), c1 = ldo(cp, o2 + 1), c2 = ldo(cp, o2 + w), c3 = ldo(cp, o2 + w + 1);
     if (!(c0.w != 0.0f && c1.w != 0.0f && c2.w != 0.0f && c3.w != 0.0f)) return false;
     float fx = px - (float)xdi, fy = py - (float)ydi;
     f3 cc{blend(c0.x, c1.x, c2.x, c3.x, fx, fy), blend(c0.y, c1.y, c2.y, c3.y, fx, fy),
@@ -880,53 +920,116 @@ __device__ __forceinline__ bool icp_mask_pixel(const float4* __restrict__ rp, co
     r = dd.x * cn.x + dd.y * cn.y + dd.z * cn.z;
     return true;
 }
-// icpResidualIndexKernel2 (rgb2gray.cu:323-390) for keyframe pixel o with its
-// squared mask residual x2, the final Student-t weight (clamped to 1) from the
-// variance sum v3 over n points: scaled residual and the 6 Jacobian entries
-// (zeros when the point leaves the view, its first tap is invalid, the weight
-// vanishes or |dz| >= 300 mm).
-__device__ __forceinline__ void icp_point_terms(const float4* __restrict__ rp, const float4* __restrict__ rn,
-                                                const float4* __restrict__ cp, int w, int h, int o, float x2, float v3,
-                                                int n, const float* T, const float* c, float a, float b, float s,
-                                                float& res, float* J) {
-    float4 p = rp[o], nn = rn[o];
+// The Student-t weight 6 / (5 + x2 / var) with var = v3 / n, the variance of
+// the third round: the same for every point of a level, so its quotient runs
+// as div_rn where no intermediate can over- or underflow.
+struct IcpWeight { float var, inv; bool plain; };
+__device__ __forceinline__ IcpWeight icp_weight(float v3, int n) {
+    IcpWeight w;
+    w.var = v3 / (float)n;
+    w.inv = 1.0f / w.var;
+    w.plain = w.var > 1e-12f && w.var < 1e24f;
+    return w;
+}
+// icpResidualIndexKernel2 (rgb2gray.cu:323-390) for the keyframe point p with
+// normal nn and squared mask residual x2, weighted by the final Student-t
+// weight (clamped to 1): scaled residual and the 6 Jacobian entries (zeros when
+// the point leaves the view, its first tap is invalid, the weight vanishes or
+// |dz| >= 300 mm). The rotated generators leave out the products with their
+// zeros and ones, which are exact, and the quotients share their reciprocals
+// (div_rn): 370 vector instructions a point with its loads, 470 before.
+__device__ __forceinline__ void icp_point_terms(float4 p, float4 nn, const float4* __restrict__ cp, int w, int h,
+                                                float x2, IcpWeight iw, const float* T, const float* c, float a,
+                                                float b, float s, float& res, float* J) {
     f3 p3{p.x, p.y, p.z}, rnv{nn.x, nn.y, nn.z};
     f3 q3 = mul4(T, p3);
     f3 cn = rot4(T, rnv);
     const float* K = c + KL;
-    float qx = q3.x / q3.z, qy = q3.y / q3.z;
+    const float iz = 1.0f / q3.z;
+    float qx = div_rn(q3.x, q3.z, iz), qy = div_rn(q3.y, q3.z, iz);
     float px = a * (K[0] * qx + K[2]) + b;
     float py = a * (K[4] * qy + K[5]) + b;
     res = 0.0f;
 #pragma unroll
     for (int k = 0; k < 6; k++) J[k] = 0.0f;
     if (px >= 0.0f && px < (float)(w - 1) && py >= 0.0f && py < (float)(h - 1)) {
-        float wt = fminf(6 / (5 + x2 / (v3 / (float)n)), 1.0f);
+        const float t2 = iw.plain ? div_rn(x2, iw.var, iw.inv) : x2 / iw.var;
+        float wt = fminf(6 / (5 + t2), 1.0f);
         int xdi = (int)px, ydi = (int)py;
         float fx = px - (float)xdi, fy = py - (float)ydi;
         int o2 = xdi + ydi * w;
-        float4 c0 = cp[o2], c1 = cp[o2 + 1], c2 = cp[o2 + w], c3 = cp[o2 + w + 1];
+        float4 c0 = ldo(cp, o2), c1 = ldo(cp, o2 + 1), c2 = ldo(cp, o2 + w), c3 = ldo(cp, o2 + w + 1);
         f3 cc{blend(c0.x, c1.x, c2.x, c3.x, fx, fy), blend(c0.y, c1.y, c2.y, c3.y, fx, fy),
               blend(c0.z, c1.z, c2.z, c3.z, fx, fy)};
         if (c0.w != 0.0f && wt > 0.0f && fabsf(cc.z - q3.z) < 300.0f) {
             f3 d{cc.x - q3.x, cc.y - q3.y, cc.z - q3.z};
             res = s * wt * (d.x * cn.x + d.y * cn.y + d.z * cn.z);
-            f3 gp[3] = {{0.0f, -p3.z, p3.y}, {p3.z, 0.0f, -p3.x}, {-p3.y, p3.x, 0.0f}};
-            f3 gn[3] = {{0.0f, -rnv.z, rnv.y}, {rnv.z, 0.0f, -rnv.x}, {-rnv.y, rnv.x, 0.0f}};
+            // the rotation generators applied to p3 and the normal, rotated by T:
+            // (0, -z, y), (z, 0, -x), (-y, x, 0)
 #pragma unroll
             for (int k = 0; k < 3; k++) {
-                f3 dB = rot4(T, gp[k]);
-                f3 dN = rot4(T, gn[k]);
+                const int i0 = k == 0 ? 1 : 0, i1 = k == 2 ? 1 : 2;  // the generator's nonzero entries
+                const float u0 = k == 0 ? -p3.z : (k == 1 ? p3.z : -p3.y), u1 = k == 0 ? p3.y : (k == 1 ? -p3.x : p3.x);
+                const float v0 = k == 0 ? -rnv.z : (k == 1 ? rnv.z : -rnv.y),
+                            v1 = k == 0 ? rnv.y : (k == 1 ? -rnv.x : rnv.x);
+                f3 dB{T[i0] * u0 + T[i1] * u1, T[4 + i0] * u0 + T[4 + i1] * u1, T[8 + i0] * u0 + T[8 + i1] * u1};
+                f3 dN{T[i0] * v0 + T[i1] * v1, T[4 + i0] * v0 + T[4 + i1] * v1, T[8 + i0] * v0 + T[8 + i1] * v1};
                 J[k] = -s * wt * (-cn.x * dB.x - cn.y * dB.y - cn.z * dB.z + d.x * dN.x + d.y * dN.y + d.z * dN.z);
             }
-            f3 e[3] = {{1.0f, 0.0f, 0.0f}, {0.0f, 1.0f, 0.0f}, {0.0f, 0.0f, 1.0f}};
+            // the translation generators: T's columns
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                f3 dB = rot4(T, e[k]);
-                J[3 + k] = -wt * (-cn.x * dB.x - cn.y * dB.y - cn.z * dB.z);
-            }
+            for (int k = 0; k < 3; k++) J[3 + k] = -wt * (-cn.x * T[k] - cn.y * T[4 + k] - cn.z * T[8 + k]);
         }
     }
+}
+
+// ------------------------------------------------------------------ Student-t sums by one wave
+// generateStudentTWeights' 1024-wide tree (rgb2gray.cu:470-568, 854-877) by one
+// wave: lane l holds elements l, l + 64, ..., l + 960, so the tree's steps 512
+// to 64 add within a lane and the rest across lanes: the same sums as the
+// reference's workgroup tree, without its ten barriers.
+__device__ __forceinline__ float wave_tree1024(float* v) {
+#pragma unroll
+    for (int s = 8; s >= 1; s >>= 1)
+#pragma unroll
+        for (int k = 0; k < s; k++) v[k] += v[k + s];
+    float r = v[0];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) r += __shfl_down(r, o, 64);
+    return __shfl(r, 0, 64);
+}
+// The variance sum from nb <= 1024 block sums of n points (the reference's
+// last-block combination): int truncation per block sum, clamped to at least n
+// with more than one block.
+__device__ __forceinline__ float wave_student_total(const float* __restrict__ bsum, int nb, int n) {
+    if (nb == 1) return bsum[0];
+    const int lane = lane_id();
+    float v[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) v[k] = bsum[min(lane + 64 * k, nb - 1)];  // all loads in flight together
+#pragma unroll
+    for (int k = 0; k < 16; k++) v[k] = lane + 64 * k < nb ? (float)(int)v[k] : 0.0f;
+    const float r = wave_tree1024(v), mn = (float)n;
+    return r < mn ? mn : r;
+}
+// The sum of block bk (1024 of the n points) in a round: weights from the
+// previous round's variance sum prev, products truncated to int per point.
+__device__ __forceinline__ float wave_student_block(const float* __restrict__ r2, int bk, int n, int round, float prev) {
+    const int lane = lane_id();
+    float v[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) v[k] = r2[min(bk * 1024 + lane + 64 * k, n - 1)];  // all loads in flight together
+    // x / 100 in the first round, then x / (prev / n)
+    IcpWeight iw = icp_weight(prev, n);
+    if (round == 1) iw = IcpWeight{100.0f, 1.0f / 100.0f, true};
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        const float x = v[k];
+        const float w = 6 / (5 + (iw.plain ? div_rn(x, iw.var, iw.inv) : x / iw.var));
+        const int sum = x * w;
+        v[k] = bk * 1024 + lane + 64 * k < n ? (float)sum : 0.0f;
+    }
+    return wave_tree1024(v);
 }
 
 }  // namespace rt

@@ -152,6 +152,36 @@ def test_batch_kernel_variants_agree(N, iters, monkeypatch, capfd):
         assert (1, True) in kinds and (1, False) in kinds
 
 
+@pytest.mark.parametrize("N,iters,robust,bins", [(256, (1, 3, 10, 5), 0, 64), (2048, (2, 0, 3, 1), 1, 256),
+                                                 (8192, (1, 3, 10, 5), 0, 64), (8448, (0, 1, 0, 2), 0, 64),
+                                                 (16640, (1, 1, 1, 1), 0, 64), (2048, (0, 0, 0, 0), 0, 64)])
+def test_lockstep_equals_the_persistent_kernel(N, iters, robust, bins, monkeypatch):
+    """Small batches track in lockstep launches, whose sums are those of a
+    1024-thread workgroup of the persistent kernel: the same poses and RMS bit
+    for bit, with points below, at and past a round's 8192 and levels or whole
+    schedules without iterations."""
+    import ctypes
+    from recon_amd import lib
+    print(f"case lockstep N {N} iters {iters}", flush=True)
+    pairs, host, _ = _batch(7, theta=2.0, tmax=30.0, seed=90, rig=True)
+    pairs = [p for p in pairs if p["width"] * p["height"] >= 2 * N]
+    info, v = (ctypes.c_int * 6)(), 0
+    while lib().rt_batch_variant_info(v, info) == 0 and not (info[0] == 1024 and not info[2] and 1024 * info[1] >= N):
+        v += 1
+    res = {}
+    for force in (None, v):
+        monkeypatch.delenv("RT_BATCH_VARIANT", raising=False)
+        if force is not None:
+            monkeypatch.setenv("RT_BATCH_VARIANT", str(force))
+        bt = BatchTracker(len(pairs), 640, 480, mode=PHOTOMETRIC, n_select=N, iters=iters, robust=robust, mad_bins=bins)
+        a = bt.track(pairs)
+        b = bt.retrack(init=a[0].reshape(-1, 16), n=len(pairs))  # a second launch, other start poses
+        bt.close()
+        res[force] = a + b
+    for x, y in zip(res[None], res[v]):
+        assert np.array_equal(x, y)
+
+
 def test_depth_blocks_are_the_current_depth_map():
     """The tracker's depth taps read kb_pyramid's copy of the current depth
     map in 8x8-pixel blocks: every pixel (x, y) must hold the input's value at
