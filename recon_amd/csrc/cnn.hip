@@ -320,7 +320,13 @@ __global__ __launch_bounds__(256) void k_conv_fwd_mfma(ConvGeom g, const bf16* _
 // to the other buffer after them, one barrier per step. Waves (WGM x 4/WGM)
 // take 16*TM x 16*TN sub-tiles with v_mfma_f32_16x16x32_bf16; the epilogue is
 // the one of k_conv_fwd_mfma.
-template <int BM, int BN, int WGM, int KS = 32>
+// D: stages whose loads are in flight in registers ahead of the one in LDS (the
+// step count is a multiple of D). A layer of few rows has one or two
+// workgroups per CU and waits on each stage's loads: with D = 3 they have two
+// stages' time to arrive (64 samples, layers 3-6: 89 us with D = 1, DEEPUS us;
+// one sample: 66 and DEEP1US us). Full layers hide them with D = 1.
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+template <int BM, int BN, int WGM, int KS = 32, int D = 1>
 __global__ __launch_bounds__(256) void k_conv_fwd_lds32(ConvGeom g, const bf16* __restrict__ X,
                                                         const bf16* __restrict__ Wp, const float* __restrict__ bias,
                                                         bf16* __restrict__ Y) {
@@ -336,58 +342,68 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds32(ConvGeom g, const bf16* 
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, r16 = lane & 15, kg = lane >> 4;
     const int M = g.B * g.Ho * g.Wo, HW = g.Ho * g.Wo;
     const int bm0 = blockIdx.x * BM, bn0 = blockIdx.y * BN;
-    int arow[AQ], apart[AQ], ayb[AQ], axb[AQ];
-    size_t anb[AQ];
-    bool av[AQ], ae[AQ];
+    // Loads without branches, so that the compiler lets them stay in flight over
+    // the MFMAs and barriers: a tap in the padding (bit `tap` of ok clear) reads
+    // the row's centre pixel instead, which always exists, and is zeroed on its
+    // way to LDS; the stages past the last repeat it.
+    constexpr bool AF = AC % 256 == 0, BF = BC % 256 == 0;  // every thread loads every chunk
+    static_assert(D == 1 || D == 3, "one or three stages");
+    static_assert(BF, "weight chunks tile the threads");
+    int arow[AQ], apart[AQ];
+    const bf16* ap[AQ];  // the row's centre pixel, at the chunk's channels
+    unsigned ok[AQ];
 #pragma unroll
     for (int q = 0; q < AQ; q++) {
         const int e = t + 256 * q;
-        ae[q] = e < AC;
         arow[q] = (e / CR) % BM;
         apart[q] = e % CR;
         const int m = bm0 + arow[q];
-        av[q] = ae[q] && m < M;
-        const int mm = av[q] ? m : 0;
+        const bool v = (AF || e < AC) && m < M;
+        const int mm = v ? m : 0;
         const int n = mm / HW, r = mm - n * HW, yo = r / g.Wo, xo = r - yo * g.Wo;
-        ayb[q] = 2 * yo - 1;
-        axb[q] = 2 * xo - 1;
-        anb[q] = (size_t)n * g.Hi * g.Wi;
+        ap[q] = X + (((size_t)n * g.Hi + 2 * yo) * g.Wi + 2 * xo) * g.Ci + 8 * apart[q];
+        ok[q] = 0u;
+#pragma unroll
+        for (int tap = 0; tap < 9; tap++) {
+            const int yi = 2 * yo - 1 + tap / 3, xi = 2 * xo - 1 + tap % 3;
+            ok[q] |= (v && yi >= 0 && yi < g.Hi && xi >= 0 && xi < g.Wi) ? 1u << tap : 0u;
+        }
     }
-    int brow[BQ], bpart[BQ];
-    bool be[BQ];
     const bf16* bp[BQ];
 #pragma unroll
     for (int q = 0; q < BQ; q++) {
         const int e = t + 256 * q;
-        be[q] = e < BC;
-        brow[q] = (e / CR) % BN;
-        bpart[q] = e % CR;
-        bp[q] = Wp + (size_t)(bn0 + brow[q]) * g.Kp + 8 * bpart[q];
+        bp[q] = Wp + (size_t)(bn0 + e / CR) * g.Kp + 8 * (e % CR);
     }
-    uint4 ra[AQ], rb[BQ];
-    auto gload = [&](int s) {
-        const int k = KS * s;
+    struct Regs {
+        u4 a[AQ], b[BQ];
+        unsigned z[AQ];  // all ones, or zero for a tap in the padding
+    };
+    const int steps = g.Kp / KS;
+    auto gload = [&](int s, Regs& r) {
+        const int k = KS * min(s, steps - 1);
         const int tap = k >> g.ci_shift, ci0 = k & (g.Ci - 1);
-        const int ky = tap / 3, kx = tap - 3 * (tap / 3);
+        const int toff = ((tap / 3 - 1) * g.Wi + tap % 3 - 1) * g.Ci;
 #pragma unroll
         for (int q = 0; q < AQ; q++) {
-            const int yi = ayb[q] + ky, xi = axb[q] + kx;
-            const bool ok = av[q] && yi >= 0 && yi < g.Hi && xi >= 0 && xi < g.Wi;
-            ra[q] = ok ? *(const uint4*)(X + (anb[q] + (size_t)yi * g.Wi + xi) * g.Ci + ci0 + 8 * apart[q])
-                       : make_uint4(0u, 0u, 0u, 0u);
+            r.z[q] = 0u - ((ok[q] >> tap) & 1u);
+            r.a[q] = *(const u4*)(ap[q] + (ci0 + (toff & (int)r.z[q])));
         }
 #pragma unroll
-        for (int q = 0; q < BQ; q++) rb[q] = be[q] ? *(const uint4*)(bp[q] + k) : make_uint4(0u, 0u, 0u, 0u);
+        for (int q = 0; q < BQ; q++) r.b[q] = *(const u4*)(bp[q] + k);
     };
-    auto sstore = [&](int buf) {
+    auto sstore = [&](int buf, const Regs& r) {
         bf16* A = lds + buf * STAGE;
         bf16* Bs = A + BM * LD;
 #pragma unroll
-        for (int q = 0; q < AQ; q++)
-            if (ae[q]) *(uint4*)(A + arow[q] * LD + 8 * apart[q]) = ra[q];
+        for (int q = 0; q < AQ; q++) {
+            if (AF || t + 256 * q < AC) *(u4*)(A + arow[q] * LD + 8 * apart[q]) = r.a[q] & r.z[q];
+        }
 #pragma unroll
-        for (int q = 0; q < BQ; q++)
-            if (be[q]) *(uint4*)(Bs + brow[q] * LD + 8 * bpart[q]) = rb[q];
+        for (int q = 0; q < BQ; q++) {
+            const int e = t + 256 * q;
+            *(u4*)(Bs + (e / CR) * LD + 8 * (e % CR)) = r.b[q];
+        }
     };
     const int wm0 = (w % WGM) * WM, wn0 = (w / WGM) * WN;
     f4 acc[TM][TN];
@@ -395,13 +411,9 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds32(ConvGeom g, const bf16* 
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-    const int steps = g.Kp / KS;
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    for (int s = 0; s < steps; s++) {
+    auto step = [&](int s, Regs& load, const Regs& store) {
         const int cur = s & 1;
-        if (s + 1 < steps) gload(s + 1);
+        gload(s + D, load);  // stage s went to LDS a step ago
         const bf16* A = lds + cur * STAGE;
         const bf16* Bs = A + BM * LD;
 #pragma unroll
@@ -416,8 +428,25 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds32(ConvGeom g, const bf16* 
 #pragma unroll
                 for (int j = 0; j < TN; j++) acc[i][j] = mfma32(a[i], b[j], acc[i][j]);
         }
-        if (s + 1 < steps) sstore(cur ^ 1);
+        sstore(cur ^ 1, store);  // after the last step: nothing reads it
         __syncthreads();
+    };
+    Regs r0, r1, r2;
+    gload(0, r0);
+    if constexpr (D == 3) {
+        gload(1, r1);
+        gload(2, r2);
+    }
+    sstore(0, r0);
+    __syncthreads();
+    if constexpr (D == 3) {
+        for (int s = 0; s < steps; s += 3) {
+            step(s, r0, r1);
+            step(s + 1, r1, r2);
+            step(s + 2, r2, r0);
+        }
+    } else {
+        for (int s = 0; s < steps; s++) step(s, r0, r0);
     }
     bf16* T = lds;
 #pragma unroll
@@ -1395,7 +1424,7 @@ static bool forward_mfma(const ConvGeom& g, const bf16* X, const bf16* Wp, const
             if (blocks(128, 128) >= 512) k_conv_fwd_lds32<128, 128, 2><<<dim3((M + 127) / 128, gy), 256, 0, s>>>(g, X, Wp, bias, Y);
             else if (blocks(64, 128) >= 512) k_conv_fwd_lds32<64, 128, 2><<<dim3((M + 63) / 64, gy), 256, 0, s>>>(g, X, Wp, bias, Y);
             else if (g.Ci % 64 == 0)  // few rows and a long k: stages of 64 halve its barriers and load round trips
-                k_conv_fwd_lds32<32, 128, 2, 64><<<dim3((M + 31) / 32, gy), 256, 0, s>>>(g, X, Wp, bias, Y);
+                k_conv_fwd_lds32<32, 128, 2, 64, 3><<<dim3((M + 31) / 32, gy), 256, 0, s>>>(g, X, Wp, bias, Y);
             else k_conv_fwd_lds32<32, 128, 2><<<dim3((M + 31) / 32, gy), 256, 0, s>>>(g, X, Wp, bias, Y);
             return true;
         }

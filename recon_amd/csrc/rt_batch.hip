@@ -403,26 +403,6 @@ __device__ __forceinline__ unsigned bytes_ge(unsigned w, unsigned U) {
     const unsigned d = (w | 0x80808080u) - (U & 0x7F7F7F7Fu);
     return ((w & ~U) | (~(w ^ U) & d)) & 0x80808080u;
 }
-// inclusive sum over the lanes of a wave
-__device__ __forceinline__ int wave_scan_incl(int v) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int u = __shfl_up(v, o, 64);
-        if (lane >= o) v += u;
-    }
-    return v;
-}
-// inclusive maximum over the lanes of a wave
-__device__ __forceinline__ int wave_scan_max(int v) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int u = __shfl_up(v, o, 64);
-        if (lane >= o) v = max(v, u);
-    }
-    return v;
-}
 __device__ __forceinline__ int wave_isum(int v) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -450,23 +430,12 @@ __device__ __forceinline__ SelFlags sel_flags(Bins8 w, int nv, unsigned T, unsig
     f.ehi = bytes_eq(w.hi, T) & vhi;
     return f;
 }
-__global__ __launch_bounds__(SEL_BS, RT_SEL_WPE) void kb_select(const PairDesc* __restrict__ P) {
-    const PairDesc& d = P[blockIdx.x];
-    __shared__ int cA[512], cE[512], sA[512], sE[512], pm[512];
-    __shared__ int wtot[3][8];
-    __shared__ int s_first;
-    int thr_i, excess;
-    find_threshold(d.ghist, d.N, thr_i, excess);
-    const unsigned T = (unsigned)thr_i * 0x01010101u;
-    const bool any_above = thr_i < 255;                      // no bin lies above 255
-    const unsigned U = (unsigned)(thr_i + 1) * 0x01010101u;  // "above" = ">= thr + 1"
-    const int t = threadIdx.x, wave = t >> 6, lane = lane_id();
-    const int npix = d.W * d.H, Pn = npix / 512, N = d.N;
-    const bool vec = (Pn & 7) == 0;
-    const RT_GLOBAL uint8_t* bins = gmem(d.bins);
-    if (t == 0) s_first = 512;
-    // pass 1: counts
-    for (int s0 = wave; s0 < 512; s0 += SEL_WAVES * SEL_U) {
+// the counts of the segments s0 = first + wave, ... below last, packed, to out(s, packed)
+template <class F>
+__device__ __forceinline__ void count_segments(const RT_GLOBAL uint8_t* bins, int Pn, bool vec, unsigned T, unsigned U,
+                                               bool any_above, int first, int last, const F& out) {
+    const int wave = threadIdx.x >> 6, lane = lane_id();
+    for (int s0 = first + wave; s0 < last; s0 += SEL_WAVES * SEL_U) {
         int ae[SEL_U];
 #pragma unroll
         for (int u = 0; u < SEL_U; u++) ae[u] = 0;
@@ -482,37 +451,57 @@ __global__ __launch_bounds__(SEL_BS, RT_SEL_WPE) void kb_select(const PairDesc* 
 #pragma unroll
         for (int u = 0; u < SEL_U; u++) {
             int v = wave_isum(ae[u]);
-            if (lane == 0) { cA[s0 + u * SEL_WAVES] = v & 0xffff; cE[s0 + u * SEL_WAVES] = v >> 16; }
+            if (lane == 0) out(s0 + u * SEL_WAVES, v);
         }
     }
-    __syncthreads();
-    // Trim of the equal counts (filterIndex256.cu:141-152). Sequentially, over
-    // segments j = 0..510 with a positive equal count m_j and a running excess
-    // T (initially the excess): if m_j >= T the segment loses T and the trim
-    // ends; otherwise the segment is emptied and T becomes m_j (the
-    // reference's update T += m_j - T). In parallel: T before j is the count
-    // of the previous non-empty segment (or the excess), the trim ends at the
-    // first non-empty j with m_j >= T, every non-empty segment before it is
-    // emptied; the last segment is never trimmed.
-    int m = 0, prevval = 0;
-    bool nz = false;
-    if (t < 512) {
-        m = cE[t];
-        nz = t < 511 && m > 0;
-        int v = wave_scan_max(nz ? t : -1);
-        if (lane == 63) wtot[0][wave] = v;
-        pm[t] = v;
+}
+// A batch of few pairs spreads a pair over `parts` workgroups (a power of two
+// up to 16, gridDim.x; SPLIT): kb_select_count leaves the segments' packed
+// counts in the pair's point array, which kb_ref_points fills later, and each
+// workgroup of kb_select repeats the trim and the offsets and scatters its own
+// segments. One pair per workgroup left most CUs idle: 64 pairs of 640x480 147
+// us, split over 16 workgroups SELUS us; 256 mixed pairs 147 and SELUM us.
+static int select_parts(int n) {
+    int parts = 1;
+    while (parts < 16 && 2 * parts * n <= 2048) parts *= 2;
+    return parts;
+}
+__global__ __launch_bounds__(SEL_BS, RT_SEL_WPE) void kb_select_count(const PairDesc* __restrict__ P) {
+    const PairDesc& d = P[blockIdx.y];
+    int thr_i, excess;
+    find_threshold(d.ghist, d.N, thr_i, excess);
+    const int Pn = d.W * d.H / 512, per = 512 / gridDim.x;
+    RT_GLOBAL int* counts = (RT_GLOBAL int*)gmem(d.pts);
+    count_segments(gmem(d.bins), Pn, (Pn & 7) == 0, (unsigned)thr_i * 0x01010101u, (unsigned)(thr_i + 1) * 0x01010101u,
+                   thr_i < 255, per * blockIdx.x, per * (blockIdx.x + 1), [&](int s, int v) { counts[s] = v; });
+}
+template <bool SPLIT>
+__global__ __launch_bounds__(SEL_BS, RT_SEL_WPE) void kb_select(const PairDesc* __restrict__ P) {
+    const PairDesc& d = P[SPLIT ? blockIdx.y : blockIdx.x];
+    __shared__ int cA[512], cE[512], sA[512], sE[512], pm[512];
+    __shared__ int wtot[3][8];
+    __shared__ int s_first;
+    int thr_i, excess;
+    find_threshold(d.ghist, d.N, thr_i, excess);
+    const unsigned T = (unsigned)thr_i * 0x01010101u;
+    const bool any_above = thr_i < 255;                      // no bin lies above 255
+    const unsigned U = (unsigned)(thr_i + 1) * 0x01010101u;  // "above" = ">= thr + 1"
+    const int t = threadIdx.x, wave = t >> 6, lane = lane_id();
+    const int npix = d.W * d.H, Pn = npix / 512, N = d.N;
+    const bool vec = (Pn & 7) == 0;
+    const RT_GLOBAL uint8_t* bins = gmem(d.bins);
+    // pass 1: counts
+    if constexpr (SPLIT) {
+        if (t < 512) {
+            const int v = ((const RT_GLOBAL int*)gmem(d.pts))[t];
+            cA[t] = v & 0xffff;
+            cE[t] = v >> 16;
+        }
+    } else {
+        count_segments(bins, Pn, vec, T, U, any_above, 0, 512, [&](int s, int v) { cA[s] = v & 0xffff; cE[s] = v >> 16; });
     }
     __syncthreads();
-    if (t < 512) {
-        int prev = -1;
-        for (int w = 0; w < wave; w++) prev = max(prev, wtot[0][w]);
-        if (t > 0) prev = max(prev, (t - 1) >> 6 == wave ? pm[t - 1] : -1);
-        prevval = prev >= 0 ? cE[prev] : excess;
-        if (excess > 0 && nz && m >= prevval) atomicMin(&s_first, t);
-    }
-    __syncthreads();
-    if (t < 512 && excess > 0 && nz && t <= s_first) m = t < s_first ? 0 : m - prevval;
+    const int m = trim_equal(cE, excess, wtot[0], pm, &s_first);
     // exclusive offsets: above-threshold indices first, then the kept equal ones
     int ia = 0, ie = 0;
     if (t < 512) {
@@ -537,7 +526,8 @@ __global__ __launch_bounds__(SEL_BS, RT_SEL_WPE) void kb_select(const PairDesc* 
     // pass 2: ordered scatter; a lane's hits are ranked by a wave scan of the
     // packed counts, then written in pixel order (bit 8j+7 is pixel j)
     RT_GLOBAL int* sel = gmem(d.sel);
-    for (int s0 = wave; s0 < 512; s0 += SEL_WAVES * SEL_U) {
+    const int per = SPLIT ? 512 / (int)gridDim.x : 512, first = SPLIT ? per * (int)blockIdx.x : 0;
+    for (int s0 = first + wave; s0 < first + per; s0 += SEL_WAVES * SEL_U) {
         int run[SEL_U];
 #pragma unroll
         for (int u = 0; u < SEL_U; u++) run[u] = 0;
@@ -569,6 +559,7 @@ __global__ __launch_bounds__(SEL_BS, RT_SEL_WPE) void kb_select(const PairDesc* 
         }
     }
     // a short selection leaves zeros behind the selected indices
+    if (first > 0) return;
     for (int k = (total > 0 ? total : 0) + t; k < N; k += SEL_BS) sel[k] = 0;
 }
 // XCD-aware: workgroup b runs on XCD b % 8 (dispatch is round-robin), and
@@ -1464,7 +1455,13 @@ static void launch_prep(const BatchView& v, hipStream_t s, int part = 0) {
         kb_bins<<<gb, 256, 0, s>>>(v.desc);
     }
     if (part == 2) return;
-    kb_select<<<n, SEL_BS, 0, s>>>(v.desc);
+    const int parts = select_parts(n);
+    if (parts > 1) {
+        kb_select_count<<<dim3(parts, n), SEL_BS, 0, s>>>(v.desc);
+        kb_select<true><<<dim3(parts, n), SEL_BS, 0, s>>>(v.desc);
+    } else {
+        kb_select<false><<<n, SEL_BS, 0, s>>>(v.desc);
+    }
     const int chunks = (v.maxN + 255) / 256;
     kb_ref_points<<<8 * ((n + 7) / 8) * chunks, 256, 0, s>>>(v.desc, n, chunks);
     if (v.mode != RT_PHOTOMETRIC) {

@@ -149,38 +149,82 @@ __device__ __forceinline__ void select_count_block(int s, const float* __restric
     }
 }
 
-// pass 2 (one workgroup of 512): segment start offsets; the trim loop of
-// filterIndex256.cu:141-152 run as written.
+// inclusive sum over the lanes of a wave
+__device__ __forceinline__ int wave_scan_incl(int v) {
+    const int lane = lane_id();
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        int u = __shfl_up(v, o, 64);
+        if (lane >= o) v += u;
+    }
+    return v;
+}
+// inclusive maximum over the lanes of a wave
+__device__ __forceinline__ int wave_scan_max(int v) {
+    const int lane = lane_id();
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        int u = __shfl_up(v, o, 64);
+        if (lane >= o) v = max(v, u);
+    }
+    return v;
+}
+// Trim of the equal counts (filterIndex256.cu:141-152). Sequentially, over
+// segments j = 0..510 with a positive equal count m_j and a running excess T
+// (initially the excess): if m_j >= T the segment loses T and the trim ends;
+// otherwise the segment is emptied and T becomes m_j (the reference's update T
+// += m_j - T). In parallel: T before j is the count of the previous non-empty
+// segment (or the excess), the trim ends at the first non-empty j with m_j >=
+// T, every non-empty segment before it is emptied; the last segment is never
+// trimmed. A workgroup of at least 512 threads, cE visible to all of them;
+// returns thread t's kept count (t < 512), cE unchanged. wtot: 8 ints, pm: 512.
+// (The loop run by one thread took 12.7 us; TRIMUS us with the offsets here.)
+__device__ __forceinline__ int trim_equal(const int* cE, int excess, int* wtot, int* pm, int* s_first) {
+    const int t = threadIdx.x, wave = t >> 6, lane = lane_id();
+    int m = 0, prevval = 0;
+    bool nz = false;
+    if (t == 0) *s_first = 512;
+    if (t < 512) {
+        m = cE[t];
+        nz = t < 511 && m > 0;
+        const int v = wave_scan_max(nz ? t : -1);
+        if (lane == 63) wtot[wave] = v;
+        pm[t] = v;
+    }
+    __syncthreads();
+    if (t < 512) {
+        int prev = -1;
+        for (int w = 0; w < wave; w++) prev = max(prev, wtot[w]);
+        if (t > 0) prev = max(prev, (t - 1) >> 6 == wave ? pm[t - 1] : -1);
+        prevval = prev >= 0 ? cE[prev] : excess;
+        if (excess > 0 && nz && m >= prevval) atomicMin(s_first, t);
+    }
+    __syncthreads();
+    if (t < 512 && excess > 0 && nz && t <= *s_first) m = t < *s_first ? 0 : m - prevval;
+    return m;
+}
+
+// pass 2 (one workgroup of 512): the trim and the segment start offsets.
 __device__ __forceinline__ void select_scan_block(int* seg) {
-    __shared__ int a[512], m[512], sa[512], se[512];
-    int t = threadIdx.x;
-    a[t] = seg[t];
-    m[t] = seg[512 + t];
+    __shared__ int cE[512], pm[512], wt[3][8], s_first;
+    const int t = threadIdx.x, wave = t >> 6, lane = lane_id();
+    const int a = seg[t];
+    cE[t] = seg[512 + t];
     __syncthreads();
-    if (t == 0) {
-        int tooMuch = seg[2561];
-        for (int i = 1; i < 512; i++) {
-            if (tooMuch > 0 && m[i - 1] > 0) {
-                m[i - 1] -= tooMuch;
-                if (m[i - 1] < 0) { tooMuch += m[i - 1]; m[i - 1] = 0; }
-                else tooMuch = 0;
-            }
-        }
-    }
-    sa[t] = a[t];
-    se[t] = m[t];
+    const int m = trim_equal(cE, seg[2561], wt[0], pm, &s_first);
+    const int ia = wave_scan_incl(a), ie = wave_scan_incl(m);
+    if (lane == 63) { wt[1][wave] = ia; wt[2][wave] = ie; }
     __syncthreads();
-    for (int off = 1; off < 512; off <<= 1) {
-        int va = t >= off ? sa[t - off] : 0, ve = t >= off ? se[t - off] : 0;
-        __syncthreads();
-        sa[t] += va; se[t] += ve;
-        __syncthreads();
+    int oa = 0, oe = 0, ta = 0, te = 0;
+#pragma unroll
+    for (int w = 0; w < 8; w++) {
+        if (w < wave) { oa += wt[1][w]; oe += wt[2][w]; }
+        ta += wt[1][w]; te += wt[2][w];
     }
-    int totalA = sa[511];
-    seg[1024 + t] = sa[t] - a[t];
-    seg[1536 + t] = totalA + se[t] - m[t];
-    seg[2048 + t] = m[t];
-    if (t == 0) { seg[2562] = totalA; seg[2563] = totalA + se[511]; }
+    seg[1024 + t] = oa + ia - a;
+    seg[1536 + t] = ta + oe + ie - m;
+    seg[2048 + t] = m;
+    if (t == 0) { seg[2562] = ta; seg[2563] = ta + te; }
 }
 
 // pass 3: ordered scatter of each segment's above- and equal-bin indices.
