@@ -323,8 +323,8 @@ __global__ __launch_bounds__(256) void k_conv_fwd_mfma(ConvGeom g, const bf16* _
 // D: stages whose loads are in flight in registers ahead of the one in LDS (the
 // step count is a multiple of D). A layer of few rows has one or two
 // workgroups per CU and waits on each stage's loads: with D = 3 they have two
-// stages' time to arrive (64 samples, layers 3-6: 89 us with D = 1, DEEPUS us;
-// one sample: 66 and DEEP1US us). Full layers hide them with D = 1.
+// stages' time to arrive (64 samples, layers 3-6: 89 us with D = 1, 61 us;
+// one sample: 66 and 45 us). Full layers hide them with D = 1.
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 template <int BM, int BN, int WGM, int KS = 32, int D = 1>
 __global__ __launch_bounds__(256) void k_conv_fwd_lds32(ConvGeom g, const bf16* __restrict__ X,
@@ -473,136 +473,170 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds32(ConvGeom g, const bf16* 
     }
 }
 
-// The first two forward layers fused, one workgroup (8 waves) per pair: the
-// first layer (4 -> C1 channels, direct 8-byte tap loads as in
-// k_conv_fwd_mfma) writes its H1 x W1 x C1 output to LDS with bias, ReLU and
-// bfloat16 rounding; after a barrier the second layer (C1 = 32 -> C2) reads
-// its A operands from that LDS map (one 16-byte run per lane and tap) and its
-// weights from global memory. The intermediate never reaches HBM; the
-// second layer's tile leaves through LDS as 16-byte row chunks. Two
-// workgroups fit in a CU's LDS.
+// The first two forward layers fused: a workgroup of 8 waves per CU takes pairs
+// in turn; the first layer (4 -> C1 channels) writes its H1 x W1 x C1 output to
+// LDS with bias, ReLU and bfloat16 rounding, and the second layer (C1 = 32 ->
+// 64) reads its operands from that map, so the intermediate never reaches HBM.
+// There are two maps: while the second layer of a pair runs from one, the
+// inputs of the next pair are in flight, and its first layer fills the other;
+// one barrier a pair. The weights are the MFMA's row operand and the pixels
+// its columns, so that a lane holds four consecutive channels of a pixel: one
+// 8-byte store. A wave keeps the second layer's weights of 32 channels in
+// registers for all its pairs and takes every fourth row tile. The map's
+// 16-byte chunks are placed so that eight lanes that read every second pixel
+// fall on different banks (f12_slot). 4096 samples: 217 us with pixels as rows
+// (14 instructions a value to round and store), weights loaded per step and
+// the map in pixel order (8-way conflicts); 188 us here, of which the vector
+// instructions (addresses, rounding) fill 83 and the MFMAs 28; one sample 22 and
+// 15 us.
 constexpr int F12_C1 = 32;
 constexpr int F12_LDS = 30 * 40 * F12_C1;  // bf16 elements: the default network's first-layer map
-template <int C2>
-__global__ __launch_bounds__(512) void k_conv12_fused(ConvGeom g1, ConvGeom g2, const bf16* __restrict__ X,
-                                                      const bf16* __restrict__ W1, const float* __restrict__ b1,
-                                                      const bf16* __restrict__ W2, const float* __restrict__ b2,
-                                                      bf16* __restrict__ Y) {
-    constexpr int NW = 8, TN2 = C2 / 16, C2LD = C2 + 8;
-    __shared__ __attribute__((aligned(16))) bf16 map[F12_LDS];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, r16 = lane & 15, kg = lane >> 4;
-    const int pair = blockIdx.x;
+constexpr int F12_RT1 = 10;                // row tiles of 16 pixels per wave: first layer (80 tiles),
+constexpr int F12_RT2 = 5;                 // second layer (20 tiles, each by two waves)
+constexpr int F12_ZERO = 2 * F12_LDS;      // byte offset of 64 zero bytes behind the first map,
+constexpr int F12_MAP = F12_ZERO + 64;     // of the second map
+// byte offset of the 16-byte chunk c of pixel p in the map
+__device__ __forceinline__ int f12_slot(int p, int c) { return ((p ^ ((p >> 3) & 1)) << 6) + ((c ^ ((p >> 1) & 3)) << 4); }
+typedef unsigned u2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+// max(v + bias, 0) of four channels as bfloat16, round to nearest even (a NaN gives 0)
+__device__ __forceinline__ u2 relu4(f4 v, f4 bias) {
+    v = v + bias;
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = v[e] > 0.0f ? v[e] : 0.0f;
+    const b2 lo = {(__bf16)v[0], (__bf16)v[1]}, hi = {(__bf16)v[2], (__bf16)v[3]};
+    return u2{__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi)};
+}
+// v, of which the compiler knows nothing: addresses formed from it stay inside
+// the loop over pairs instead of filling registers across it
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+__global__ __launch_bounds__(512, 2) void k_conv12_fused(ConvGeom g1, ConvGeom g2, const bf16* __restrict__ X,
+                                                         const bf16* __restrict__ W1, const float* __restrict__ b1,
+                                                         const bf16* __restrict__ W2, const float* __restrict__ b2,
+                                                         bf16* __restrict__ Y) {
+    constexpr int NW = 8;
+    extern __shared__ __attribute__((aligned(16))) char lds12[];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), r16 = lane & 15, kg = lane >> 4;
     const int H1 = g1.Ho, Wd1 = g1.Wo, M1 = H1 * Wd1, H2 = g2.Ho, Wd2 = g2.Wo, M2 = H2 * Wd2;
-    const bf16* Xp = X + (size_t)pair * g1.Hi * g1.Wi * 4;
-    // ---- first layer: K = 36 in two steps of 32 (taps 8s + 2kg, 8s + 2kg + 1)
-    bf8 bw[2][2];
+    const float i1 = 1.0f / (float)Wd1, i2 = 1.0f / (float)Wd2;
+    if (t < 4) ((u4*)(lds12 + F12_ZERO))[t] = u4{0u, 0u, 0u, 0u};  // what a tap in the padding reads
+    // first layer: K = 36 in two steps of 32; lane group kg holds taps 2 kg and
+    // 2 kg + 1 of the first step, tap 8 in group 0 of the second
+    bf8 aw1[2][2];
+    f4 bias1[2], bias2[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            aw1[j][s] = __builtin_bit_cast(bf8, *(const u4*)(W1 + (size_t)(16 * j + r16) * g1.Kp + 32 * s + 8 * kg));
+        bias1[j] = *(const f4*)(b1 + 16 * j + 4 * kg);
+        bias2[j] = *(const f4*)(b2 + 32 * (w & 1) + 16 * j + 4 * kg);
+    }
+    int dy[3], dx[3], off[3];
+    unsigned hl[3];  // rows of the input for the tap: none for tap 8 outside group 0
+#pragma unroll
+    for (int h = 0; h < 3; h++) {
+        const int tap = h < 2 ? 2 * kg + h : 8;
+        dy[h] = tap / 3 - 1;
+        dx[h] = tap % 3 - 1;
+        off[h] = (dy[h] * g1.Wi + dx[h]) * 4;
+        hl[h] = h < 2 || kg == 0 ? (unsigned)g1.Hi : 0u;
+    }
+    // second layer: this wave's 32 channels, one tap of 32 channels per step
+    bf8 aw2[2][9];
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
-        for (int s = 0; s < 2; s++)
-            bw[j][s] = __builtin_bit_cast(bf8, *(const uint4*)(W1 + (size_t)(16 * j + r16) * g1.Kp + 32 * s + 8 * kg));
-    float bias1[2];
+        for (int s = 0; s < 9; s++)
+            aw2[j][s] = __builtin_bit_cast(
+                bf8, *(const u4*)(W2 + (size_t)(32 * (w & 1) + 16 * j + r16) * g2.Kp + 32 * s + 8 * kg));
+    const int RT2 = (M2 + 15) / 16;
+    // first layer of one pair: every tap of the wave's row tiles, without
+    // branches; a tap in the padding reads eight of the weights' zero padding
+    // bytes (k = 36 ..) instead, so no mask has to outlive its load
+    const bf16* zero = W1 + 40;
+    u2 v[F12_RT1][3];
+    auto load1 = [&](int pair) {
+        const bf16* Xp = X + (size_t)pair * g1.Hi * g1.Wi * 4;
+        const int r = opaque(r16);
 #pragma unroll
-    for (int j = 0; j < 2; j++) bias1[j] = b1[16 * j + r16];
-    const int RT1 = (M1 + 15) / 16;
-    constexpr int G1 = 4;  // row tiles whose loads are in flight together
-    for (int rt0 = w; rt0 < RT1; rt0 += G1 * NW) {
-        bf8 a[G1][2];
+        for (int u = 0; u < F12_RT1; u++) {
+            const int m = (w + NW * u) * 16 + r;
+            const int yo = (int)(((float)m + 0.5f) * i1), xo = m - yo * Wd1;  // yo >= H1 past the last pixel
+            const int base = (2 * yo * g1.Wi + 2 * xo) * 4;
 #pragma unroll
-        for (int u = 0; u < G1; u++) {
-            const int m = (rt0 + NW * u) * 16 + r16;
-            const bool mv = rt0 + NW * u < RT1 && m < M1;
-            const int yb = 2 * (m / Wd1) - 1, xb = 2 * (m % Wd1) - 1;
-#pragma unroll
-            for (int s = 0; s < 2; s++) {
-                uint2 v[2];
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const int tap = 8 * s + 2 * kg + h;
-                    const int yi = yb + tap / 3, xi = xb + tap % 3;
-                    const bool ok = mv && tap < 9 && yi >= 0 && yi < g1.Hi && xi >= 0 && xi < g1.Wi;
-                    v[h] = ok ? *(const uint2*)(Xp + ((size_t)yi * g1.Wi + xi) * 4) : make_uint2(0u, 0u);
-                }
-                a[u][s] = __builtin_bit_cast(bf8, make_uint4(v[0].x, v[0].y, v[1].x, v[1].y));
+            for (int h = 0; h < 3; h++) {
+                const int yi = 2 * yo + dy[h], xi = 2 * xo + dx[h];
+                const bool ok = ((unsigned)yi < hl[h]) & ((unsigned)xi < (unsigned)g1.Wi) & (yo < H1);
+                const bf16* q = Xp + (base + off[h]);
+                q = ok ? q : zero;
+                v[u][h] = *(const u2*)q;
             }
         }
+    };
+    auto layer1 = [&](char* map) {
+        const int r = opaque(r16);
 #pragma unroll
-        for (int u = 0; u < G1; u++) {
-            const int rt = rt0 + NW * u;
-            if (rt >= RT1) continue;
+        for (int u = 0; u < F12_RT1; u++) {
+            const int p = (w + NW * u) * 16 + r;
+            const bf8 x0 = __builtin_bit_cast(bf8, u4{v[u][0].x, v[u][0].y, v[u][1].x, v[u][1].y});
+            const bf8 x1 = __builtin_bit_cast(bf8, u4{v[u][2].x, v[u][2].y, 0u, 0u});
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-                acc = mfma32(a[u][0], bw[j][0], acc);
-                acc = mfma32(a[u][1], bw[j][1], acc);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int mr = rt * 16 + 4 * kg + e;
-                    const float v = acc[e] + bias1[j];
-                    if (mr < M1) map[mr * F12_C1 + 16 * j + r16] = f2bf(v > 0.0f ? v : 0.0f);
-                }
+                acc = mfma32(aw1[j][0], x0, acc);
+                acc = mfma32(aw1[j][1], x1, acc);
+                // channels 16 j + 4 kg .. + 3 of pixel p: half of chunk 2 j + kg / 2
+                if (p < M1) *(u2*)(map + f12_slot(p, 2 * j + (kg >> 1)) + 8 * (kg & 1)) = relu4(acc, bias1[j]);
             }
         }
-    }
+    };
+    load1(blockIdx.x);
+    layer1(lds12);
     __syncthreads();
-    // ---- second layer: K = 9 taps x 32 channels, one tap per step
-    const int RT2 = (M2 + 15) / 16;
-    constexpr int MAXRT = 3;  // row tiles per wave: the default network has 19 over 8 waves
-    f4 acc[MAXRT][TN2];
+    int cur = 0;
+    for (int pair = blockIdx.x; pair < g1.B; pair += gridDim.x, cur = F12_MAP - cur) {
+        const int next = pair + gridDim.x;
+        if (next < g1.B) load1(next);  // in flight over this pair's second layer
+        f4 acc[F12_RT2][2];
+        int p0[F12_RT2], okm[F12_RT2];  // the centre tap's pixel; bit s: tap s is inside the map
+        const int r = opaque(r16);
 #pragma unroll
-    for (int q = 0; q < MAXRT; q++)
+        for (int q = 0; q < F12_RT2; q++) {
+            const int m = min(((w >> 1) + 4 * q) * 16 + r, M2 - 1);  // past the last pixel: read, not stored
+            const int yo = (int)(((float)m + 0.5f) * i2), xo = m - yo * Wd2;
+            p0[q] = 2 * yo * Wd1 + 2 * xo;
+            const int rows = (yo > 0 ? 0x7 : 0) | 0x38 | (2 * yo + 1 < H1 ? 0x1c0 : 0);
+            const int cols = (xo > 0 ? 0x49 : 0) | 0x92 | (2 * xo + 1 < Wd1 ? 0x124 : 0);
+            okm[q] = rows & cols;
 #pragma unroll
-        for (int j = 0; j < TN2; j++) acc[q][j] = f4{0.f, 0.f, 0.f, 0.f};
-    int yb[MAXRT], xb[MAXRT];
-    bool mv[MAXRT];
-#pragma unroll
-    for (int q = 0; q < MAXRT; q++) {
-        const int m = (w + NW * q) * 16 + r16;
-        mv[q] = (w + NW * q) < RT2 && m < M2;
-        yb[q] = 2 * (m / Wd2) - 1;
-        xb[q] = 2 * (m % Wd2) - 1;
-    }
-    const bool any1 = w + NW < RT2, any2 = w + 2 * NW < RT2;
-    for (int s = 0; s < 9; s++) {
-        const int ky = s / 3, kx = s % 3;
-        bf8 b[TN2];
-#pragma unroll
-        for (int j = 0; j < TN2; j++)
-            b[j] = __builtin_bit_cast(bf8, *(const uint4*)(W2 + (size_t)(16 * j + r16) * g2.Kp + 32 * s + 8 * kg));
-#pragma unroll
-        for (int q = 0; q < MAXRT; q++) {
-            if ((q == 1 && !any1) || (q == 2 && !any2)) continue;
-            const int yi = yb[q] + ky, xi = xb[q] + kx;
-            const bool ok = mv[q] && yi >= 0 && yi < H1 && xi >= 0 && xi < Wd1;
-            const uint4 v = ok ? *(const uint4*)(map + (yi * Wd1 + xi) * F12_C1 + 8 * kg) : make_uint4(0u, 0u, 0u, 0u);
-            const bf8 a = __builtin_bit_cast(bf8, v);
-#pragma unroll
-            for (int j = 0; j < TN2; j++) acc[q][j] = mfma32(a, b[j], acc[q][j]);
+            for (int j = 0; j < 2; j++) acc[q][j] = f4{0.f, 0.f, 0.f, 0.f};
         }
-    }
-    __syncthreads();  // the map is read by every wave; its LDS now holds the output tile
-    bf16* T = map;
 #pragma unroll
-    for (int q = 0; q < MAXRT; q++) {
-        const int rt = w + NW * q;
-        if (rt >= RT2) continue;
+        for (int s = 0; s < 9; s++) {
+            const int d = (s / 3 - 1) * Wd1 + s % 3 - 1;
 #pragma unroll
-        for (int j = 0; j < TN2; j++) {
-            const float bv = b2[16 * j + r16];
+            for (int q = 0; q < F12_RT2; q++) {
+                const int at = cur + f12_slot(p0[q] + d, kg);
+                const bf8 x = *(const bf8*)(lds12 + (okm[q] & (1 << s) ? at : F12_ZERO + 16 * kg));
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int mr = rt * 16 + 4 * kg + e;
-                const float v = acc[q][j][e] + bv;
-                if (mr < M2) T[mr * C2LD + 16 * j + r16] = f2bf(v > 0.0f ? v : 0.0f);
+                for (int j = 0; j < 2; j++) acc[q][j] = mfma32(aw2[j][s], x, acc[q][j]);
             }
         }
-    }
-    __syncthreads();
-    constexpr int CPR = C2 / 8;
-    bf16* Yp = Y + (size_t)pair * M2 * C2;
-    for (int e = t; e < M2 * CPR; e += 512) {
-        const int rr = e / CPR, c = e - rr * CPR;
-        *(uint4*)(Yp + (size_t)rr * C2 + 8 * c) = *(const uint4*)(T + rr * C2LD + 8 * c);
+        bf16* Yp = Y + (size_t)pair * M2 * 64;
+#pragma unroll
+        for (int q = 0; q < F12_RT2; q++) {
+            const int rt = (w >> 1) + 4 * q, m = rt * 16 + r;
+            if (rt >= RT2 || m >= M2) continue;
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                *(u2*)(Yp + (size_t)m * 64 + 32 * (w & 1) + 16 * j + 4 * kg) = relu4(acc[q][j], bias2[j]);
+        }
+        if (next < g1.B) layer1(lds12 + (F12_MAP - cur));  // the other map: last read before the previous barrier
+        __syncthreads();
     }
 }
 
@@ -1218,7 +1252,8 @@ using namespace rt;
 
 // ---------------------------------------------------------------- host object
 struct rt_cnn {
-    int device = 0, max_batch = 0;
+    int device = 0, max_batch = 0, cus = 256;
+    bool fused12 = false;       // k_conv12_fused may use the LDS it needs on this device
     rt_cnn_config cfg;
     hipStream_t stream = nullptr;
     rt::HostStage st_src, st_flags;  // pinned staging of the frame table and the augmentation flags
@@ -1298,6 +1333,10 @@ extern "C" int rt_cnn_create(int device, const rt_cnn_config* c, int max_batch, 
     if (hipSetDevice(device) != hipSuccess) return set_error(RT_ERR_HIP, "hipSetDevice");
     rt_cnn* net = new rt_cnn();
     net->device = device; net->max_batch = max_batch; net->cfg = cfg;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0) net->cus = cus;
+    net->fused12 = hipFuncSetAttribute((const void*)k_conv12_fused, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       F12_MAP + 2 * F12_LDS) == hipSuccess;
     net->H[0] = cfg.in_height; net->W[0] = cfg.in_width;
     for (int l = 1; l < 7; l++) { net->H[l] = (net->H[l - 1] + 1) / 2; net->W[l] = (net->W[l - 1] + 1) / 2; }
     size_t o = 0;
@@ -1446,14 +1485,14 @@ static bool forward_mfma(const ConvGeom& g, const bf16* X, const bf16* Wp, const
 
 // The first two layers in one launch when their shapes are the fused
 // kernel's: 4 -> 32 -> 64 channels, the first layer's map within its LDS, the
-// second layer's rows within 3 row tiles per wave.
+// second layer's rows within a wave's row tiles.
 static bool forward_fused12(rt_cnn* net, int n, hipStream_t s) {
     const ConvGeom g1 = geom(net, 0, n), g2 = geom(net, 1, n);
     if (g1.Ci != 4 || g1.Co != F12_C1 || g1.Kp != 64 || g2.Ci != F12_C1 || g2.Co != 64 || g2.Kp != 9 * F12_C1 ||
-        g2.Hi != g1.Ho || g2.Wi != g1.Wo || g1.Ho * g1.Wo * F12_C1 > F12_LDS ||
-        g2.Ho * g2.Wo * (64 + 8) > F12_LDS || (g2.Ho * g2.Wo + 15) / 16 > 3 * 8)
+        g2.Hi != g1.Ho || g2.Wi != g1.Wo || (g1.Ho * g1.Wo + 1) / 2 * 2 * F12_C1 > F12_LDS ||
+        (g1.Ho * g1.Wo + 15) / 16 > 8 * F12_RT1 || (g2.Ho * g2.Wo + 15) / 16 > 4 * F12_RT2 || !net->fused12)
         return false;
-    k_conv12_fused<64><<<n, 512, 0, s>>>(g1, g2, net->act[0], net->Wp[0], net->params + net->b_off[0], net->Wp[1],
+    k_conv12_fused<<<std::min(n, net->cus), 512, F12_MAP + 2 * F12_LDS, s>>>(g1, g2, net->act[0], net->Wp[0], net->params + net->b_off[0], net->Wp[1],
                                          net->params + net->b_off[1], net->act[2]);
     return true;
 }

@@ -460,7 +460,8 @@ __device__ __forceinline__ void count_segments(const RT_GLOBAL uint8_t* bins, in
 // counts in the pair's point array, which kb_ref_points fills later, and each
 // workgroup of kb_select repeats the trim and the offsets and scatters its own
 // segments. One pair per workgroup left most CUs idle: 64 pairs of 640x480 147
-// us, split over 16 workgroups SELUS us; 256 mixed pairs 147 and SELUM us.
+// us, split over 16 workgroups 45 us (both launches); 256 mixed pairs 147 and 92
+// us.
 static int select_parts(int n) {
     int parts = 1;
     while (parts < 16 && 2 * parts * n <= 2048) parts *= 2;
