@@ -120,3 +120,42 @@ def test_reset_and_argument_errors():
         g.resample_from(g, np.eye(4))
     with pytest.raises(ValueError):
         g.set_depth(np.zeros((H + 1, W), np.uint16))
+
+
+@pytest.mark.parametrize("res,dim,W,H", [(8, (1500.0, 1500.0, 1500.0), 40, 24), (24, (1433.3, 1371.7, 1490.1), 50, 38),
+                                         (72, (1433.3, 1371.7, 1490.1), 96, 72), (136, (1500.0, 1500.0, 1500.0), 97, 61),
+                                         (264, (1500.0, 1433.3, 1500.0), 64, 48), (520, (1500.0, 1433.3, 1500.0), 64, 48)])
+def test_sign_map_and_slice_cull_at_tile_edges_bitexact(res, dim, W, H):
+    """Resolutions with partial 16-voxel tiles, one and several skip blocks, both block sizes,
+    voxel centres that floats hold and that they round; cameras outside and inside the grid,
+    behind the scene and along an axis; surfaces that move, so that signs turn both ways;
+    a resampled grid, then fused again."""
+    K = normalized_k(W, H)
+    print(f"tsdf grid res={res} image={W}x{H} dim={dim}", flush=True)
+    params = default_params(resolution=res, width=W, height=H, dim=dim)
+    g, o = VoxelGrid(params), Grid(res, W, H, ORIGIN, dim)
+    inside = pose(3, 100, (200, 30, -1500))
+    views = [pose(), UNFUSED, inside, pose(0, 180, (0, 0, -3600)), pose(90, 0, (10, 1800, -1600))]
+    ramp = (600 + 4 * np.arange(W)[None, :] + 3 * np.arange(H)[:, None]).astype(np.uint16)
+    d0 = np.round(render_depth(pose(), K, W, H)).astype(np.uint16)
+    frames = [(d0, pose()), (np.where(d0 > 400, d0 - 300, 0).astype(np.uint16), pose()), (ramp, inside), (d0, UNFUSED)]
+
+    def check(grid, oracle, what, poses):
+        assert _bits_equal(grid.read(), oracle.data), what
+        for k, Tr in enumerate(poses):
+            for name, a, b in zip(("xyz", "normals", "shade"), grid.raycast(Tr, K, True), oracle.raycast(Tr, K, True)):
+                assert _bits_equal(a, b), f"{name}, {what}, view {k}"
+
+    for i, (d, T) in enumerate(frames[:2] if res > 260 else frames):
+        g.integrate(d, T, K)
+        o.update(d.astype(np.float32), T, K)
+        check(g, o, f"frame {i}", views)
+    if res > 260:
+        return
+    dst, odst = VoxelGrid(params), Grid(res, W, H, ORIGIN, dim)
+    dst.resample_from(g, POSES[1])
+    odst.resample_from(o, POSES[1])
+    check(dst, odst, "resampled", views[:3])
+    dst.integrate(ramp, inside, K)
+    odst.update(ramp.astype(np.float32), inside, K)
+    check(dst, odst, "fused after resampling", views[:3])
