@@ -653,6 +653,23 @@ struct TrackCfg {
 };
 
 
+// The solve of one pair's photometric system as a call (on wave 0). Inlined,
+// its FP64 registers exceed the 128 per lane that a 1024-thread workgroup
+// leaves, and 70 of the passes' registers were spilled around it by every
+// wave; 10 with the call, whose cost only wave 0 pays: 6.39 -> 6.32 ms for 4096
+// pairs of 640 x 480 with 8192 points, 360 -> 355 us for 64. (The registers
+// that this frees do not hold a level's Jacobians: kept there, eight points a
+// thread, the passes spill again, 7.3 to 7.9 ms.)
+#define RT_LDS __attribute__((address_space(3)))
+__device__ __attribute__((noinline)) bool solve_photo(RT_LDS double* sys, RT_LDS float* T, RT_LDS double* ws, int solver,
+                                                      int robust, int mad_bins, float scale_out, int N) {
+    SolveCfg sc;
+    sc.solver = __builtin_amdgcn_readfirstlane(solver);
+    sc.mode = RT_PHOTOMETRIC; sc.lambda = 0.0f; sc.scale_out = scale_out;
+    sc.robust = robust; sc.mad_bins = mad_bins; sc.scale_in = 1e-3f;
+    return solve_update_wave((const double*)sys, (float*)T, sc, N, 0, (double*)ws);
+}
+
 // RZ: residual and zWeight of each point kept in registers (0) or in LDS (1,
 // at most RZ_MAX points per pair), trading LDS for occupancy.
 constexpr int RZ_MAX = 8192;
@@ -829,10 +846,8 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
                 }
                 __syncthreads();
                 if (wave == 0) {
-                    SolveCfg sc;
-                    sc.solver = cfg.solver; sc.mode = RT_PHOTOMETRIC; sc.lambda = 0.0f; sc.scale_out = cfg.scale_out;
-                    sc.robust = cfg.robust; sc.mad_bins = cfg.mad_bins; sc.scale_in = 1e-3f;
-                    const bool ok = solve_update_wave(sys, T, sc, N, 0, ws);
+                    const bool ok = solve_photo((RT_LDS double*)sys, (RT_LDS float*)T, (RT_LDS double*)ws, cfg.solver,
+                                                cfg.robust, cfg.mad_bins, cfg.scale_out, N);
                     if (t == 0) {
                         if (!ok) s_ok = 0;
                         rms_last = sys[28] > 0.0 ? (float)sqrt(sys[27] / sys[28]) : 0.0f;
