@@ -89,7 +89,7 @@ int rt_tsdf_resample(rt_tsdf* dst, const rt_tsdf* src, const float* T);
  * (host buffer). */
 int rt_tsdf_read(rt_tsdf* g, float* host, size_t bytes);
 /* Device pointer of the grid (the same layout), for callers that inspect it
- * on the device. */
+ * on the device (read only: the grid keeps a sign map beside it). */
 const float* rt_tsdf_data(rt_tsdf* g);
 /* The grid's stream (a hipStream_t) and a wait for everything queued on it. */
 void* rt_tsdf_stream(rt_tsdf* g);

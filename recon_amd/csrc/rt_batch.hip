@@ -8,10 +8,12 @@
 // coarse-to-fine photometric loop of a pair with workgroup barriers only:
 // residuals stay in registers between the residual and the system pass, the MAD
 // histogram lives in LDS, the 27 normal-equation terms are reduced in FP32 per
-// wave and combined across waves in FP64, and one lane runs the FP64 solve and
+// wave and combined across waves in FP64, and one wave runs the FP64 solve and
 // SE(3) update. Workgroup size and points per thread are template parameters
 // picked per batch by a timing autotuner; the pipeline is captured once into a
-// hipGraph and replayed.
+// hipGraph and replayed. Geometric and bi-objective batches, and small
+// photometric ones, track in lockstep instead: a few launches over all pairs
+// per iteration (launch_lockstep), with the same sums.
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include <math.h>
