@@ -1326,12 +1326,27 @@ struct rt_batch {
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Photometric batches up to this many pairs track in lockstep; larger ones
-// keep enough CUs busy with a workgroup of kb_track each. Tracking alone at
-// 8192 points, lockstep and the best kb_track variant: 640x480, 1 pair 259 and
-// 300 us, 16 pairs 293 and 325, 32 pairs 335 and 331, 64 pairs 440 and 371;
-// 320x240, 1 pair 198 and 243 us, 16 pairs 214 and 257, 32 pairs 244 and 260,
-// 64 pairs 318 and 282.
+// Photometric batches up to LOCK_PHOTO_PAIRS pairs of at least LOCK_PHOTO_POINTS
+// points track in lockstep; larger ones keep enough CUs busy with a workgroup
+// of kb_track each, and fewer points leave a lockstep launch with nothing but
+// its latency. Tracking alone in us, lockstep and the variant of kb_track that
+// the tuner picks:
+//   points       2048       4096       6144       8192      16384       32768
+//   640x480
+//    1 pair   261 188    262 233    264 273    265 313    278  710    313 1490
+//   16 pairs  279 202    282 249    287 299    295 348    335  794    411 1973
+//   24 pairs  287 201    297 249    314 299    325 348    383  921    498 1977
+//   320x240
+//    1 pair   195 142    195 176    198 207    199 237    208  535    233 1101
+//   24 pairs  213 153    217 190    227 226    232 263    279  658    373 1462
+//   160x120
+//   24 pairs  214 151    217 188    226 227    232 266
+// and at 8192 points 32 pairs of 640x480 335 and 331, 64 pairs 440 and 371.
+// The line lies at 8192 for the results as well: a thread's sums follow the
+// workgroup size, which is 1024 in lockstep, and there is where the tuner picks
+// a workgroup of 1024 by more than timings differ (7 % ahead at 8192 points, 2
+// to 4 % at 6144 and 160x120, behind 512 below 2048).
+constexpr int LOCK_PHOTO_POINTS = 8192;
 constexpr int LOCK_PHOTO_PAIRS = 24;
 
 // Device memory a batch's descriptors point into: per-pair arenas of
@@ -1402,13 +1417,15 @@ extern "C" int rt_batch_create(int device, int max_pairs, int max_w, int max_h, 
               dal((void**)&b->queue, 256) && dal((void**)&b->calib_dev, 96 * 4 * (size_t)max_pairs) &&
               dal((void**)&b->trel_in, 64 * (size_t)max_pairs) && dal((void**)&b->trel_out, 64 * (size_t)max_pairs) &&
               dal((void**)&b->rms, 4 * (size_t)max_pairs) && dal((void**)&b->status, 4 * (size_t)max_pairs);
-    b->lock_pairs = b->prm.mode == RT_PHOTOMETRIC ? std::min(max_pairs, LOCK_PHOTO_PAIRS) : max_pairs;
+    b->lock_pairs = max_pairs;
+    if (b->prm.mode == RT_PHOTOMETRIC)
+        b->lock_pairs = b->prm.n_select < LOCK_PHOTO_POINTS ? 0 : std::min(max_pairs, LOCK_PHOTO_PAIRS);
     const bool icp = b->prm.mode != RT_PHOTOMETRIC;
     b->lock.o_rz = align256(LK_FIXED);
     b->lock.o_bits = b->lock.o_rz + align256(8 * (size_t)b->prm.n_select);
     b->lock.o_rfull = b->lock.o_bits + (icp ? 8 * 16 * (size_t)LK_BLOCKS : 0);
     b->lock.stride = align256(b->lock.o_rfull + (icp ? 4 * (size_t)max_w * max_h : 0));
-    ok = ok && dal((void**)&b->lock.base, b->lock.stride * (size_t)b->lock_pairs);
+    ok = ok && (b->lock_pairs == 0 || dal((void**)&b->lock.base, b->lock.stride * (size_t)b->lock_pairs));
     if (!ok) {
         rt_batch_destroy(b);
         return set_error(RT_ERR_NOMEM, "batch buffers");
@@ -1641,8 +1658,8 @@ static void launch_lockstep(const rt_batch* b, int depths, hipStream_t s) {
         kl_solve<<<n, 64, 0, s>>>(v.desc, b->lock, step, cfg);
     }
 }
-// The geometric modes always, photometric batches while they are small (a
-// variant forced through the environment keeps kb_track).
+// The geometric modes always, photometric batches of few pairs with many points
+// (lock_pairs; a variant forced through the environment keeps kb_track).
 static bool tracks_in_lockstep(const rt_batch* b) {
     if (b->prm.mode != RT_PHOTOMETRIC) return true;
     return b->n <= b->lock_pairs && !getenv("RT_BATCH_VARIANT");

@@ -152,14 +152,14 @@ def test_batch_kernel_variants_agree(N, iters, monkeypatch, capfd):
         assert (1, True) in kinds and (1, False) in kinds
 
 
-@pytest.mark.parametrize("N,iters,robust,bins", [(256, (1, 3, 10, 5), 0, 64), (2048, (2, 0, 3, 1), 1, 256),
+@pytest.mark.parametrize("N,iters,robust,bins", [(8192, (2, 0, 3, 1), 1, 256),
                                                  (8192, (1, 3, 10, 5), 0, 64), (8448, (0, 1, 0, 2), 0, 64),
-                                                 (16640, (1, 1, 1, 1), 0, 64), (2048, (0, 0, 0, 0), 0, 64)])
+                                                 (16640, (1, 1, 1, 1), 0, 64), (8192, (0, 0, 0, 0), 0, 64)])
 def test_lockstep_equals_the_persistent_kernel(N, iters, robust, bins, monkeypatch):
-    """Small batches track in lockstep launches, whose sums are those of a
-    1024-thread workgroup of the persistent kernel: the same poses and RMS bit
-    for bit, with points below, at and past a round's 8192 and levels or whole
-    schedules without iterations."""
+    """Batches of few pairs with 8192 points or more track in lockstep launches,
+    whose sums are those of a 1024-thread workgroup of the persistent kernel:
+    the same poses and RMS bit for bit, with points at and past a round's 8192
+    and levels or whole schedules without iterations."""
     import ctypes
     from recon_amd import lib
     print(f"case lockstep N {N} iters {iters}", flush=True)
@@ -179,6 +179,34 @@ def test_lockstep_equals_the_persistent_kernel(N, iters, robust, bins, monkeypat
         bt.close()
         res[force] = a + b
     for x, y in zip(res[None], res[v]):
+        assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("n,N", [(1, 256), (5, 1536), (7, 4096), (3, 7936)])
+def test_few_points_track_with_the_tuned_kernel(n, N, monkeypatch, capfd):
+    """Below 8192 points a batch of few pairs runs the kernel that the tuner
+    picks, whose workgroup size gives the order of its sums: its poses and RMS
+    are that variant's, bit for bit."""
+    import ctypes
+    from recon_amd import lib
+    print(f"case tuned batch n {n} N {N}", flush=True)
+    pairs, host, _ = _batch(n, theta=2.0, tmax=30.0, seed=130, rig=True)
+    monkeypatch.setenv("RT_VERBOSE", "1")
+    monkeypatch.delenv("RT_BATCH_VARIANT", raising=False)
+    bt = BatchTracker(n, 640, 480, mode=PHOTOMETRIC, n_select=N)
+    capfd.readouterr()
+    got = bt.track(pairs)
+    lines = [s for s in capfd.readouterr().err.splitlines() if "rt_batch autotune" in s and "->" in s]
+    assert len(lines) == 1, "the tuner's choice"
+    f = lines[0].split("->")[1].split()
+    cfg = dict(zip(f[0:10:2], map(int, f[1:10:2])))
+    info, v = (ctypes.c_int * 6)(), 0
+    while lib().rt_batch_variant_info(v, info) == 0 and [cfg[k] for k in ("bs", "ppt", "rz", "pc", "wpe")] != info[:5]:
+        v += 1
+    monkeypatch.setenv("RT_BATCH_VARIANT", str(v))
+    forced = BatchTracker(n, 640, 480, mode=PHOTOMETRIC, n_select=N).track(pairs)
+    assert np.all(got[3] == 0)
+    for x, y in zip(got, forced):
         assert np.array_equal(x, y)
 
 
