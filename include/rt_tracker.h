@@ -287,6 +287,11 @@ int rt_batch_debug_read(rt_batch* b, int pair, int what, int level, void* host, 
  * the work order (n ints); maxes: the largest width, height and point count. */
 int rt_batch_layout(const rt_params* params, int max_width, int max_height, int n, const rt_pair* pairs,
                     int64_t* fields, int* order, int maxes[3]);
+/* The same for the memory of a pair in lockstep tracking (few pairs, and the
+ * geometric and bi-objective modes): off: the offsets of its wave sums,
+ * histograms, block counts, block sums of the three Student-t rounds,
+ * residuals, validity bits, residual map, and its size. */
+int rt_batch_lock_layout(const rt_params* params, int max_width, int max_height, int64_t off[10]);
 
 /* No counterpart in the reference. For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that

@@ -94,6 +94,7 @@ SIGNATURES = {
     "rt_batch_variant_info": (c_int, [c_int, P(c_int)]),
     "rt_batch_track_noalloc": (c_int, [c_int, c_int, P(RtPair), P(RtParams), c_void_p, P(RtPairResult)]),
     "rt_batch_layout": (c_int, [P(RtParams), c_int, c_int, c_int, P(RtPair), P(ctypes.c_int64), P(c_int), P(c_int)]),
+    "rt_batch_lock_layout": (c_int, [P(RtParams), c_int, c_int, P(ctypes.c_int64)]),
     "rt_batch_debug_read": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_size_t]),
     "rt_debug_read": (c_int, [c_void_p, c_int, c_int, c_void_p, c_size_t]),
     "rt_debug_set_trel": (c_int, [c_void_p, P(c_float)]),

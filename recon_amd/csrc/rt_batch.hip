@@ -879,7 +879,9 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
 // the points j = 8 round + w (one per lane) and leaves them in LDS, and after
 // a barrier four of the waves add eight terms each over the round's eight j, so
 // that the points are formed by eight waves while each sum stays one chain.
-constexpr int LK_BLOCKS = 512;  // blocks of 1024 pixels: W x H <= 512 x 1024, checked at preparation
+// Most pixels of a pair (build_batch refuses more: whole segments of its 512 in
+// the selection hold up to 1024 pixels), and their blocks of 1024.
+constexpr int MAX_PIXELS = 512 * 1025 - 1, LK_BLOCKS = (MAX_PIXELS + 1023) / 1024;
 struct LockBufs {
     char* base;        // per pair: the arrays below
     size_t stride, o_rz, o_bits, o_rfull;
@@ -1349,6 +1351,17 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 constexpr int LOCK_PHOTO_POINTS = 8192;
 constexpr int LOCK_PHOTO_PAIRS = 24;
 
+// The arrays of lockstep tracking for pairs of up to max_w x max_h and nsel
+// points (base unset); icp: with those of the ICP selection.
+static LockBufs lock_layout(int max_w, int max_h, size_t nsel, bool icp) {
+    LockBufs k{};
+    k.o_rz = align256(LK_FIXED);
+    k.o_bits = k.o_rz + align256(8 * nsel);
+    k.o_rfull = k.o_bits + (icp ? 8 * 16 * (size_t)LK_BLOCKS : 0);
+    k.stride = align256(k.o_rfull + (icp ? 4 * (size_t)max_w * max_h : 0));
+    return k;
+}
+
 // Device memory a batch's descriptors point into: per-pair arenas of
 // pair_bytes (sized for max_w x max_h and nsel points) and the per-pair tables.
 struct BatchMem {
@@ -1420,11 +1433,7 @@ extern "C" int rt_batch_create(int device, int max_pairs, int max_w, int max_h, 
     b->lock_pairs = max_pairs;
     if (b->prm.mode == RT_PHOTOMETRIC)
         b->lock_pairs = b->prm.n_select < LOCK_PHOTO_POINTS ? 0 : std::min(max_pairs, LOCK_PHOTO_PAIRS);
-    const bool icp = b->prm.mode != RT_PHOTOMETRIC;
-    b->lock.o_rz = align256(LK_FIXED);
-    b->lock.o_bits = b->lock.o_rz + align256(8 * (size_t)b->prm.n_select);
-    b->lock.o_rfull = b->lock.o_bits + (icp ? 8 * 16 * (size_t)LK_BLOCKS : 0);
-    b->lock.stride = align256(b->lock.o_rfull + (icp ? 4 * (size_t)max_w * max_h : 0));
+    b->lock = lock_layout(max_w, max_h, (size_t)b->prm.n_select, b->prm.mode != RT_PHOTOMETRIC);
     ok = ok && (b->lock_pairs == 0 || dal((void**)&b->lock.base, b->lock.stride * (size_t)b->lock_pairs));
     if (!ok) {
         rt_batch_destroy(b);
@@ -1757,7 +1766,7 @@ static int build_batch(const rt_params& prm, const BatchMem& m, int n, const rt_
         if (!p.ref_gray || !p.ref_depth || !p.cur_gray || !p.cur_depth || !p.calib) return set_error(RT_ERR_ARG, "null pair input");
         if (p.width > m.max_w || p.height > m.max_h || p.width % (2 * mm) || p.height % mm || p.width < 32 || p.height < 32)
             return set_error(RT_ERR_ARG, "pair size not supported by this batch");
-        if ((p.width * p.height) / 512 > 1024) return set_error(RT_ERR_ARG, "pair too large");
+        if ((int64_t)p.width * p.height > MAX_PIXELS) return set_error(RT_ERR_ARG, "pair too large");
         int N = q.n_select;
         if (N > p.width * p.height / 2) return set_error(RT_ERR_ARG, "n_select above half the pixels of a pair");
         PairDesc& d = desc[i];
@@ -2170,5 +2179,19 @@ extern "C" int rt_batch_layout(const rt_params* params, int max_w, int max_h, in
         f[37] = off(d.zblk);
         f[38] = f[39] = 0;
     }
+    return RT_OK;
+}
+
+// A pair's memory in lockstep tracking, as byte offsets from its start (host
+// code only, for bounds checks of the launches on the CPU).
+extern "C" int rt_batch_lock_layout(const rt_params* params, int max_w, int max_h, int64_t off[10]) {
+    if (!off || max_w < 32 || max_h < 32) return set_error(RT_ERR_ARG, "rt_batch_lock_layout: bad argument");
+    rt_params prm;
+    if (params) prm = *params; else rt_default_params(&prm);
+    LockBufs k = lock_layout(max_w, max_h, (size_t)prm.n_select, prm.mode != RT_PHOTOMETRIC);
+    k.base = reinterpret_cast<char*>((uintptr_t)1 << 40);  // nominal: only offsets from it are reported
+    const void* const at[10] = {k.wsum(0, 0), k.hist(0, 0), k.cnt(0),  k.bsum(0, 0),  k.bsum(0, 1),
+                                k.bsum(0, 2), k.rz(0),      k.bits(0), k.rfull(0), k.base + k.stride};
+    for (int i = 0; i < 10; i++) off[i] = (const char*)at[i] - k.base;
     return RT_OK;
 }

@@ -313,6 +313,57 @@ def _check_kernels(f, maxes, max_w, max_h, pcs=(0, 5120, 5632, 8192)):
                     assert v[0] <= v[1], (p, k, v)
 
 
+def _lock_layout(max_w, max_h, N, mode):
+    off = np.zeros(10, np.int64)
+    prm = default_params(n_select=N, mode=mode)
+    assert lib().rt_batch_lock_layout(ctypes.byref(prm), max_w, max_h,
+                                      off.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))) == 0
+    names = ("wsum", "hist", "cnt", "bsum0", "bsum1", "bsum2", "rz", "bits", "rfull", "end")
+    return dict(zip(names, (int(v) for v in off)))
+
+
+def _check_lockstep(W, H, L, N, off, mode):
+    """Largest byte that the kl_* launches touch in each of a pair's arrays,
+    against the start of the next one."""
+    names = list(off)
+    end = {a: off[b] for a, b in zip(names, names[1:])}
+    used = {"wsum": 4 * (512 + 32 * 15 + 31), "hist": 4 * (256 + 255), "rz": 8 * (N - 1) + 4}
+    if mode != 1:
+        for layer in range(L):
+            npix = (W >> layer) * (H >> layer)
+            blocks = (npix + 1023) // 1024              # kl_icp_mask, kl_icp_compact: one per 1024 pixels
+            assert blocks <= 1024                       # wave_student_total's reach, and cnt[t], t < g
+            used["cnt"] = max(used.get("cnt", 0), 4 * (blocks - 1))
+            used["bits"] = max(used.get("bits", 0), 8 * (16 * (blocks - 1) + 15))   # the words of every wave
+            used["rfull"] = max(used.get("rfull", 0), 4 * (npix - 1))
+            for r in range(3):                          # a block sum per 1024 of at most npix points
+                used[f"bsum{r}"] = max(used.get(f"bsum{r}", 0), 4 * (blocks - 1))
+    for k, last in used.items():
+        elem = 8 if k == "bits" else 4
+        assert off[k] % (8 if k in ("bits", "rz") else 4) == 0
+        assert off[k] + last + elem <= end[k], (W, H, L, N, k, last, off[k], end[k])
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("W,H,levels", [(160, 120, 0), (640, 480, 0), (904, 580, 3), (1024, 512, 4), (656, 799 // 8 * 8, 4),
+                                        (32, 32, 1)])
+def test_lockstep_launches_stay_in_bounds(W, H, levels, mode):
+    """Up to the most pixels that a preparation admits (524,799: 904x580 is
+    513 blocks of 1024), each array's last element lies before the next one."""
+    N = min(8192, W * H // 2 // 256 * 256)
+    L = levels or (4 if W == 640 else 3)
+    prm = default_params(n_select=N, mode=mode, levels=levels)
+    f, order, maxes = np.zeros(FIELDS, np.int64), np.zeros(1, np.int32), np.zeros(3, np.int32)
+    cal = np.ones(96, np.float32)
+    p = RtPair(ref_gray=0x1000, ref_depth=0x2000, cur_gray=0x3000, cur_depth=0x4000, width=W, height=H,
+               calib=cal.ctypes.data_as(ctypes.POINTER(ctypes.c_float)))
+    assert lib().rt_batch_layout(ctypes.byref(prm), W, H, 1, ctypes.byref(p),
+                                 f.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)),
+                                 order.ctypes.data_as(ctypes.POINTER(ctypes.c_int)),
+                                 maxes.ctypes.data_as(ctypes.POINTER(ctypes.c_int))) == 0
+    _check_lockstep(W, H, L, N, _lock_layout(W, H, N, mode), mode)
+
+
 def _mixed_256():
     """The mixed-size workload's 256 pairs: sizes drawn by rng(3)."""
     rng = np.random.default_rng(3)
