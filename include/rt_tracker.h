@@ -358,6 +358,10 @@ int rt_debug_linearize(rt_tracker* t, int level, int it);
  * No counterpart in the reference (whose kernels divide); it lets a test
  * compare the device reciprocal with IEEE division over every input. */
 int rt_debug_depth_reciprocals(int device, float* host, int n);
+/* The number of floats z, of either sign, with 2^-60 <= |z| < 2^61 whose
+ * reciprocal, as the depth and voxel kernels take it, is not the IEEE quotient
+ * 1 / z on this device. */
+int rt_debug_reciprocals(int device, int64_t* bad);
 
 const char* rt_last_error(void);
 

@@ -1986,10 +1986,33 @@ extern "C" int rt_batch_results(rt_batch* b, rt_pair_result* out) {
     return fetch_results(b, out);
 }
 
-// rcp_depth(-u) for u = 1 .. n, the reciprocal kb_bins takes of each 16-bit depth
+// rcp_rn(-u) for u = 1 .. n, the reciprocal kb_bins takes of each 16-bit depth
 __global__ __launch_bounds__(256) void k_depth_reciprocals(float* out, int n) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] = rcp_depth(-(float)(i + 1));
+    if (i < n) out[i] = rcp_rn(-(float)(i + 1));
+}
+// counts the floats of either sign with 2^-60 <= |z| < 2^61 where rcp_rn is not the IEEE quotient
+__global__ __launch_bounds__(256) void k_reciprocals(unsigned long long* bad) {
+    const unsigned long long total = 2ull * 121 << 23;
+    unsigned long long n = 0;
+    for (unsigned long long i = blockIdx.x * 256ull + threadIdx.x; i < total; i += gridDim.x * 256ull) {
+        const unsigned m = (unsigned)i & 0x7fffffu, se = (unsigned)(i >> 23);  // mantissa; sign and binade
+        const float z = __uint_as_float((se / 121) << 31 | (127 - 60 + se % 121) << 23 | m);
+        n += __float_as_uint(rcp_rn(z)) != __float_as_uint(1.0f / z);
+    }
+    if (n) atomicAdd(bad, n);
+}
+extern "C" int rt_debug_reciprocals(int device, int64_t* bad) {
+    if (!bad) return set_error(RT_ERR_ARG, "rt_debug_reciprocals: null argument");
+    if (hipSetDevice(device) != hipSuccess) return set_error(RT_ERR_HIP, "hipSetDevice");
+    unsigned long long *d = nullptr, n = 0;
+    if (hipMalloc(&d, sizeof(n)) != hipSuccess) return set_error(RT_ERR_HIP, "rt_debug_reciprocals: alloc");
+    bool ok = hipMemcpy(d, &n, sizeof(n), hipMemcpyHostToDevice) == hipSuccess;
+    if (ok) k_reciprocals<<<4096, 256>>>(d);
+    ok = ok && hipGetLastError() == hipSuccess && hipMemcpy(&n, d, sizeof(n), hipMemcpyDeviceToHost) == hipSuccess;
+    hipFree(d);
+    *bad = (int64_t)n;
+    return ok ? RT_OK : set_error(RT_ERR_HIP, "rt_debug_reciprocals: launch or copy");
 }
 extern "C" int rt_debug_depth_reciprocals(int device, float* host, int n) {
     if (!host || n < 1 || n > 65535) return set_error(RT_ERR_ARG, "rt_debug_depth_reciprocals: n outside [1, 65535]");

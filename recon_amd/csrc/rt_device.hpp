@@ -261,13 +261,16 @@ __device__ __forceinline__ float div_rn(float a, float b, float y) {
 // an 8-bit gray value t as (float)t / 255, the IEEE quotient, by div_rn
 // (three instructions; all 256 values checked against IEEE division)
 __device__ __forceinline__ float u8_unit(unsigned t) { return div_rn((float)t, 255.0f, 1.0f / 255.0f); }
-// RN(1 / z) for z = -u, u an integer in [1, 65535] (a negated 16-bit depth
-// value): the hardware reciprocal (within 1 ulp) refined by one Newton step
-// with fused multiply-adds, y + y (1 - z y). The residual 1 - z y is exact,
-// and for these 65535 inputs the result equals the IEEE division 1.0f / z bit
-// for bit (compared exhaustively against IEEE float32 division by a test); it
-// is not claimed for other inputs. Three instructions instead of about eleven.
-__device__ __forceinline__ float rcp_depth(float z) {
+// RN(1 / z) for 2^-60 <= |z| < 2^61: the hardware reciprocal (within 1 ulp)
+// refined by one Newton step with fused multiply-adds, y + y (1 - z y). The
+// residual 1 - z y is exact, but the step alone does not round every value that
+// starts within 1 ulp to RN(1 / z): it leaves one float below it where z has an
+// all-ones mantissa and the start is the float below 1 / z, and at 32 further
+// starts one float above RN(1 / z). gfx950's v_rcp_f32 starts from none of them:
+// a test compares all 2 x 121 x 2^23 values of the range with the IEEE division
+// on the device (and the 65535 negated 16-bit depths with the host's). Three
+// instructions instead of about eleven.
+__device__ __forceinline__ float rcp_rn(float z) {
     const float y = __builtin_amdgcn_rcpf(z);
     const float e = __builtin_fmaf(-z, y, 1.0f);
     return __builtin_fmaf(e, y, y);
@@ -294,7 +297,7 @@ struct LdsTile {
 // (the same quotients; a zero coordinate may change sign, which the
 // projection maps to the same position: it is only ever added to cx, cy or
 // scaled into a sum). SIMPLE: the calibration satisfies calib_simple; then
-// the projection divides by zc itself, whose reciprocal rcp_depth gives.
+// the projection divides by zc itself, whose reciprocal rcp_rn gives.
 // In bounds, p.x >= 10, so p.x - 1 is exact and (int)(p.x - 1) = xdi - 1
 // (likewise for y): of the four neighbour positions only p + 1 can round
 // onto the next integer, and only xe and ys are tested.
@@ -309,7 +312,7 @@ __device__ __forceinline__ float grad_mag_tiled(float zc, const ZS& z, const GS&
     }
     if (p3.z < 0.0f) {
         f3 r3 = SIMPLE ? p3 : mul4(c + TLR, p3);
-        const float iz = SIMPLE ? rcp_depth(r3.z) : 1.0f / r3.z;
+        const float iz = SIMPLE ? rcp_rn(r3.z) : 1.0f / r3.z;
         f2 pu{div_rn(r3.x, r3.z, iz), div_rn(r3.y, r3.z, iz)};
         f2 p = SIMPLE ? project_simple(pu, c + KR) : distort(pu, c + KCR, c + KR);
         if (in_bounds(p, k.xmax, k.ymax)) {

@@ -79,13 +79,12 @@ struct TsdfCull {
 };
 
 // rx / rz and ry / rz, the IEEE quotients. With all three between 2^-60 and
-// 2^60 in magnitude nothing over- or underflows: the reciprocal (within 1 ulp,
-// refined by one fused Newton step) is RN(1 / rz) and div_rn is exact; a zero,
-// a huge or a tiny value takes the divisions. Twelve instructions for about 22.
+// 2^60 in magnitude nothing over- or underflows, the reciprocal is RN(1 / rz)
+// (rcp_rn's range) and div_rn is exact; a zero, a huge or a tiny value takes the
+// divisions. Twelve instructions for about 22.
 __device__ __forceinline__ void quotients(float rx, float ry, float rz, float& qx, float& qy) {
     const float big = 1152921504606846976.0f, small = 1.0f / 1152921504606846976.0f;
-    const float y0 = __builtin_amdgcn_rcpf(rz);
-    const float y = __builtin_fmaf(y0, __builtin_fmaf(-rz, y0, 1.0f), y0);
+    const float y = rcp_rn(rz);
     qx = div_rn(rx, rz, y); qy = div_rn(ry, rz, y);
     const float hi = fmaxf(fmaxf(fabsf(rx), fabsf(ry)), fabsf(rz)), lo = fminf(fminf(fabsf(rx), fabsf(ry)), fabsf(rz));
     if (!(hi <= big && lo >= small)) { qx = rx / rz; qy = ry / rz; }

@@ -3,8 +3,10 @@
  * IEEE division: random normal operands over 56 binades, and the
  * back-projection domain of the gradient pass, a = (x - c) z over pixel
  * columns x and every 16-bit depth z, divided by the focal length and then by
- * z, and the 256 8-bit gray values over 255. Prints the mismatch count;
- * exit status 1 on any mismatch. */
+ * z, and the 256 8-bit gray values over 255; and the Newton step of rcp_rn from
+ * RN(1/z) and the floats beside it, over every mantissa: the 33 starts from
+ * which it misses RN(1/z), the all-ones mantissa from the float below among
+ * them. Prints the mismatch count; exit status 1 on any mismatch. */
 #include <math.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -48,6 +50,21 @@ int main(int argc, char** argv) {
     }
     /* the 8-bit gray values over 255 (the pyramid's conversion, u8_unit) */
     for (int t = 0; t < 256; t++) { n++; bad += !same(div_rn((float)t, 255.0f, 1.0f / 255.0f), (float)t / 255.0f); }
+    long missed = 0, below = 0;
+    for (uint32_t m = 0; m < 1u << 23; m++) {
+        const uint32_t uz = 0x3f800000u | m;
+        float z, rn;
+        memcpy(&z, &uz, 4);
+        rn = 1.0f / z;
+        for (int s = -1; s <= 1; s++) {
+            float y0 = s < 0 ? nextafterf(rn, 0.0f) : s > 0 ? nextafterf(rn, 2.0f) : rn;
+            int miss = !same(fmaf(y0, fmaf(-z, y0, 1.0f), y0), rn);
+            missed += miss;
+            below += miss && s <= 0 && m == 0x7fffffu;
+            bad += miss && s <= 0 && m != 0x7fffffu;
+        }
+    }
+    bad += missed != 33 || below != 1;
     printf("%ld mismatches in %ld divisions\n", bad, n);
     return bad ? 1 : 0;
 }
