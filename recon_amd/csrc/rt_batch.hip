@@ -1415,6 +1415,7 @@ extern "C" int rt_batch_create(int device, int max_pairs, int max_w, int max_h, 
     }
     if (b->prm.mode < RT_GEOMETRIC || b->prm.mode > RT_BIOBJECTIVE) { rt_batch_destroy(b); return set_error(RT_ERR_ARG, "bad mode"); }
     b->prm.lambda = std::min(1.0f, std::max(0.0f, b->prm.lambda));  // setLambda's clamp (phototracker.cpp:163-168)
+    for (int& n : b->prm.iters) n = std::max(0, n);  // a count below one is a level without iterations
     b->pair_bytes = pair_arena_bytes(max_w, max_h, (size_t)b->prm.n_select, b->prm.mode != RT_PHOTOMETRIC);
     size_t total = b->pair_bytes * (size_t)max_pairs;
     void* q = nullptr;

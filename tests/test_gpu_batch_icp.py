@@ -90,3 +90,17 @@ def test_batch_icp_matches_single_and_oracle(mode):
         assert np.radians(es[0]) < 1e-5 and es[1] < 1e-2, i
         assert np.radians(e32[0]) < 1e-5 and e32[1] < 1e-2, i
     bt.close()
+
+
+@pytest.mark.parametrize("mode,iters", [(BIOBJECTIVE, (-1, 3, 2, 1)), (GEOMETRIC, (2, -7, 1, -1)),
+                                        (GEOMETRIC, (-1, -1, -1, -1))])
+def test_negative_iteration_counts_are_levels_without_iterations(mode, iters):
+    print(f"case batch icp mode {mode} iters {iters}", flush=True)
+    pairs = _pairs(4, 1300)
+    res = []
+    for it in (iters, [max(0, k) for k in iters]):
+        bt = BatchTracker(len(pairs), 640, 480, mode=mode, n_select=2048, iters=it, lam=0.5)
+        res.append(bt.track(pairs, init=[p["init"] for p in pairs]))
+        bt.close()
+    for x, y in zip(*res):
+        assert np.array_equal(x, y)
