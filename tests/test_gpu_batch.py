@@ -154,12 +154,14 @@ def test_batch_kernel_variants_agree(N, iters, monkeypatch, capfd):
 
 @pytest.mark.parametrize("N,iters,robust,bins", [(8192, (2, 0, 3, 1), 1, 256),
                                                  (8192, (1, 3, 10, 5), 0, 64), (8448, (0, 1, 0, 2), 0, 64),
-                                                 (16640, (1, 1, 1, 1), 0, 64), (8192, (0, 0, 0, 0), 0, 64)])
+                                                 (16640, (1, 1, 1, 1), 0, 64), (8192, (0, 0, 0, 0), 0, 64),
+                                                 (8192, (340, 350, 340, 10), 0, 64)])
 def test_lockstep_equals_the_persistent_kernel(N, iters, robust, bins, monkeypatch):
     """Batches of few pairs with 8192 points or more track in lockstep launches,
     whose sums are those of a 1024-thread workgroup of the persistent kernel:
-    the same poses and RMS bit for bit, with points at and past a round's 8192
-    and levels or whole schedules without iterations."""
+    the same poses and RMS bit for bit, with points at and past a round's 8192,
+    levels or whole schedules without iterations, and a schedule past the 1024
+    steps that a graph holds."""
     import ctypes
     from recon_amd import lib
     print(f"case lockstep N {N} iters {iters}", flush=True)
