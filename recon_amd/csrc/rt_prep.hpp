@@ -816,6 +816,13 @@ __device__ __forceinline__ float robust_weight(float r, float zw, float s, int r
 
 
 // ------------------------------------------------------------------ A18-A23 per pixel / point
+// div_rn where a or b may be infinite or b zero: the remainder is not a number
+// then, and the product is the IEEE quotient itself (infinite, zero, or NaN).
+__device__ __forceinline__ float div_rn_inf(float a, float b, float y) {
+    const float q = a * y;
+    const float r = __builtin_fmaf(-b, q, a);
+    return r == r ? __builtin_fmaf(r, y, q) : q;
+}
 // backproject with the quotients by the focal lengths as div_rn (ifx, ify: RN
 // of their reciprocals): the same values, a zero coordinate's sign aside.
 __device__ __forceinline__ bool backproject_rn(float z, int xi, int yi, const float* c, float ifx, float ify, f3& p) {
@@ -862,12 +869,13 @@ __device__ __forceinline__ void ref_cloud_pixel(const ZS& zs, int W, int H, int 
     }
     pos = make_float4(p.x, p.y, p.z, mask);
 }
-// genPointsCloud6Kernel (d2z.cu:436-469) for pixel (x, y): every z < 0 is valid.
+// genPointsCloud6Kernel (d2z.cu:436-469) for pixel (x, y): every z < 0 is valid,
+// an infinite one (of a float depth map) too.
 __device__ __forceinline__ float4 cur_cloud_pixel(float z, int x, int y, const float* __restrict__ c, float ifx,
                                                   float ify) {
     if (!(z < 0.0f)) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    return make_float4(div_rn(((float)x - c[KL + 2]) * z, c[KL], ifx), div_rn(((float)y - c[KL + 5]) * z, c[KL + 4], ify),
-                       z, 1.0f);
+    return make_float4(div_rn_inf(((float)x - c[KL + 2]) * z, c[KL], ifx),
+                       div_rn_inf(((float)y - c[KL + 5]) * z, c[KL + 4], ify), z, 1.0f);
 }
 // downSampleCloud6Kernel (d2z.cu:557-588) for one pixel from its four taps:
 // masked mean position and, with normals, their masked mean renormalised.
@@ -946,10 +954,8 @@ __device__ __forceinline__ bool icp_mask_pixel(const float4* __restrict__ rp, co
     f3 q3 = mul4(T, p3);
     f3 cn = rot4(T, n3);
     const float* K = c + KL;
-    // the quotients as div_rn (a zero or non-finite z gives NaN where the
-    // division gives an infinity, which the bounds reject alike)
     const float iz = 1.0f / q3.z;
-    float qx = div_rn(q3.x, q3.z, iz), qy = div_rn(q3.y, q3.z, iz);
+    float qx = div_rn_inf(q3.x, q3.z, iz), qy = div_rn_inf(q3.y, q3.z, iz);
     float px = a * (K[0] * qx + K[2]) + b;
     float py = a * (K[4] * qy + K[5]) + b;
     if (!(px >= 0.0f && px < (float)(w - 1) && py >= 0.0f && py < (float)(h - 1))) return false;
@@ -989,6 +995,8 @@ __device__ __forceinline__ void icp_point_terms(float4 p, float4 nn, const float
     f3 q3 = mul4(T, p3);
     f3 cn = rot4(T, rnv);
     const float* K = c + KL;
+    // a zero or infinite z gives NaN here, which the bounds reject: the IEEE
+    // quotient by zero leaves the view too, and at an infinite z no term remains
     const float iz = 1.0f / q3.z;
     float qx = div_rn(q3.x, q3.z, iz), qy = div_rn(q3.y, q3.z, iz);
     float px = a * (K[0] * qx + K[2]) + b;
@@ -997,7 +1005,8 @@ __device__ __forceinline__ void icp_point_terms(float4 p, float4 nn, const float
 #pragma unroll
     for (int k = 0; k < 6; k++) J[k] = 0.0f;
     if (px >= 0.0f && px < (float)(w - 1) && py >= 0.0f && py < (float)(h - 1)) {
-        const float t2 = iw.plain ? div_rn(x2, iw.var, iw.inv) : x2 / iw.var;
+        // x2 up to 1e24: nothing overflows, and a residual whose square did weighs 0
+        const float t2 = iw.plain && x2 <= 1e24f ? div_rn(x2, iw.var, iw.inv) : x2 / iw.var;
         float wt = fminf(6 / (5 + t2), 1.0f);
         int xdi = (int)px, ydi = (int)py;
         float fx = px - (float)xdi, fy = py - (float)ydi;
@@ -1070,7 +1079,7 @@ __device__ __forceinline__ float wave_student_block(const float* __restrict__ r2
     for (int k = 0; k < 16; k++) {
         const float x = v[k];
         const float w = 6 / (5 + (iw.plain ? div_rn(x, iw.var, iw.inv) : x / iw.var));
-        const int sum = x * w;
+        const int sum = x * w;  // 0 for an infinite x: x * w is not a number
         v[k] = bk * 1024 + lane + 64 * k < n ? (float)sum : 0.0f;
     }
     return wave_tree1024(v);

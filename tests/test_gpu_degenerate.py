@@ -89,3 +89,46 @@ def test_geometric_levels_without_points(mode):
     tr.track_from(np.linalg.inv(init))
     assert np.allclose(tr.trel().astype(np.float64), init.astype(np.float32), atol=1e-6)
     assert np.all(tr.debug_read("ICP_COUNT", 0, np.int32, 4)[:3] == 0)
+
+
+def test_infinite_and_huge_depths_of_a_float_frame():
+    """A float depth map may hold infinities: their points are IEEE's
+    quotients, infinite or not a number as (x - cx) z / fx is. A depth whose
+    squared residual overflows at the selection gives its point the weight 0
+    from then on."""
+    print("case infinite depths", flush=True)
+    p = _pair(7)
+    cal = p["calib"]
+    KL, mn, mx = 43, float(cal[62]), float(cal[63])
+    g0, d0, g1, d1 = p["host"]
+    def rgbd(z):
+        out = np.full((H, W, 4), 0.5, np.float32)
+        out[..., 3] = (z.astype(np.float32) - mn) / (mx - mn)
+        return np.ascontiguousarray(out[::-1])
+    tr = PhotoTracker(W, H, cal, mode=GEOMETRIC, n_select=N)
+    tr.set_reference_points(g0, d0, mode=GEOMETRIC, force=True)
+    z = np.where(d1 > 0, d1, 1000).astype(np.float32)
+    z[40:60, 100:220] = np.inf
+    z[100:110, :] = np.float32(3e38)
+    tr.set_current_rgbd(rgbd(z))
+    tr.debug_prepare()
+    got = tr.debug_read("CUR_CLOUD", 0, np.float32, 4 * W * H).reshape(H, W, 4)
+    with np.errstate(all="ignore"):
+        zz = -(rgbd(z)[::-1][..., 3] * np.float32(np.float32(mx) - np.float32(mn)) + np.float32(mn))
+        yy, xx = np.mgrid[0:H, 0:W].astype(np.float32)
+        X = (xx - cal[KL + 2]) * zz / cal[KL]
+        Y = (yy - cal[KL + 5]) * zz / cal[KL + 4]
+    assert np.isinf(X).any() and np.isinf(zz).any()
+    assert np.array_equal(got[..., 2], zz) and np.all(got[..., 3] == 1)
+    assert np.array_equal(got[..., 0], X, equal_nan=True) and np.array_equal(got[..., 1], Y, equal_nan=True)
+    # every selected residual's square infinite, then a finite frame: no weight, no system
+    tr.set_current_rgbd(rgbd(np.full((H, W), 1e25, np.float32)))
+    tr.debug_prepare()
+    tr.debug_set_trel(np.eye(4))
+    tr.debug_linearize(0, 0)
+    n = int(tr.debug_read("ICP_COUNT", 0, np.int32, 4)[0])
+    assert n > 1024 and np.all(np.isinf(tr.debug_read("ICP_R2", 0, np.float32, W * H)[:n]))
+    tr.set_current_image(g1, d1)
+    tr.debug_prepare()
+    _, (A, b) = tr.debug_linearize(0, 1)
+    assert not A.any() and not b.any()
