@@ -585,8 +585,7 @@ __device__ __forceinline__ void normalize_mat4_safe_regs(double* T) {
     T[1] = v[0]; T[5] = v[1]; T[9] = v[2];
     T[2] = w[0]; T[6] = w[1]; T[10] = w[2];
 }
-// TI: the pose before the update, TO: where it is stored (may be the same)
-__device__ __forceinline__ void expm_update_regs(const double* x, const float* TI, float* TO, double scale, bool writer) {
+__device__ __forceinline__ void expm_update_regs(const double* x, float* T, double scale, bool writer) {
     double Ti[12];  // rows 0-2 of the increment; row 3 is 0 0 0 1
     double mx = 0;
 #pragma unroll
@@ -627,7 +626,7 @@ __device__ __forceinline__ void expm_update_regs(const double* x, const float* T
     double R[12];
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        const double t0 = TI[i * 4 + 0], t1 = TI[i * 4 + 1], t2 = TI[i * 4 + 2], t3 = TI[i * 4 + 3];
+        const double t0 = T[i * 4 + 0], t1 = T[i * 4 + 1], t2 = T[i * 4 + 2], t3 = T[i * 4 + 3];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             R[i * 4 + j] = t0 * Ti[0 * 4 + j] + t1 * Ti[1 * 4 + j] + t2 * Ti[2 * 4 + j];
@@ -635,7 +634,7 @@ __device__ __forceinline__ void expm_update_regs(const double* x, const float* T
         }
     }
     // the last row of a pose is 0 0 0 1 and stays so; another one is multiplied out
-    float b3[4] = {TI[12], TI[13], TI[14], TI[15]};
+    float b3[4] = {T[12], T[13], T[14], T[15]};
     if (b3[0] != 0.0f || b3[1] != 0.0f || b3[2] != 0.0f || b3[3] != 1.0f) {
         const double t0 = b3[0], t1 = b3[1], t2 = b3[2], t3 = b3[3];
 #pragma unroll
@@ -645,9 +644,9 @@ __device__ __forceinline__ void expm_update_regs(const double* x, const float* T
     normalize_mat4_safe_regs(R);
     if (writer) {
 #pragma unroll
-        for (int i = 0; i < 12; i++) TO[i] = (float)R[i];
+        for (int i = 0; i < 12; i++) T[i] = (float)R[i];
 #pragma unroll
-        for (int i = 0; i < 4; i++) TO[12 + i] = b3[i];
+        for (int i = 0; i < 4; i++) T[12 + i] = b3[i];
     }
 }
 
@@ -668,22 +667,15 @@ __device__ __forceinline__ double lane_bcast(double v, int src) {
 // the same operations), and every entry is computed by the same operations in
 // the same order as in solve_cholesky, so the result is the same bit for bit;
 // the exponential update runs in every lane's registers and lane 0 stores the
-// pose from TI to TO (the same array unless TO is given). The CG solver runs
-// solve_update on lane 0. The return value is meaningful in lane 0. Bound by
-// its serial chain of FP64 operations: 1,158 of them with a separate forward
-// substitution and every structural zero multiplied out, 710 now.
-__device__ bool solve_update_wave(const double* sys, float* TI, const SolveCfg& cfg, int N1, int N2, double* w,
-                                  float* TO = nullptr) {
+// pose in place. The CG solver runs solve_update on lane 0. The return value is
+// meaningful in lane 0. Bound by its serial chain of FP64 operations: 1,158 of
+// them with a separate forward substitution and every structural zero
+// multiplied out, 710 now.
+__device__ bool solve_update_wave(const double* sys, float* T, const SolveCfg& cfg, int N1, int N2, double* w) {
     const int lane = lane_id();
-    if (!TO) TO = TI;
     if (cfg.solver != 0) {
         bool ok = true;
-        if (lane == 0) {
-            float T[16];
-            for (int i = 0; i < 16; i++) T[i] = TI[i];
-            ok = solve_update(sys, T, cfg, N1, N2, w);
-            for (int i = 0; i < 16; i++) TO[i] = T[i];
-        }
+        if (lane == 0) ok = solve_update(sys, T, cfg, N1, N2, w);
         return ok;
     }
     const int r = lane < 6 ? lane : 6;
@@ -732,7 +724,7 @@ __device__ bool solve_update_wave(const double* sys, float* TI, const SolveCfg& 
             x[i] = div_rn64(t, lane_bcast(diag, i), lane_bcast(inv, i));
         }
     }
-    expm_update_regs(x, TI, TO, (double)cfg.scale_out, lane == 0);
+    expm_update_regs(x, T, (double)cfg.scale_out, lane == 0);
     return ok;
 }
 
