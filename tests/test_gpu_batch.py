@@ -115,6 +115,31 @@ def test_batch_preparation_bitexact_against_oracle(N, rig):
             assert np.array_equal(jac[6 * N:], rec[:, color_slot[l]]), f"reference gray pair {i} level {l}"
 
 
+def test_selection_is_the_same_in_every_split():
+    """The selection of a pair runs on 16 to 1 workgroups by the number of
+    pairs (2048 / pairs, a power of two); past 1024 pairs one workgroup counts
+    and scatters. Pairs at both ends of each batch against the eight-pair
+    batch, whose selection the oracle gives."""
+    print("case selection splits", flush=True)
+    from tests._oracle_steps import Steps
+    N, kinds, most = 768, 4, 1032
+    base, host = [], []
+    for i in range(kinds):
+        g0, d0, g1, d1, _ = synth.make_pair(700 + i, 160, 120, 2.0, 30.0)
+        bufs = [DeviceBuffer.from_array(a) for a in (g0, d0, g1, d1)]
+        host.append((g0, d0, g1, d1, bufs))
+        base.append(dict(ref_gray=bufs[0].ptr, ref_depth=bufs[1].ptr, cur_gray=bufs[2].ptr, cur_depth=bufs[3].ptr,
+                         width=160, height=120, calib=synth.calib_block_np(160, 120)))
+    want = []
+    for p, (g0, d0, g1, d1, _) in zip(base, host):
+        want.append(Steps(160, 120, 3, p["calib"], g0, d0, g1, d1, nselect=N, dtype=np.float32).features().sel)
+    bt = BatchTracker(most, 160, 120, mode=PHOTOMETRIC, n_select=N)
+    for n in (8, 128, 129, 256, 257, 512, 513, 1024, 1025, most):
+        bt.prepare_only(bt.prepare([base[i % kinds] for i in range(n)]))
+        for i in list(range(kinds)) + [n // 2] + list(range(n - kinds, n)):
+            assert np.array_equal(bt.debug_read(i, "SELECTED", 0, np.int32, N), want[i % kinds]), (n, i)
+
+
 @pytest.mark.parametrize("N,iters", [(8192, (1, 3, 10, 5)), (12288, (0, 3, 4, 2))])
 def test_batch_kernel_variants_agree(N, iters, monkeypatch, capfd):
     """Every variant of the persistent kernel the autotuner may pick, forced one

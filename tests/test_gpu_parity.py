@@ -86,6 +86,33 @@ def test_selection_bitexact(W, H, L, N, seed, calib):
     assert np.array_equal(tr.debug_read("SELECTED", 0, np.int32, N), st.sel)
 
 
+@pytest.mark.parametrize("W,H,N,seed", [(160, 360, 1536, 1), (160, 360, 256, 8), (128, 96, 1024, 8), (352, 464, 2816, 1)])
+def test_selection_whose_trim_passes_the_first_segments(W, H, N, seed):
+    """Narrow and small images with few points: the trim of the equal bins runs
+    past the first 64 of the 512 segments (61 at 352x464), which several waves
+    of the scan hold. Single pair and batch."""
+    print(f"case selection trim {W}x{H} N {N} seed {seed}", flush=True)
+    from recon_amd.hip import DeviceBuffer
+    from recon_amd.tracker import BatchTracker
+    tr, st, _ = _setup(W, H, 3, N, seed)
+    tr.debug_prepare()
+    st.features()
+    per = W * H // 512
+    bins = np.floor(st.gmag[:512 * per].astype(np.float64) * 255 + 0.5).reshape(512, per)  # grad_bin but for ties
+    equal, left, last = (bins == st.thr).sum(1), st.excess, -1
+    for j in np.nonzero(equal[:511])[0]:
+        if left > 0:
+            last, left = j, (0 if equal[j] >= left else equal[j])
+    assert last > 60
+    assert np.array_equal(tr.debug_read("SELECTED", 0, np.int32, N), st.sel)
+    bufs = [DeviceBuffer.from_array(a) for a in _pair(W, H, seed)[:4]]
+    pair = dict(ref_gray=bufs[0].ptr, ref_depth=bufs[1].ptr, cur_gray=bufs[2].ptr, cur_depth=bufs[3].ptr, width=W,
+                height=H, calib=CALIBS["pinhole"](W, H))
+    bt = BatchTracker(1, W, H, mode=PHOTOMETRIC, n_select=N)
+    bt.prepare_only(bt.prepare([pair]))
+    assert np.array_equal(bt.debug_read(0, "SELECTED", 0, np.int32, N), st.sel)
+
+
 @pytest.mark.parametrize("W,H,L,N,seed,calib", [c + ("pinhole",) for c in CASES] + [c + ("rig",) for c in RIG_CASES])
 def test_points_and_jacobians_bitexact(W, H, L, N, seed, calib):
     print(f"case jacobians {W}x{H} seed {seed} {calib}", flush=True)
