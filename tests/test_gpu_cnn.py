@@ -73,6 +73,36 @@ def test_forward_matches_oracle(kw, B):
     assert np.abs(out - ref).max() <= 2e-3 * scale, (out, ref)
 
 
+# The fused first layers: a workgroup per CU takes samples in turn between two
+# maps, so only more samples than twice the CUs alternate them; odd maps end
+# inside a row tile.
+@pytest.mark.parametrize("kw", [{}, dict(channels=[4, 32, 64, 128, 32, 64, 32], in_width=21, in_height=13),
+                                dict(channels=[4, 32, 64, 16, 16, 128, 64], in_width=35, in_height=50)])
+def test_forward_of_many_samples_equals_small_batches(kw):
+    """600 samples at once, those of batches of 60 bit for bit (every layer
+    adds in the same order whatever its tile), and the oracle's for the last
+    ones."""
+    print(f"case cnn forward {kw} B=600", flush=True)
+    from recon_amd.hip import hip
+    B, part = 600, 60
+    cfg = default_config(**kw)
+    net = PoseNet(B, config=cfg)
+    p, xr, xb, y, wn = case(cfg, B, 3)
+    net.set_params(p)
+    xd, od = DeviceBuffer.from_array(xb), DeviceBuffer(24 * B)
+
+    def run(n, first):
+        net.forward(n, xd.ptr + first * xb[0].nbytes, od.ptr)
+        hip().hipDeviceSynchronize()
+        return od.to_array(np.float32, 6 * n).reshape(n, 6)
+
+    out = run(B, 0)
+    for first in range(0, B, part):
+        assert np.array_equal(out[first:first + part], run(part, first)), first
+    _, ref, _ = oracle_fb(cfg, p, xr[-4:], y[-4:], wn[-4:], grad=False)
+    assert np.abs(out[-4:] - ref).max() <= 2e-3 * max(1.0, float(np.abs(ref).max()))
+
+
 @pytest.mark.parametrize("kw,B", [({}, 3), (SMALL, 5)])
 def test_gradients_match_oracle(kw, B):
     print(f"case cnn gradients {kw} B={B}", flush=True)
