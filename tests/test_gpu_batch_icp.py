@@ -1,5 +1,4 @@
-"""Batched geometric and bi-objective tracking (kb_track with the ICP terms)
-against the single-pair tracker and the oracle, on a mixed-size batch
+"""Batched geometric and bi-objective tracking (the lockstep launches) against the single-pair tracker and the oracle, on a mixed-size batch
 (160x120 .. 640x480).
 
 - The batch's keyframe and current clouds of every level equal the FP32
@@ -89,6 +88,34 @@ def test_batch_icp_matches_single_and_oracle(mode):
               f"{et[1]:.2f} mm; ICP points {list(cnt[:L])}", flush=True)
         assert np.radians(es[0]) < 1e-5 and es[1] < 1e-2, i
         assert np.radians(e32[0]) < 1e-5 and e32[1] < 1e-2, i
+    bt.close()
+
+
+@pytest.mark.parametrize("mode,W,H,L,N", [(GEOMETRIC, 904, 580, 3, 2048), (BIOBJECTIVE, 904, 580, 3, 8192),
+                                          (BIOBJECTIVE, 320, 240, 3, 16384), (BIOBJECTIVE, 192, 144, 2, 256),
+                                          (GEOMETRIC, 192, 144, 1, 256)])
+def test_batch_icp_at_the_ends_of_its_sizes(mode, W, H, L, N):
+    """The most pixels of a pair (513 blocks of 1024), more points than a
+    round's 8192, few points and levels: three pairs against the FP32 oracle
+    from the same start."""
+    print(f"case batch icp mode {mode} {W}x{H} levels {L} N {N}", flush=True)
+    iters = (2, 4, 3, 0)
+    pairs, host = [], []
+    for i in range(3):
+        g0, d0, g1, d1, Tgt = synth.make_pair(1400 + i, W, H, 3.0, 50.0)
+        bufs = [DeviceBuffer.from_array(a) for a in (g0, d0, g1, d1)]
+        host.append((g0, d0, g1, d1, bufs, synth.sample_motion(7000 + i, 1.0, 15.0) @ Tgt))
+        pairs.append(dict(ref_gray=bufs[0].ptr, ref_depth=bufs[1].ptr, cur_gray=bufs[2].ptr, cur_depth=bufs[3].ptr,
+                          width=W, height=H, calib=synth.calib_block_np(W, H)))
+    bt = BatchTracker(3, W, H, mode=mode, n_select=N, iters=iters, lam=0.5, levels=L)
+    Trel, _, rms, st = bt.track(pairs, init=[h[5] for h in host])
+    assert np.all(st == 0)
+    for i, (g0, d0, g1, d1, _, init) in enumerate(host):
+        ot = oracle.Tracker(W, H, pairs[i]["calib"], mode=mode, levels=L, iters=iters, nselect=N, lam=0.5, dtype=np.float32)
+        ot.set_reference(g0, d0); ot.set_current(g1, d1); ot.prepare(); ot.set_trel(init); ot.track()
+        e = synth.pose_error(Trel[i], ot.poses()[0])
+        print(f"  pair {i}: vs FP32 oracle {e[0]:.2e} deg {e[1]:.2e} mm", flush=True)
+        assert np.radians(e[0]) < 1e-5 and e[1] < 1e-2, i
     bt.close()
 
 

@@ -159,3 +159,90 @@ def test_sign_map_and_slice_cull_at_tile_edges_bitexact(res, dim, W, H):
     dst.integrate(ramp, inside, K)
     odst.update(ramp.astype(np.float32), inside, K)
     check(dst, odst, "fused after resampling", views[:3])
+
+
+def _fused(res, zs, depth, Tcur, K, W, H):
+    """One frame fused into the slices zs of a new grid (updateVoxelsKernel in
+    float32, every voxel projected): (len(zs), res, res, 2)."""
+    f = np.float32
+    org, dim = np.array(ORIGIN, f), np.array(DIM, f)
+    vs = dim / f(res)
+    start, edge = (org - dim) + vs, vs * f(2)
+    R, t = np.asarray(Tcur, f)[:3, :3], np.asarray(Tcur, f)[:3, 3]
+    i = np.arange(res, dtype=f)
+    px, py = (start[0] + i * edge[0])[None, None, :], (start[1] + i * edge[1])[None, :, None]
+    pz = (start[2] + np.asarray(zs, f) * edge[2])[:, None, None]
+    r = [R[0, k] * px + R[1, k] * py + R[2, k] * pz + -(R[0, k] * t[0] + R[1, k] * t[1] + R[2, k] * t[2]) for k in range(3)]
+    dist, vox = np.asarray(depth, f), -r[2]
+    with np.errstate(all="ignore"):
+        u = (r[0] / r[2] * K[0] + K[2]) * f(W)
+        v = (r[1] / r[2] * K[4] + K[5]) * f(H)
+        ok = (u >= 1) & (u < W - 2) & (v >= 1) & (v < H - 2)
+    u, v = np.where(ok, u, f(1)), np.where(ok, v, f(1))
+    ui, vi = u.astype(np.int32), v.astype(np.int32)
+    m = [dist[vi + b, ui + a] for b in (0, 1) for a in (0, 1)]
+    fu, fv = u - ui.astype(f), v - vi.astype(f)
+    d = (1 - fu) * (1 - fv) * m[0] + fu * (1 - fv) * m[1] + (1 - fu) * fv * m[2] + fu * fv * m[3]
+    for k in m:
+        ok &= (k >= edge[0]) & (np.abs(d - k) <= dim[0] / f(200))
+    sdf = -(vox - d) / (dim[0] * f(0.030))
+    ok &= sdf >= f(-1.25)
+    out = np.empty(ok.shape + (2,), f)
+    out[..., 0] = np.where(ok, np.clip(sdf, f(-1), f(1)), f(1))
+    out[..., 1] = ok
+    return out
+
+
+def test_slice_cull_at_1024_voxels_an_axis():
+    """The largest grid, whose oracle would not fit the host: chosen slices
+    against every voxel's own projection in numpy, which equals the oracle on a
+    small grid."""
+    from recon_amd import lib
+    from recon_amd.hip import hip
+    W, H, res = 160, 120, 1024
+    K = normalized_k(W, H)
+    print(f"tsdf grid res={res} image={W}x{H}", flush=True)
+    views = [pose(), pose(7, -11, (80, -20, 30)), pose(3, 100, (200, 30, -1500)), pose(0, 180, (0, 0, -3600))]
+    for T in views:
+        d = np.round(render_depth(T, K, W, H)).astype(np.uint16)
+        o = Grid(40, W, H, ORIGIN, DIM)
+        o.update(d.astype(np.float32), T, K)
+        assert _bits_equal(_fused(40, np.arange(40), d, T, K, W, H), o.data)
+    g = VoxelGrid(default_params(resolution=res, width=W, height=H))
+    buf, hit = np.empty((res, res, 2), np.float32), 0
+    for T in views:
+        d = np.round(render_depth(T, K, W, H)).astype(np.uint16)
+        g.reset()
+        g.integrate(d, T, K)
+        g.synchronize()
+        for z in (0, 15, 16, 511, 640, 1023):
+            assert hip().hipMemcpy(buf.ctypes.data, lib().rt_tsdf_data(g.h) + z * buf.nbytes, buf.nbytes, 2) == 0
+            want = _fused(res, [z], d, T, K, W, H)[0]
+            hit += int(want[..., 1].sum())
+            assert _bits_equal(buf, want), z
+    assert hit > 500000
+    g.close()
+
+
+def test_poses_that_are_not_finite_bitexact():
+    """Poses and projections that are infinite, huge or not a number: voxels
+    whose projection leaves the image stay as they are, and no slice is culled
+    that the update would change."""
+    W, H, res = 64, 48, 40
+    K = normalized_k(W, H)
+    d = np.full((H, W), 1500, np.uint16)
+    bad = []
+    for i, x in ((3, np.nan), (3, np.inf), (11, np.inf), (11, -np.inf), (0, np.nan), (10, np.inf), (7, 1e30), (11, 3e38),
+                 (0, 1e38)):
+        T = pose(3, 5, (10, 20, 30)).ravel()
+        T[i] = x
+        bad.append((i, x, T.reshape(4, 4)))
+    for i, x, T in bad:
+        g, o = _grids(res, W, H)
+        g.integrate(d, pose(), K)
+        o.update(d.astype(np.float32), pose(), K)
+        with np.errstate(all="ignore"):
+            g.integrate(d, T, K)
+            o.update(d.astype(np.float32), T, K)
+        a, b = g.read(), o.data
+        assert np.array_equal(a, b, equal_nan=True), (i, x)
