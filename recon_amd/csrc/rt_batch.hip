@@ -871,14 +871,16 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
 // one workgroup: 64 pairs of 320x240 took 4.05 ms on 64 of the 256 CUs) and the
 // small photometric batches, which would leave most CUs idle.
 //
-// The sums are those of a 1024-thread workgroup of kb_track, bit for bit:
-// virtual lane (wave v of 16, lane l) adds its points 64 v + l + 1024 j in
-// order of j in FP32, the 64 lanes of a wave meet in the exchange order
-// 32, 16, ..., 1, and the 16 waves add in order in FP64. A workgroup of 8
-// waves is one virtual wave: in each round wave w forms the terms' factors of
-// the points j = 8 round + w (one per lane) and leaves them in LDS, and after
-// a barrier four of the waves add eight terms each over the round's eight j, so
-// that the points are formed by eight waves while each sum stays one chain.
+// The sums are those of a 1024-thread workgroup: the photometric ones equal
+// kb_track's bit for bit, the geometric ones follow the same order. Virtual
+// lane (wave v of 16, lane l) adds its points 64 v + l + 1024 j in order of j in
+// FP32, the 64 lanes of a wave meet in the exchange order 32, 16, ..., 1, and
+// the 16 waves add in order in FP64. A workgroup of 8 waves is one virtual wave:
+// in each round wave w forms the terms' factors of the points j = 8 round + w
+// (one per lane) and leaves them in LDS, and after a barrier four of the waves
+// add eight terms each over the round's eight j, so that the points are formed
+// by eight waves while each sum stays one chain.
+
 // Most pixels of a pair (build_batch refuses more: whole segments of its 512 in
 // the selection hold up to 1024 pixels), and their blocks of 1024.
 constexpr int MAX_PIXELS = 512 * 1025 - 1, LK_BLOCKS = (MAX_PIXELS + 1023) / 1024;

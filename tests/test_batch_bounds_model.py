@@ -2,10 +2,11 @@
 
 The library's own descriptor builder (rt_batch_layout: the code rt_batch_prepare
 runs, reporting offsets instead of touching a device) places every pair's
-buffers in the arena; this model replays the launch grids of the preparation
-and tracking launches (launch_prep, launch_track in rt_batch.hip) for those
-descriptors and forms every index the kernels form, from their code, asserting
-that each lies inside its buffer. It runs on the 256-pair mixed-size batch of
+buffers in the arena, and rt_batch_lock_layout places the lockstep launches'
+arrays; this model replays the launch grids of the preparation and tracking
+launches (launch_prep, launch_track, launch_lockstep in rt_batch.hip) for them
+and forms the indices the kernels form, from their code, asserting that each
+lies inside its buffer. It runs on the 256-pair mixed-size batch of
 the mixed-size workload (160x120 .. 640x480, 8192 points), the 4096-pair
 640x480 batch of the headline and small mixed batches."""
 import ctypes
@@ -194,16 +195,39 @@ def _kb_bins(W, H, maxW, maxH):
     return out
 
 
-def _kb_select(W, H, N):
+SEL_WAVES, SEL_U = 8, 2
+
+
+def _select_parts(n):
+    parts = 1
+    while parts < 16 and 2 * parts * n <= 2048:
+        parts *= 2
+    return parts
+
+
+def _kb_select(W, H, N, n):
     npix = W * H
     Pn = npix // 512
     assert Pn >= 1 and (Pn * 512) <= npix
+    # the segments that the workgroups of a pair count and scatter: each of the
+    # 512 once (wave + 16 k + 8 u inside a workgroup's range)
+    parts = _select_parts(n)
+    per = 512 // parts
+    g, wave, k, u = np.meshgrid(np.arange(parts), np.arange(SEL_WAVES), np.arange(0, per, SEL_WAVES * SEL_U),
+                                np.arange(SEL_U), indexing="ij")
+    live = wave + k < per                                   # the loops' condition, before u is added
+    seg = (per * g + wave + k + SEL_WAVES * u)[live]
+    assert np.array_equal(np.sort(seg), np.arange(512))
+    # packed counts: both below 2^16; split, they wait in the pair's points (512 words)
+    assert Pn < 1 << 16
+    out = {"counts": 4 * 511 + 3 if parts > 1 else -1}
     # last byte a segment load may touch: clamped to the segment's last byte
     # (byte path) or an 8-byte load at min(base, end - 8) (only when Pn % 8 == 0)
     last = 512 * Pn - 1
     if Pn % 8 == 0:
         assert Pn >= 8
-    return {"bins": last, "sel": N - 1}
+    out.update(bins=last, sel=N - 1)
+    return out
 
 
 def _ref_points_blocks(n, chunks):
@@ -215,6 +239,12 @@ def _ref_points_blocks(n, chunks):
     assert np.all(pair % 8 == b % 8)
     live = pair < n
     return pair[live], chunk[live]
+
+
+@pytest.mark.parametrize("n", [1, 2, 64, 128, 129, 256, 257, 512, 513, 1024, 1025, 4096])
+def test_selection_splits_cover_each_segment_once(n):
+    """Any number of pairs, at the fewest points (whose records hold the counts)."""
+    assert _kb_select(160, 120, 256, n)["counts"] < 16 * 256
 
 
 @pytest.mark.parametrize("n,chunks", [(1, 1), (3, 32), (8, 32), (13, 7), (4096, 32), (257, 5)])
@@ -250,27 +280,38 @@ def _kb_track(W, H, L, N, maxN, pc):
 
 
 def _geometric(W, H, L):
-    """kb_clouds, kb_clouds_down and the geometric terms of kb_track: largest
-    element index per buffer (float4 clouds, isel / ir2)."""
+    """kb_clouds and the ICP terms: largest element index per buffer (float4
+    clouds, isel / ir2)."""
     out = {}
     # kb_clouds: 16x16 pixel tiles; the normal's four neighbours only for
     # 1 <= x <= W - 2, 1 <= y <= H - 2
     out["depth"] = max((W - 1) + (H - 1) * W, (W - 2 + 1) + (H - 2) * W, (W - 2) + (H - 2 + 1) * W)
     out["cloud0"] = W * H - 1
+    # cloud_tile_levels: level l of a tile from level l - 1 in LDS (256 + 64 + 16
+    # + 4 records), stored inside the level's image; a pixel's four taps lie in
+    # the tile and, the sizes being multiples of 2^(L-1), in the image
+    src, dst = 0, 256
     for l in range(1, L):
-        Wd, Hd = W >> l, H >> l
-        assert (W >> (l - 1)) == 2 * Wd and (H >> (l - 1)) == 2 * Hd
-        i = Wd * Hd - 1
-        x, y = i % Wd, i // Wd
-        src = x * 2 + 1 + (y * 2 + 1) * 2 * Wd              # the last 2x2 source tap
-        out[f"down{l}"] = (src, (W >> (l - 1)) * (H >> (l - 1)) - 1)
+        Wl, Hl, side = W >> l, H >> l, 16 >> l
+        assert (W >> (l - 1)) == 2 * Wl and (H >> (l - 1)) == 2 * Hl
+        t = np.arange(side * side)
+        x, y = t & (side - 1), t // side
+        o = src + 2 * x + 4 * y * side
+        taps = np.stack([o, o + 1, o + 2 * side, o + 2 * side + 1])
+        assert taps.min() >= src and taps.max() < dst and np.unique(taps).size == 4 * t.size
+        assert dst + t.max() < 256 + 64 + 16 + 4
+        gx = (np.arange((W + 15) // 16)[:, None] * side + np.arange(side)[None, :]).ravel()
+        gy = (np.arange((H + 15) // 16)[:, None] * side + np.arange(side)[None, :]).ravel()
+        gx, gy = gx[gx < Wl], gy[gy < Hl]
+        assert np.array_equal(gx, np.arange(Wl)) and np.array_equal(gy, np.arange(Hl))     # every pixel once
+        out[f"level{l}"] = (gx.max() + gy.max() * Wl, Wl * Hl - 1)
+        src, dst = dst, dst + side * side
     for l in range(L):
         w, h = W >> l, H >> l
         # mask / system taps: 0 <= xdi < w - 1, 0 <= ydi < h - 1, taps o2 .. o2 + w + 1
         out[f"taps{l}"] = ((w - 2) + (h - 2) * w + w + 1, w * h - 1)
         out[f"isel{l}"] = (w * h - 1, W * H - 1)               # at most w*h selected points
-    # the Student-t block sums: n <= W*H <= 512 * 1024 -> at most 512 blocks
-    out["bsum"] = ((W * H + 1023) // 1024, 512)
+        assert w * h < 1 << 28                                 # 32-bit byte offsets of the records (ldo)
     return out
 
 
@@ -292,8 +333,8 @@ def _check_kernels(f, maxes, max_w, max_h, pcs=(0, 5120, 5632, 8192)):
         for k, v in bins.items():
             if k.startswith("gray_") and k != "gray_taps" and int(k[5:]) < L:
                 assert v < bufsz[k], (p, "kb_bins", k, v)
-        sel = _kb_select(W, H, N)
-        assert sel["bins"] < W * H and sel["sel"] < N
+        sel = _kb_select(W, H, N, len(f))
+        assert sel["bins"] < W * H and sel["sel"] < N and sel["counts"] < 16 * N
         ref = _kb_ref_points(W, H, L, N)
         for k, v in ref.items():
             if k.startswith("gray_"):
@@ -338,6 +379,7 @@ def _check_lockstep(W, H, L, N, off, mode):
             used["rfull"] = max(used.get("rfull", 0), 4 * (npix - 1))
             for r in range(3):                          # a block sum per 1024 of at most npix points
                 used[f"bsum{r}"] = max(used.get(f"bsum{r}", 0), 4 * (blocks - 1))
+    # kl_terms' grid is kb_ref_points': _ref_points_blocks' test covers it
     for k, last in used.items():
         elem = 8 if k == "bits" else 4
         assert off[k] % (8 if k in ("bits", "rz") else 4) == 0
