@@ -655,21 +655,36 @@ struct TrackCfg {
 };
 
 
-// The solve of one pair's photometric system as a call (on wave 0). Inlined,
-// its FP64 registers exceed the 128 per lane that a 1024-thread workgroup
-// leaves, and 70 of the passes' registers were spilled around it by every
-// wave; 10 with the call, whose cost only wave 0 pays: 6.39 -> 6.32 ms for 4096
-// pairs of 640 x 480 with 8192 points, 360 -> 355 us for 64. (The registers
-// that this frees do not hold a level's Jacobians: kept there, eight points a
-// thread, the passes spill again, 7.3 to 7.9 ms.)
+// The solve of one pair's photometric system on wave 0, inline or as a call
+// (CALL). Inlined, its FP64 registers exceed the 128 per lane that a 1024-thread
+// workgroup leaves, and 70 of the passes' registers are spilled around it by
+// every wave; 10 with the call, whose cost only wave 0 pays. The kernels with
+// residuals in LDS and 512 or 1024 threads call it (640x480 and 8192 points, us
+// inline and called: 4096 pairs 6520 and 6400, 256 pairs 451 and 435). Those with
+// residuals in registers spill these around the call instead (256 pairs of
+// 12288 points 1064 and 1080, 48 pairs 746 and 782), and 256 threads have the
+// registers (512 pairs of 320x240 with 1024 points 178 and 188): inline. (The
+// registers that the call frees do not hold a level's Jacobians: kept there,
+// eight points a thread, the passes spill again, 7.3 to 7.9 ms.)
 #define RT_LDS __attribute__((address_space(3)))
-__device__ __attribute__((noinline)) bool solve_photo(RT_LDS double* sys, RT_LDS float* T, RT_LDS double* ws, int solver,
-                                                      int robust, int mad_bins, float scale_out, int N) {
+__device__ __forceinline__ bool solve_photo_body(RT_LDS double* sys, RT_LDS float* T, RT_LDS double* ws, int solver,
+                                                 int robust, int mad_bins, float scale_out, int N) {
     SolveCfg sc;
     sc.solver = __builtin_amdgcn_readfirstlane(solver);
     sc.mode = RT_PHOTOMETRIC; sc.lambda = 0.0f; sc.scale_out = scale_out;
     sc.robust = robust; sc.mad_bins = mad_bins; sc.scale_in = 1e-3f;
     return solve_update_wave((const double*)sys, (float*)T, sc, N, 0, (double*)ws);
+}
+__device__ __attribute__((noinline)) bool solve_photo_call(RT_LDS double* sys, RT_LDS float* T, RT_LDS double* ws,
+                                                           int solver, int robust, int mad_bins, float scale_out, int N) {
+    return solve_photo_body(sys, T, ws, solver, robust, mad_bins, scale_out, N);
+}
+constexpr bool solve_is_call(int bs, int ppt, int rz) { return rz && bs >= 512; }
+template <bool CALL>
+__device__ __forceinline__ bool solve_photo(RT_LDS double* sys, RT_LDS float* T, RT_LDS double* ws, int solver,
+                                            int robust, int mad_bins, float scale_out, int N) {
+    if constexpr (CALL) return solve_photo_call(sys, T, ws, solver, robust, mad_bins, scale_out, N);
+    else return solve_photo_body(sys, T, ws, solver, robust, mad_bins, scale_out, N);
 }
 
 // RZ: residual and zWeight of each point kept in registers (0) or in LDS (1,
@@ -848,8 +863,9 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
                 }
                 __syncthreads();
                 if (wave == 0) {
-                    const bool ok = solve_photo((RT_LDS double*)sys, (RT_LDS float*)T, (RT_LDS double*)ws, cfg.solver,
-                                                cfg.robust, cfg.mad_bins, cfg.scale_out, N);
+                    const bool ok = solve_photo<solve_is_call(BS, PPT, RZ)>(
+                        (RT_LDS double*)sys, (RT_LDS float*)T, (RT_LDS double*)ws, cfg.solver, cfg.robust, cfg.mad_bins,
+                        cfg.scale_out, N);
                     if (t == 0) {
                         if (!ok) s_ok = 0;
                         rms_last = sys[28] > 0.0 ? (float)sqrt(sys[27] / sys[28]) : 0.0f;
