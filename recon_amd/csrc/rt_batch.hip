@@ -11,9 +11,10 @@
 // wave and combined across waves in FP64, and one wave runs the FP64 solve and
 // SE(3) update. Workgroup size and points per thread are template parameters
 // picked per batch by a timing autotuner; the pipeline is captured once into a
-// hipGraph and replayed. Geometric and bi-objective batches, and small
-// photometric ones, track in lockstep instead: a few launches over all pairs
-// per iteration (launch_lockstep), with the same sums.
+// hipGraph and replayed. Geometric and bi-objective batches (but many pairs of
+// small images), and photometric ones of few pairs with many points, track in
+// lockstep instead: a few launches over all pairs per iteration
+// (launch_lockstep), with the same sums.
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include <math.h>
@@ -644,12 +645,118 @@ __device__ __forceinline__ void median_bin(const unsigned* hist, int N, int* med
     if (lane == 0) *med = m == (1 << 30) ? 0 : m;
 }
 
+// Most pixels of a pair (build_batch refuses more: whole segments of its 512 in
+// the selection hold up to 1024 pixels), and their blocks of 1024.
+constexpr int MAX_PIXELS = 512 * 1025 - 1, LK_BLOCKS = (MAX_PIXELS + 1023) / 1024;
+
+// ------------------------------------------------------------------ geometric terms in one workgroup
+// ICP selection of one level (icpResidualKernel2 + selectValidIndex +
+// packIndex, rgb2gray.cu:223-260,827-850): ordered compaction of the valid
+// keyframe pixels into d.isel / d.ir2 (squared residual), BS pixels a step: a
+// ballot per wave, the waves' counts in LDS. Returns the count (the same in
+// every thread).
+template <int BS>
+__device__ int icp_select_wg(const PairDesc& d, int layer, const float* T, const float* c) {
+    constexpr int NW = BS / 64;
+    __shared__ int wc[NW];
+    const int t = threadIdx.x, wave = t >> 6, lane = lane_id();
+    const int w = d.W >> layer, h = d.H >> layer, npix = w * h;
+    const float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
+    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    int base = 0;
+    for (int o0 = 0; o0 < npix; o0 += BS) {
+        const int o = o0 + t;
+        float r = 0.0f;
+        const bool valid = o < npix && icp_mask_pixel(d.rpos[layer], d.rnrm[layer], d.cpos[layer], w, h, o, T, c, a, b, r);
+        const uint64_t bl = __ballot(valid);
+        if (lane == 0) wc[wave] = __popcll(bl);
+        __syncthreads();
+        int off = 0, tot = 0;
+#pragma unroll
+        for (int q = 0; q < NW; q++) {
+            off += q < wave ? wc[q] : 0;
+            tot += wc[q];
+        }
+        if (valid) {
+            const int k = base + off + __popcll(bl & lt);
+            gmem(d.isel)[k] = o;
+            gmem(d.ir2)[k] = r * r;
+        }
+        base += tot;
+        __syncthreads();
+    }
+    return base;
+}
+// generateStudentTWeights (rgb2gray.cu:470-568, 854-877) in one workgroup, one
+// wave per block of 1024 points. var: three values in LDS, unchanged when n = 0
+// (no solve follows then). n <= MAX_PIXELS.
+template <int BS>
+__device__ void student_t_wg(const float* __restrict__ r2, int n, float* var) {
+    __shared__ float bsum[LK_BLOCKS];
+    const int wave = threadIdx.x >> 6;
+    if (n <= 0) return;
+    const int nb = (n + 1023) / 1024;
+    for (int round = 1; round <= 3; round++) {
+        const float prev = round > 1 ? var[round - 2] : 0.0f;
+        for (int bk = wave; bk < nb; bk += BS / 64) {
+            const float s = wave_student_block(r2, bk, n, round, prev);
+            if (lane_id() == 0) bsum[bk] = s;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const float v = wave_student_total(bsum, nb, n);
+            if (lane_id() == 0) var[round - 1] = v;
+        }
+        __syncthreads();
+    }
+}
+// The geometric system of one iteration (icpResidualIndexKernel2,
+// rgb2gray.cu:323-390, and the 27 dot products): per thread in FP32 over its
+// points, per wave by halving exchanges, across waves in FP64 into sysg[27].
+template <int BS>
+__device__ void icp_system_wg(const PairDesc& d, int layer, int n, float v3, const float* T, const float* c,
+                              double (*wsum)[29], double* sysg) {
+    const int t = threadIdx.x, wave = t >> 6, lane = lane_id();
+    const int w = d.W >> layer, h = d.H >> layer;
+    const float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
+    const IcpWeight iw = icp_weight(v3, n);
+    float acc[27];
+#pragma unroll
+    for (int k = 0; k < 27; k++) acc[k] = 0.0f;
+    for (int i = t; i < n; i += BS) {
+        const int o = gmem(d.isel)[i];
+        float res, J[6];
+        icp_point_terms(ldo(d.rpos[layer], o), ldo(d.rnrm[layer], o), d.cpos[layer], w, h, gmem(d.ir2)[i], iw, T, c, a, b,
+                        1e-3f, res, J);
+        int q = 0;
+#pragma unroll
+        for (int r0 = 0; r0 < 6; r0++)
+#pragma unroll
+            for (int c0 = r0; c0 < 6; c0++) acc[q++] += J[r0] * J[c0];
+#pragma unroll
+        for (int r0 = 0; r0 < 6; r0++) acc[21 + r0] += J[r0] * res;
+    }
+    float v32[32];
+#pragma unroll
+    for (int k = 0; k < 32; k++) v32[k] = k < 27 ? acc[k] : 0.0f;
+    const float tot = wave_sum32(v32);
+    if ((lane & 1) == 0 && (lane >> 1) < 27) wsum[wave][lane >> 1] = (double)tot;
+    __syncthreads();
+    if (t < 27) {
+        double v = 0.0;
+        for (int w2 = 0; w2 < BS / 64; w2++) v += wsum[w2][t];
+        sysg[t] = v;
+    }
+    __syncthreads();
+}
+
 // ------------------------------------------------------------------ persistent tracking
 struct TrackCfg {
     int solver;
     int robust;
     int mad_bins;
     float scale_out;
+    float lambda;  // bi-objective weight of the geometric system (linearFuse)
     int pc_cap;  // point-cache capacity (points; PC variants)
     int rz_len;  // length of the RZ residual array (the batch's largest point count)
 };
@@ -703,11 +810,19 @@ constexpr int PC_MAX = 8192;
 // would overlap one pair's serial phases with the other's point passes, were
 // measured slower than one 1024-thread workgroup at 640x480: the kernel is
 // bound by memory traffic, not by those phases.
-template <int BS, int PPT, int RZ, int WPE = 1, int PC = 0>
+// MODE: the tracking mode (RT_GEOMETRIC 0, RT_PHOTOMETRIC 1, RT_BIOBJECTIVE 2).
+// The geometric modes add, per level, the ICP selection and Student-t weights
+// at its first iteration and the geometric system every iteration
+// (ShapeTracker::updateLinearSystem, shapetracker.cpp:357-382), fused with the
+// photometric one by linearFuse in the bi-objective mode (:392-394): for many
+// pairs of small images, where a workgroup per pair fills the chip (icp_variant).
+template <int BS, int PPT, int RZ, int WPE = 1, int PC = 0, int MODE = RT_PHOTOMETRIC>
 __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__ P, const int* __restrict__ order,
                                                     int npairs, int* queue, TrackCfg cfg) {
     constexpr int NW = BS / 64;
-    constexpr int NSYS = 29;  // 27 system terms | the two sums of the residual RMS
+    // system terms: photometric 27 | geometric 27 (geometric modes) | the two
+    // sums of the photometric residual RMS
+    constexpr int NSYS = MODE == RT_PHOTOMETRIC ? 29 : 56, RMS0 = NSYS - 2;
     __shared__ float cal[96];
     __shared__ float T[16];
     __shared__ unsigned hist[256];
@@ -716,6 +831,7 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
     __shared__ double ws[SOLVE_WS];
     __shared__ int s_pair, s_med;
     __shared__ int s_ok;
+    __shared__ float s_var[3];
     __shared__ float lut[256];
     // RZ: dynamic LDS after every static array, so that the static arrays keep
     // small addresses (immediate offsets from one base register)
@@ -753,12 +869,14 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
             const JacView jv = jac_view(d.jac[layer], N);
             const int wl = W >> layer, hl = H >> layer;
             const float a = 1.0f / (float)(1 << layer), b = 0.5f * (a - 1.0f);
+            int nicp = 1;  // ICP points of the level (geometric modes)
             for (int it = 0; it < nit; it++) {
                 for (int k = t; k < 256; k += BS) hist[k] = 0u;
                 float Tl[16];
 #pragma unroll
                 for (int k = 0; k < 16; k++) Tl[k] = uni(T[k]);
                 __syncthreads();
+              if constexpr (MODE != RT_GEOMETRIC) {
                 // residual pass: r and zWeight stay in registers (RZ 0) or go to LDS (RZ 1)
                 float r[RZ ? 1 : PPT], zw[RZ ? 1 : PPT];
                 auto residual = [&](int i, float& rr, float& zz) {
@@ -859,16 +977,39 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
                 if (t < 29) {
                     double v = 0.0;
                     for (int w2 = 0; w2 < NW; w2++) v += wsum[w2][t];
-                    sys[t] = v;
+                    sys[t < 27 ? t : RMS0 + t - 27] = v;
                 }
                 __syncthreads();
+              }
+                if constexpr (MODE != RT_PHOTOMETRIC) {
+                    // the level's ICP points and Student-t weights at its first
+                    // iteration (under the pose the iteration starts from)
+                    if (it == 0) {
+                        nicp = icp_select_wg<BS>(d, layer, Tl, cl);
+                        student_t_wg<BS>(d.ir2, nicp, s_var);
+                        if (t == 0) {
+                            d.icnt[layer] = nicp;
+                            for (int k = 0; k < 3; k++) d.ivar[layer * 3 + k] = nicp > 0 ? s_var[k] : 0.0f;
+                        }
+                    }
+                    icp_system_wg<BS>(d, layer, nicp, s_var[2], Tl, cl, wsum, sys + 27);
+                }
                 if (wave == 0) {
-                    const bool ok = solve_photo<solve_is_call(BS, PPT, RZ)>(
-                        (RT_LDS double*)sys, (RT_LDS float*)T, (RT_LDS double*)ws, cfg.solver, cfg.robust, cfg.mad_bins,
-                        cfg.scale_out, N);
+                    bool ok = true;
+                    if constexpr (MODE == RT_PHOTOMETRIC) {
+                        ok = solve_photo<solve_is_call(BS, PPT, RZ)>((RT_LDS double*)sys, (RT_LDS float*)T,
+                                                                     (RT_LDS double*)ws, cfg.solver, cfg.robust,
+                                                                     cfg.mad_bins, cfg.scale_out, N);
+                    } else if (nicp > 0) {  // no update from an empty geometric selection
+                        SolveCfg sc;
+                        sc.solver = cfg.solver; sc.mode = MODE; sc.lambda = cfg.lambda; sc.scale_out = cfg.scale_out;
+                        sc.robust = cfg.robust; sc.mad_bins = cfg.mad_bins; sc.scale_in = 1e-3f;
+                        ok = solve_update_wave(sys, T, sc, N, nicp, ws);
+                    }
                     if (t == 0) {
                         if (!ok) s_ok = 0;
-                        rms_last = sys[28] > 0.0 ? (float)sqrt(sys[27] / sys[28]) : 0.0f;
+                        if (MODE != RT_GEOMETRIC)
+                            rms_last = sys[RMS0 + 1] > 0.0 ? (float)sqrt(sys[RMS0] / sys[RMS0 + 1]) : 0.0f;
                     }
                 }
                 __syncthreads();
@@ -882,24 +1023,20 @@ __global__ __launch_bounds__(BS, WPE) void kb_track(const PairDesc* __restrict__
 // ------------------------------------------------------------------ lockstep tracking
 // The Gauss-Newton loop of every pair at once, one launch per pass instead of
 // one workgroup per pair: all pairs advance one iteration per step, and a
-// pair's points are spread over many workgroups. It tracks the geometric and
-// bi-objective batches (a level has up to W x H points, 75 to 300 per lane of
+// pair's points are spread over many workgroups. It tracks most geometric and
+// bi-objective batches (icp_variant; a level has up to W x H points, 75 to 300 per lane of
 // one workgroup: 64 pairs of 320x240 took 4.05 ms on 64 of the 256 CUs) and the
 // small photometric batches, which would leave most CUs idle.
 //
-// The sums are those of a 1024-thread workgroup: the photometric ones equal
-// kb_track's bit for bit, the geometric ones follow the same order. Virtual
-// lane (wave v of 16, lane l) adds its points 64 v + l + 1024 j in order of j in
-// FP32, the 64 lanes of a wave meet in the exchange order 32, 16, ..., 1, and
-// the 16 waves add in order in FP64. A workgroup of 8 waves is one virtual wave:
-// in each round wave w forms the terms' factors of the points j = 8 round + w
-// (one per lane) and leaves them in LDS, and after a barrier four of the waves
-// add eight terms each over the round's eight j, so that the points are formed
-// by eight waves while each sum stays one chain.
+// The sums are those of a 1024-thread workgroup of kb_track, bit for bit:
+// virtual lane (wave v of 16, lane l) adds its points 64 v + l + 1024 j in
+// order of j in FP32, the 64 lanes of a wave meet in the exchange order
+// 32, 16, ..., 1, and the 16 waves add in order in FP64. A workgroup of 8
+// waves is one virtual wave: in each round wave w forms the terms' factors of
+// the points j = 8 round + w (one per lane) and leaves them in LDS, and after
+// a barrier four of the waves add eight terms each over the round's eight j, so
+// that the points are formed by eight waves while each sum stays one chain.
 
-// Most pixels of a pair (build_batch refuses more: whole segments of its 512 in
-// the selection hold up to 1024 pixels), and their blocks of 1024.
-constexpr int MAX_PIXELS = 512 * 1025 - 1, LK_BLOCKS = (MAX_PIXELS + 1023) / 1024;
 struct LockBufs {
     char* base;        // per pair: the arrays below
     size_t stride, o_rz, o_bits, o_rfull;
@@ -1266,7 +1403,7 @@ __global__ __launch_bounds__(64) void kl_solve(const PairDesc* __restrict__ P, L
 }
 
 typedef void (*TrackFn)(const PairDesc*, const int*, int, int*, TrackCfg);
-struct Variant { int bs, ppt, rz, wpe; TrackFn fn; int pc = 0; };
+struct Variant { int bs, ppt, rz, wpe; TrackFn fn; int pc = 0; int mode = RT_PHOTOMETRIC; };
 static const Variant kVariants[] = {
     {256, 8, 0, 1, kb_track<256, 8, 0>},     {256, 16, 0, 1, kb_track<256, 16, 0>},
     {256, 32, 0, 1, kb_track<256, 32, 0>},   {512, 4, 0, 1, kb_track<512, 4, 0>},
@@ -1285,6 +1422,11 @@ static const Variant kVariants[] = {
     {512, 16, 0, 1, kb_track<512, 16, 0, 1, 1>, 8192},
     {1024, 2, 1, 1, kb_track<1024, 2, 1, 1, 1>, 5632},   {1024, 4, 1, 1, kb_track<1024, 4, 1, 1, 1>, 5632},
     {512, 4, 1, 1, kb_track<512, 4, 1, 1, 1>, 5632},     {1024, 2, 1, 1, kb_track<1024, 2, 1, 1, 1>, 5120},
+    // the geometric modes, with 1024 threads (256 and 512 were slower by a fifth
+    // to a half at every size); ppt and rz serve the photometric points, and the
+    // selection's LDS leaves room for a smaller point cache
+    {1024, 2, 1, 1, kb_track<1024, 2, 1, 1, 1, RT_BIOBJECTIVE>, 4608, RT_BIOBJECTIVE},
+    {1024, 1, 0, 1, kb_track<1024, 1, 0, 1, 0, RT_GEOMETRIC>, 0, RT_GEOMETRIC},
 };
 
 }  // namespace rt
@@ -1534,6 +1676,7 @@ static void launch_prep(const BatchView& v, hipStream_t s, int part = 0) {
 
 static TrackCfg track_cfg(const BatchView& bv, const Variant& v) {
     TrackCfg c;
+    c.lambda = bv.lambda;
     c.pc_cap = v.pc;
     c.rz_len = bv.maxN;
     c.solver = bv.solver;
@@ -1604,6 +1747,7 @@ static int autotune(rt_batch* b) {
     int bv = -1, bg = 0;
     for (int v = 0; v < NUM_VARIANTS; v++) {
         const Variant& var = kVariants[v];
+        if (var.mode != RT_PHOTOMETRIC) continue;  // the geometric modes do not tune (icp_variant)
         if (var.rz) {
             if (!lds_variant_ready(var, b->maxN)) continue;
         } else {
@@ -1697,11 +1841,42 @@ static void launch_lockstep(const rt_batch* b, int depths, hipStream_t s) {
         kl_solve<<<n, 64, 0, s>>>(v.desc, b->lock, step, cfg);
     }
 }
-// The geometric modes always, photometric batches of few pairs with many points
-// (lock_pairs; a variant forced through the environment keeps kb_track).
-static bool tracks_in_lockstep(const rt_batch* b) {
-    if (b->prm.mode != RT_PHOTOMETRIC) return true;
+// Photometric batches of few pairs with many points (lock_pairs; a variant
+// forced through the environment keeps kb_track).
+static bool photo_in_lockstep(const rt_batch* b) {
     return b->n <= b->lock_pairs && !getenv("RT_BATCH_VARIANT");
+}
+// The kb_track variant of a batch in a geometric mode, -1: lockstep. A workgroup
+// per pair is faster once the pairs fill the chip and a level holds few points
+// per lane: tracking alone in us, lockstep and kb_track,
+//   pairs              128         192         256         512
+//   160x120 geometric  675  843    934  878   1221 1009   2359 2000
+//           bi-obj.   1037 1124   1527 1307   2007 1409   3784 2772
+//   224x168 geometric 1018 1828   1577 2014   1971 2086   3690 4124
+//           bi-obj.   1489 2240   2134 2353   2753 2445   5193 4890
+//   320x240 bi-obj.   2311 4276               4305 4604   8224 9214
+// (8192 points, kb_track as it was before its ICP terms were shortened; with
+// them 160x120 bi-objective takes 1102, 1211 and 2376 us, 224x168 2035 and 4009
+// for 256 and 512 pairs; 512 pairs of 160x120 and 320x240 mixed 6310 and
+// 5050).
+// Both take the same sums. The environment may name a variant.
+static int icp_variant(const rt_batch* b) {
+    const char* force = getenv("RT_BATCH_VARIANT");
+    double total = 0, largest = 0;  // pixels
+    for (const PairDesc& d : b->desc) {
+        const double px = (double)d.W * d.H;
+        total += px;
+        largest = std::max(largest, px);
+    }
+    const double fill = total / (largest * b->cus), mean = total / b->n;  // fill: the queue's rounds of the largest pair
+    const bool persistent = (fill >= 0.75 && mean <= 27000) ||
+                            (b->prm.mode == RT_BIOBJECTIVE && fill >= 1.0 && mean <= 50000);
+    for (int v = 0; v < NUM_VARIANTS; v++) {
+        const Variant& var = kVariants[v];
+        if (var.mode != b->prm.mode || !(force ? atoi(force) == v : persistent)) continue;
+        if (lds_variant_ready(var, b->maxN)) return v;
+    }
+    return -1;
 }
 
 // The kernel variant table, for tests that force each variant through
@@ -1710,7 +1885,7 @@ static bool tracks_in_lockstep(const rt_batch* b) {
 extern "C" int rt_batch_variant_info(int v, int info[6]) {
     if (!info || v < 0 || v >= NUM_VARIANTS) return set_error(RT_ERR_ARG, "rt_batch_variant_info: no such variant");
     const Variant& k = kVariants[v];
-    info[0] = k.bs; info[1] = k.ppt; info[2] = k.rz; info[3] = k.pc; info[4] = k.wpe; info[5] = RT_PHOTOMETRIC;
+    info[0] = k.bs; info[1] = k.ppt; info[2] = k.rz; info[3] = k.pc; info[4] = k.wpe; info[5] = k.mode;
     return RT_OK;
 }
 
@@ -1757,7 +1932,12 @@ static int fetch_results(rt_batch* b, rt_pair_result* out) {
 
 static int run_track(rt_batch* b, rt_pair_result* out) {
     int rc;
-    if (tracks_in_lockstep(b)) {
+    const bool icp = b->prm.mode != RT_PHOTOMETRIC;
+    const int fixed = icp ? icp_variant(b) : -1;
+    if (fixed >= 0) {
+        b->variant = fixed;
+        b->grid = std::min(b->n, b->cus);
+    } else if (icp || photo_in_lockstep(b)) {
         int depths = 0;
         for (const PairDesc& d : b->desc) depths |= 1 << d.L;
         if (lock_steps(b, depths) > LOCK_GRAPH_STEPS) {
@@ -1773,8 +1953,7 @@ static int run_track(rt_batch* b, rt_pair_result* out) {
         if (hipGraphLaunch(b->graph_lock, b->stream) != hipSuccess) return set_error(RT_ERR_HIP, "graph launch");
         return out ? fetch_results(b, out) : RT_OK;
     }
-    rc = autotune(b);
-    if (rc) return rc;
+    if (fixed < 0 && (rc = autotune(b))) return rc;
     // the captured launch depends on the batch size, the variant, the grid and,
     // through its dynamic LDS, on the largest point count
     if (!b->graph_track || b->graph_n != b->n || b->graph_variant != b->variant || b->graph_grid != b->grid ||
@@ -2116,7 +2295,7 @@ int noalloc_variant(int maxN) {
     int fallback = -1;
     for (int v = 0; v < NUM_VARIANTS; v++) {
         const rt::Variant& k = rt::kVariants[v];
-        if (k.bs != 1024) continue;
+        if (k.bs != 1024 || k.mode != RT_PHOTOMETRIC) continue;
         if (k.rz && k.pc && k.ppt == 4 && lds_variant_ready(k, maxN)) return v;
         if (!k.rz && !k.pc && k.bs * k.ppt >= maxN && fallback < 0) fallback = v;
     }

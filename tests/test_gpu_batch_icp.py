@@ -1,4 +1,5 @@
-"""Batched geometric and bi-objective tracking (the lockstep launches) against the single-pair tracker and the oracle, on a mixed-size batch
+"""Batched geometric and bi-objective tracking (the lockstep launches, and a
+workgroup per pair for many small ones) against the single-pair tracker and the oracle, on a mixed-size batch
 (160x120 .. 640x480).
 
 - The batch's keyframe and current clouds of every level equal the FP32
@@ -89,6 +90,63 @@ def test_batch_icp_matches_single_and_oracle(mode):
         assert np.radians(es[0]) < 1e-5 and es[1] < 1e-2, i
         assert np.radians(e32[0]) < 1e-5 and e32[1] < 1e-2, i
     bt.close()
+
+
+def _variant(mode):
+    import ctypes
+    from recon_amd import lib
+    info, v = (ctypes.c_int * 6)(), 0
+    while lib().rt_batch_variant_info(v, info) == 0 and info[5] != mode:
+        v += 1
+    return v
+
+
+@pytest.mark.parametrize("mode,N,iters", [(BIOBJECTIVE, 8192, ITERS), (BIOBJECTIVE, 256, (2, 0, 3, 1)),
+                                          (GEOMETRIC, 8192, ITERS), (GEOMETRIC, 2048, (0, 1, 0, 2)),
+                                          (BIOBJECTIVE, 2048, (0, 0, 0, 0))])
+def test_lockstep_equals_the_persistent_kernel(mode, N, iters, monkeypatch):
+    """The geometric modes' two ways, a launch per pass over all pairs and a
+    workgroup per pair, take the same sums in the same order: the same poses,
+    RMS, counts and variances bit for bit, on mixed sizes."""
+    print(f"case batch icp ways mode {mode} N {N} iters {iters}", flush=True)
+    pairs = _pairs(5, 1500)
+    res = []
+    for force in (None, _variant(mode)):
+        monkeypatch.delenv("RT_BATCH_VARIANT", raising=False)
+        if force is not None:
+            monkeypatch.setenv("RT_BATCH_VARIANT", str(force))
+        bt = BatchTracker(len(pairs), 640, 480, mode=mode, n_select=N, iters=iters, lam=0.5)
+        out = list(bt.track(pairs, init=[p["init"] for p in pairs]))
+        out += list(bt.retrack(init=out[0].reshape(-1, 16), n=len(pairs)))
+        for i, p in enumerate(pairs):
+            L = 4 if p["width"] == 640 else 3
+            for l in range(L):
+                if iters[L - 1 - l]:
+                    out.append(bt.debug_read(i, "ICP_COUNT", 0, np.int32, 4)[l:l + 1])
+                    out.append(bt.debug_read(i, "ICP_VAR", l, np.float32, 3))
+        bt.close()
+        res.append(out)
+    for x, y in zip(*res):
+        assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("mode,W,H,n", [(GEOMETRIC, 160, 120, 200), (BIOBJECTIVE, 160, 120, 200), (BIOBJECTIVE, 224, 168, 260)])
+def test_many_small_pairs_equal_few(mode, W, H, n):
+    """Batches past the line to a workgroup per pair against the same pairs in
+    a batch before it."""
+    print(f"case batch icp many {n} {W}x{H} mode {mode}", flush=True)
+    kinds, pairs, keep = 4, [], []
+    for i in range(kinds):
+        g0, d0, g1, d1, Tgt = synth.make_pair(1600 + i, W, H, 3.0, 50.0)
+        bufs = [DeviceBuffer.from_array(a) for a in (g0, d0, g1, d1)]
+        keep.append(bufs)
+        pairs.append(dict(ref_gray=bufs[0].ptr, ref_depth=bufs[1].ptr, cur_gray=bufs[2].ptr, cur_depth=bufs[3].ptr,
+                          width=W, height=H, calib=synth.calib_block_np(W, H)))
+    few = BatchTracker(kinds, W, H, mode=mode, n_select=2048, iters=ITERS, lam=0.5).track(pairs)
+    many = BatchTracker(n, W, H, mode=mode, n_select=2048, iters=ITERS, lam=0.5).track([pairs[i % kinds] for i in range(n)])
+    for x, y in zip(few, many):
+        for i in range(n):
+            assert np.array_equal(x[i % kinds], y[i]), i
 
 
 @pytest.mark.parametrize("mode,W,H,L,N", [(GEOMETRIC, 904, 580, 3, 2048), (BIOBJECTIVE, 904, 580, 3, 8192),
