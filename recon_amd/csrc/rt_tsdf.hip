@@ -45,12 +45,16 @@ struct TsdfMap {
 __device__ __forceinline__ size_t map_tile(const TsdfMap& m, int xt, int y4, int z4) {
     return ((size_t)z4 * m.ny + y4) * m.nx + xt;
 }
+// which of the four nibbles of 16 signs hold one
+__device__ __forceinline__ unsigned nibbles(unsigned r) {
+    return ((r & 0xfu) ? 1u : 0u) | ((r & 0xf0u) ? 2u : 0u) | ((r & 0xf00u) ? 4u : 0u) | ((r & 0xf000u) ? 8u : 0u);
+}
 // the occ byte of a tile from its four slices' signs (16 bits per row of four
 // rows), one per lane of a group of four lanes
 __device__ __forceinline__ unsigned occ_of_words(unsigned long long w) {
     unsigned r = (unsigned)w | (unsigned)(w >> 32);
     r |= r >> 16;
-    unsigned f = ((r & 0xfu) ? 1u : 0u) | ((r & 0xf0u) ? 2u : 0u) | ((r & 0xf00u) ? 4u : 0u) | ((r & 0xf000u) ? 8u : 0u);
+    unsigned f = nibbles(r);
     f |= __shfl_xor(f, 1); f |= __shfl_xor(f, 2);
     return f;
 }
@@ -254,57 +258,79 @@ __device__ __forceinline__ float trilinear(const float2* __restrict__ g, int res
 }
 // resampleVoxelsKernel with trilinearDensity / trilinearWeight
 // (VoxelGrid_cuda.cu:181-262, 897-939): T maps dst voxel centres into src
-// A wave takes 16 x 4 voxels of eight slices: a tile of the sign map.
-__global__ __launch_bounds__(256) void k_tsdf_resample(float2* __restrict__ dst, TsdfMap map, const float2* __restrict__ src,
-                                                       TsdfArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int xt = blockIdx.x, y4 = blockIdx.y * 4 + (threadIdx.x >> 6), z8 = blockIdx.z;
-    if (y4 >= map.ny) return;
+__host__ __device__ __forceinline__ int resample_xcds(int res) { return res > 256 ? 8 : 1; }
+// The resampled voxel (ix, iy, iz); (1, 0) outside src.
+__device__ __forceinline__ float2 resampled(const float2* __restrict__ src, const TsdfArgs& a, int ix, int iy, int iz) {
     const int res = a.res;
-    const int ix = xt * 16 + (lane & 15), iy = y4 * 4 + (lane >> 4);
     const float* T = a.T;
     const float sx = a.ox - a.dx + a.vx, sy = a.oy - a.dy + a.vy, sz = a.oz - a.dz + a.vz;
     const float ex = a.vx * 2, ey = a.vy * 2, ez = a.vz * 2;
-    const float px = sx + ix * ex, py = sy + iy * ey;
+    const float px = sx + ix * ex, py = sy + iy * ey, pz = sz + iz * ez;
+    const float rx = T[0] * px + T[1] * py + T[2] * pz + T[3];
+    const float ry = T[4] * px + T[5] * py + T[6] * pz + T[7];
+    const float rz = T[8] * px + T[9] * py + T[10] * pz + T[11];
+    const float qx = (rx - sx) / ex, qy = (ry - sy) / ey, qz = (rz - sz) / ez;
     const float hi = (float)(res - 2);
-    unsigned long long myneg = 0;
-    for (int k = 0; k < 8; k++) {
-        const int iz = z8 * 8 + k;
-        const float pz = sz + iz * ez;
-        const float rx = T[0] * px + T[1] * py + T[2] * pz + T[3];
-        const float ry = T[4] * px + T[5] * py + T[6] * pz + T[7];
-        const float rz = T[8] * px + T[9] * py + T[10] * pz + T[11];
-        const float qx = (rx - sx) / ex, qy = (ry - sy) / ey, qz = (rz - sz) / ez;
-        float2 out = make_float2(1.0f, 0.0f);
-        // in range, so the cell index is at most res-2 on every axis and all eight reads are inside the grid
-        if (qx >= 0 && qx <= hi && qy >= 0 && qy <= hi && qz >= 0 && qz <= hi) {
-            const unsigned cx = (unsigned)qx, cy = (unsigned)qy, cz = (unsigned)qz;
-            const float fx = qx - cx, fy = qy - cy, fz = qz - cz;
-            const size_t ys = res, zs = (size_t)res * res;
-            const size_t o = cx + cy * ys + cz * zs;
-            const float2 d000 = src[o], d001 = src[o + zs], d010 = src[o + ys], d011 = src[o + ys + zs];
-            const float2 d100 = src[o + 1], d101 = src[o + 1 + zs], d110 = src[o + 1 + ys], d111 = src[o + 1 + ys + zs];
-            float r2[2];
+    float2 out = make_float2(1.0f, 0.0f);
+    // in range, so the cell index is at most res-2 on every axis and all eight reads are inside the grid
+    if (qx >= 0 && qx <= hi && qy >= 0 && qy <= hi && qz >= 0 && qz <= hi) {
+        const unsigned cx = (unsigned)qx, cy = (unsigned)qy, cz = (unsigned)qz;
+        const float fx = qx - cx, fy = qy - cy, fz = qz - cz;
+        const size_t ys = res, zs = (size_t)res * res;
+        const size_t o = cx + cy * ys + cz * zs;
+        const float2 d000 = src[o], d001 = src[o + zs], d010 = src[o + ys], d011 = src[o + ys + zs];
+        const float2 d100 = src[o + 1], d101 = src[o + 1 + zs], d110 = src[o + 1 + ys], d111 = src[o + 1 + ys + zs];
+        float r2[2];
 #pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const float a000 = c ? d000.y : d000.x, a001 = c ? d001.y : d001.x, a010 = c ? d010.y : d010.x,
-                            a011 = c ? d011.y : d011.x, a100 = c ? d100.y : d100.x, a101 = c ? d101.y : d101.x,
-                            a110 = c ? d110.y : d110.x, a111 = c ? d111.y : d111.x;
-                const float x00 = (1 - fx) * a000 + fx * a100, x01 = (1 - fx) * a001 + fx * a101;
-                const float x10 = (1 - fx) * a010 + fx * a110, x11 = (1 - fx) * a011 + fx * a111;
-                const float z0 = (1 - fy) * x00 + fy * x10, z1 = (1 - fy) * x01 + fy * x11;
-                r2[c] = (1 - fz) * z0 + fz * z1;
-            }
-            out = make_float2(r2[0], r2[1]);
+        for (int c = 0; c < 2; c++) {
+            const float a000 = c ? d000.y : d000.x, a001 = c ? d001.y : d001.x, a010 = c ? d010.y : d010.x,
+                        a011 = c ? d011.y : d011.x, a100 = c ? d100.y : d100.x, a101 = c ? d101.y : d101.x,
+                        a110 = c ? d110.y : d110.x, a111 = c ? d111.y : d111.x;
+            const float x00 = (1 - fx) * a000 + fx * a100, x01 = (1 - fx) * a001 + fx * a101;
+            const float x10 = (1 - fx) * a010 + fx * a110, x11 = (1 - fx) * a011 + fx * a111;
+            const float z0 = (1 - fy) * x00 + fy * x10, z1 = (1 - fy) * x01 + fy * x11;
+            r2[c] = (1 - fz) * z0 + fz * z1;
         }
-        if (ix < res) dst[ix + (size_t)iy * res + (size_t)iz * res * res] = out;
-        const unsigned long long neg = __ballot(ix < res && out.x < 0.0f);
-        myneg = lane == k ? neg : myneg;
+        out = make_float2(r2[0], r2[1]);
     }
-    if (lane >= 8) return;
-    store_rows(map.neg + ((size_t)(z8 * 8 + lane) * res + y4 * 4) * map.nx + xt, map.nx, myneg);
-    const unsigned f = occ_of_words(myneg);
-    if ((lane & 3) == 0) map.occ[map_tile(map, xt, y4, z8 * 2 + (lane >> 2))] = (uint8_t)f;
+    return out;
+}
+// A workgroup takes 64 x 4 x 4 voxels, a wave the rows of four slices: reads
+// and writes run along x in 512 bytes, and the four tiles' occ bytes need no
+// other workgroup. Bound by memory. What it costs beyond the voxels are the sign
+// words, 8 bytes of a row per wave: past 256 voxels an axis the workgroups of a
+// row run on one XCD (dispatch is round-robin over 8), so that they meet in one
+// L2. us without the map, and with it in this order or x before y:
+//   256^3 72, 76 / 73   384^3 251, 255 / 262   512^3 575, 586 / 615   768^3 1863, 1980 / 2088
+// under a translation; 73, 76 at 256^3 and 605, 690 at 512^3 with a rotation, whose
+// reads stray. (Tiles of 16 x 4 voxels and eight slices a wave took 94 and 926.)
+__global__ __launch_bounds__(256) void k_tsdf_resample(float2* __restrict__ dst, TsdfMap map, const float2* __restrict__ src,
+                                                       TsdfArgs a) {
+    __shared__ unsigned long long rows[4];
+    const int res = a.res, nxb = (res + 63) / 64, xcds = resample_xcds(res);
+    const int b = blockIdx.x / xcds, xb = b % nxb, y4 = b / nxb * xcds + blockIdx.x % xcds, z4 = blockIdx.y;
+    if (y4 >= map.ny) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, xt = xb * 4 + (threadIdx.x & 3);
+    const int ix = xb * 64 + lane, iy = y4 * 4 + wave;
+    unsigned long long any = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int iz = z4 * 4 + k;
+        float2 out = make_float2(1.0f, 0.0f);
+        if (ix < res) {
+            out = resampled(src, a, ix, iy, iz);
+            dst[ix + (size_t)iy * res + (size_t)iz * res * res] = out;
+        }
+        const unsigned long long neg = __ballot(out.x < 0.0f);
+        any |= neg;
+        if (lane < 4 && xt < map.nx) map.neg[((size_t)iz * res + iy) * map.nx + xt] = (uint16_t)(neg >> 16 * lane);
+    }
+    if (lane == 0) rows[wave] = any;
+    __syncthreads();
+    if (threadIdx.x < 4 && xt < map.nx) {
+        const unsigned r = (unsigned)((rows[0] | rows[1] | rows[2] | rows[3]) >> 16 * lane);
+        map.occ[map_tile(map, xt, y4, z4)] = (uint8_t)nibbles(r);
+    }
 }
 
 // The skip table of a ray cast: for every block of (1 << LB)^3 voxels, whether
@@ -858,7 +884,8 @@ extern "C" int rt_tsdf_resample(rt_tsdf* dst, const rt_tsdf* src, const float* T
     // src's queued work is ordered before the resample
     if (hipEventRecord(src->done, src->stream) != hipSuccess || hipStreamWaitEvent(dst->stream, src->done, 0) != hipSuccess)
         return set_error(RT_ERR_HIP, "rt_tsdf_resample");
-    const dim3 grid(dst->map.nx, (dst->map.ny + 3) / 4, a.resolution / 8);
+    const int xcds = resample_xcds(a.resolution);
+    const dim3 grid((a.resolution + 63) / 64 * ((dst->map.ny + xcds - 1) / xcds * xcds), a.resolution / 4);
     k_tsdf_resample<<<grid, 256, 0, dst->stream>>>(dst->grid, dst->map, src->grid, args);
     if (hipGetLastError() != hipSuccess) return set_error(RT_ERR_HIP, "rt_tsdf_resample");
     // src's later work is ordered after the resample has read it

@@ -161,6 +161,26 @@ def test_sign_map_and_slice_cull_at_tile_edges_bitexact(res, dim, W, H):
     check(dst, odst, "fused after resampling", views[:3])
 
 
+@pytest.mark.parametrize("res", [8, 40, 264])
+def test_resample_at_workgroup_edges(res):
+    """Workgroups of 64 x 4 x 4 voxels that end past the grid, and above 256
+    voxels their order by XCD with rows of workgroups to spare: grid and ray
+    cast (which reads the sign map) bit for bit."""
+    W, H = 64, 48
+    K = normalized_k(W, H)
+    src, osrc = _grids(res, W, H)
+    d = np.round(render_depth(POSES[0], K, W, H)).astype(np.uint16)
+    src.integrate(d, POSES[0], K)
+    osrc.update(d.astype(np.float32), POSES[0], K)
+    dst, odst = _grids(res, W, H)
+    T = pose(4, -6, (70, 30, -40))
+    dst.resample_from(src, T)
+    odst.resample_from(osrc, T)
+    assert _bits_equal(dst.read(), odst.data)
+    for name, a, b in zip(("xyz", "normals", "shade"), dst.raycast(UNFUSED, K, True), odst.raycast(UNFUSED, K, True)):
+        assert _bits_equal(a, b), name
+
+
 def _fused(res, zs, depth, Tcur, K, W, H):
     """One frame fused into the slices zs of a new grid (updateVoxelsKernel in
     float32, every voxel projected): (len(zs), res, res, 2)."""
