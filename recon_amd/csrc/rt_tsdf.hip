@@ -102,12 +102,14 @@ __device__ __forceinline__ void quotients(float rx, float ry, float rz, float& q
 // them. The voxel is read and written only where it is updated, and a wave
 // that changed any voxel brings the tile's signs and occ bytes up to date.
 // Bound by vector instructions (about 110 per slice that is left, busy for four
-// fifths of the time): 31 us at 256^3 and 320 x 240 with 40 % of the slices in
-// the image, where one thread per voxel and two divisions each took 42.
-constexpr int UPDATE_Z = 16;
+// fifths of the time): 29 us at 256^3 and 320 x 240 with 40 % of the slices in
+// the image, where one thread per voxel and two divisions each took 38. Grids of
+// up to 128^3 take 1 us longer than so: bringing the signs up to date is a load
+// and a store more, which the ray cast gives back (10 us and more from 64^3 on).
 __device__ __forceinline__ float from_lane(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
+template <int UPDATE_Z>
 __global__ __launch_bounds__(256) void k_tsdf_update(float2* __restrict__ tsdf, TsdfMap map, const float* __restrict__ dist,
                                                      TsdfArgs a, TsdfCull c) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -838,8 +840,19 @@ extern "C" int rt_tsdf_update(rt_tsdf* g, const float* T, const float* K) {
     float iT[16];
     invert_rt4f(T, iT);  // VoxelGrid::setCameraParams (VoxelGrid.cpp:275-282): the kernel maps world -> camera
     const TsdfArgs a = tsdf_args(g, iT, K);
-    const dim3 grid(g->map.nx, (g->map.ny + 3) / 4, (g->p.resolution + UPDATE_Z - 1) / UPDATE_Z);
-    k_tsdf_update<<<grid, 256, 0, g->stream>>>(g->grid, g->map, g->dist, a, tsdf_cull(a));
+    auto update = [&](auto slices) {
+        constexpr int Z = decltype(slices)::value;
+        const dim3 grid(g->map.nx, (g->map.ny + 3) / 4, (g->p.resolution + Z - 1) / Z);
+        k_tsdf_update<Z><<<grid, 256, 0, g->stream>>>(g->grid, g->map, g->dist, a, tsdf_cull(a));
+    };
+    // Slices a wave: few where the grid has few waves, and one follows the other's
+    // latency; many where they are plenty and share the wave's set-up. us of an
+    // update at 4 and 16 slices: 64^3 5.1 10.3, 128^3 8.7 11.8, 192^3 14.6 17.8,
+    // 256^3 29.0 29.4, 384^3 70.8 63.6, 512^3 214 190 (one thread per voxel 4.2,
+    // 7.6, 17.4, 38, 117 and 298); of frames in flight, each with its ray cast,
+    // 192^3 32.1 33.6, 256^3 49.3 47.6.
+    if (g->p.resolution < 256) update(std::integral_constant<int, 4>());
+    else update(std::integral_constant<int, 16>());
     if (hipGetLastError() != hipSuccess) return set_error(RT_ERR_HIP, "rt_tsdf_update");
     return RT_OK;
 }
