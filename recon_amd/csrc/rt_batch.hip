@@ -463,7 +463,7 @@ __device__ __forceinline__ void count_segments(const RT_GLOBAL uint8_t* bins, in
 // counts in the pair's point array, which kb_ref_points fills later, and each
 // workgroup of kb_select repeats the trim and the offsets and scatters its own
 // segments. One pair per workgroup left most CUs idle: 64 pairs of 640x480 147
-// us, split over 16 workgroups 45 us (both launches); 256 mixed pairs 147 and 92
+// us, split over 16 workgroups 39 us (both launches); 256 mixed pairs 147 and 94
 // us.
 static int select_parts(int n) {
     int parts = 1;
@@ -767,7 +767,7 @@ struct TrackCfg {
 // workgroup leaves, and 70 of the passes' registers are spilled around it by
 // every wave; 10 with the call, whose cost only wave 0 pays. The kernels with
 // residuals in LDS and 512 or 1024 threads call it (640x480 and 8192 points, us
-// inline and called: 4096 pairs 6520 and 6400, 256 pairs 451 and 435). Those with
+// inline and called: 4096 pairs 6520 and 6340, 256 pairs 451 and 435). Those with
 // residuals in registers spill these around the call instead (256 pairs of
 // 12288 points 1064 and 1080, 48 pairs 746 and 782), and 256 threads have the
 // registers (512 pairs of 320x240 with 1024 points 178 and 188): inline. (The

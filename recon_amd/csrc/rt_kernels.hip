@@ -179,8 +179,9 @@ __device__ __forceinline__ void reduce27(const double* acc, double* part, int gr
 // (k_solve) costs a kernel boundary and another round trip to memory per
 // iteration. Measured with the separate launch and without: a 320x240
 // photometric pair of 8192 points 277 and 270 us, a 640x480 geometric pair 507
-// and 457 us. Bound by latency: kernel start, the partials' round trip, the
-// serial FP64 solve (1.4 us), the taps' round trip, the kernel's end.
+// and 457 us. Bound by latency: of a residual launch's 9.8 us 2.6 are the pass,
+// 4.8 the combine (a round trip to sums that other XCDs have just written) and
+// 2.4 the serial FP64 solve.
 // Wave w sums terms w, w + NW, ... of the 54; lane l adds groups l, l + 64, ...
 // in order (all its loads issued first), then the lanes' sums meet in a fixed
 // exchange tree: the same order for every workgroup size. No update from an
