@@ -1,6 +1,6 @@
 """Batched geometric and bi-objective tracking (the lockstep launches, and a
-workgroup per pair for many small ones) against the single-pair tracker and the oracle, on a mixed-size batch
-(160x120 .. 640x480).
+workgroup per pair for many small ones) against the single-pair tracker and
+the oracle, on a mixed-size batch (160x120 .. 640x480), and against each other.
 
 - The batch's keyframe and current clouds of every level equal the FP32
   oracle's bit for bit.
